@@ -1168,6 +1168,19 @@ int build_slot(fct_batch* b, BatchSlot& s, const fct_step_args* args) {
         std::vector<unsigned char> desc;
         std::vector<int2> bv, bn, ba, bns, bnd, bpa, bp1, be2, be1;
         const bool split = g.ns == 2;     // every instance of such a group has node lists
+        int64_t np2 = 0, np1 = 0;         // edge patches of the two-tracer and one-tracer launches
+        int lmax = 0;
+        for (int i = 0; i < n; ++i) {
+            if (cls[i] != (int)c) continue;
+            const int64_t np = b->plans[i]->tab.ep.np;
+            np2 += np * (args[i].ntracers / 2);
+            np1 += np * (args[i].ntracers % 2);
+            lmax = std::max(lmax, b->plans[i]->m.L);
+        }
+        if (t.adfh_kc) {
+            g.nseg2 = adfh_segments(np2, lmax, t.adfh_kc);
+            g.nseg1 = adfh_segments(np1, lmax, t.adfh_kc);
+        }
         for (int i = 0; i < n; ++i) {
             if (cls[i] != (int)c) continue;
             fct_plan* p = b->plans[i];
@@ -1192,10 +1205,17 @@ int build_slot(fct_batch* b, BatchSlot& s, const fct_step_args* args) {
             } else {
                 block_table(bn, inst, node_waves(p->m.N, K), t.wpb);
             }
-            if (t.adfh_kc && p->tab.ep.np) {
+            // the patch kernel's pairs of tracers and a last one alone, or, where the
+            // group has too few patches, every tracer by wavefronts
+            if (t.adfh_kc && p->tab.ep.np && (K < 2 || g.nseg2) && (K % 2 == 0 || g.nseg1)) {
                 for (int j0 = 0; j0 < K; j0 += 2) {
-                    std::vector<int2>& be = K - j0 >= 2 ? be2 : be1;
-                    for (int q = 0; q < p->tab.ep.np; ++q) be.push_back(make_int2(inst, q | (j0 << 24)));
+                    const bool two = K - j0 >= 2;
+                    std::vector<int2>& be = two ? be2 : be1;
+                    const int nseg = two ? g.nseg2 : g.nseg1;
+                    for (int q = 0; q < p->tab.ep.np; ++q)
+                        for (int sg = 0; sg < nseg; ++sg)
+                            be.push_back(make_int2(inst, (int)((unsigned)q | ((unsigned)j0 << 24) |
+                                                               ((unsigned)sg << 27))));
                 }
             } else {
                 block_table(ba, inst, adfh_waves(p->m.D, K, t), t.wpb);

@@ -248,13 +248,19 @@ struct BatchGroup {
     // its high 16 bits; the deep nodes (nl > 64) stay in blk_nd
     const int2* blk_pa = nullptr;
     const int2* blk_p1 = nullptr;
-    // adf_h by edge patches: per workgroup (instance, patch | first tracer << 24), two
-    // tracers per thread (e2) or one (e1); instances without patches stay in blk_a
+    // adf_h by edge patches: per workgroup (instance, patch | first tracer << 24 |
+    // level segment << 27), two tracers per thread (e2) or one (e1), every patch's levels
+    // in nseg2 (nseg1) segments; instances without patches stay in blk_a
     const int2* blk_e2 = nullptr;
     const int2* blk_e1 = nullptr;
+    int nseg2 = 1, nseg1 = 1;
     unsigned nb_v = 0, nb_n = 0, nb_a = 0, nb_ns = 0, nb_nd = 0, nb_pa = 0, nb_p1 = 0, nb_e2 = 0,
              nb_e1 = 0;
 };
+
+// Workgroups per edge patch of an adf_h launch over `patches` patches of nl = L levels in
+// chunks of kc; 0: too few for the patch kernel (fct_fused.hip).
+int adfh_segments(int64_t patches, int L, int kc);
 
 // Fused launcher (fct_fused.hip): kw = tracers per chunk (workspace slots).
 int launch_fused(const DevMesh& m, const NodeTab& tab, const int2* ekr, const fct_step_args* a,

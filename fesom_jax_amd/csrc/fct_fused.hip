@@ -616,8 +616,16 @@ __device__ __forceinline__ void adfh_group(const FusedArgs& a, int g, int j) {
 // once per chunk instead of once per incident edge; only the node-averaged gradients
 // (read on the few levels where an edge does not use its up/down triangles) are still
 // gathered per edge.
+// Keeps a 32-bit row index from being widened to one 64-bit pointer per array and item for
+// the whole chunk loop: with those (and 22 to 75 registers spilled to scratch) the
+// one-tracer kernel ran the icosa-7 x 70 step in 973 us, without them in 797.
+__device__ __forceinline__ uint32_t opaque32(uint32_t x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
 template <int KT, int KC, int TPE>
-__device__ __forceinline__ void adfh_patch(const FusedArgs& a, int p, int j0) {
+__device__ __forceinline__ void adfh_patch(const FusedArgs& a, int p, int j0, int seg, int nseg) {
     constexpr int NT = FCT_EP * TPE;              // threads
     constexpr int PS = FCT_PU + 1;                // row pitches padded against bank conflicts
     constexpr int ES = FCT_EP + 1;
@@ -631,7 +639,13 @@ __device__ __forceinline__ void adfh_patch(const FusedArgs& a, int p, int j0) {
     const int L = m.L;
     const int4 pt = ldc(a.tab.ep.ptab, p);
     const int first = pt.x, noff = pt.y, cnt = pt.z & 0xffff, U = pt.z >> 16;
-    const int klo = pt.w & 0xff, khi = (pt.w >> 8) & 0xff;
+    int klo = pt.w & 0xff, khi = (pt.w >> 8) & 0xff;
+    {   // this workgroup's segment of the patch's level chunks
+        const int per = ((khi - klo + KC - 1) / KC + nseg - 1) / nseg * KC;
+        klo += seg * per;
+        khi = khi < klo + per ? khi : klo + per;
+        if (klo >= khi) return;
+    }
     const int t = threadIdx.x, q = t % FCT_EP, kq = (t / FCT_EP) * LPT;
     int2 kr = make_int2(0, 0), ur = kr, nd = kr, sl = kr;
     double2 cc = make_double2(0.0, 0.0);
@@ -657,18 +671,18 @@ __device__ __forceinline__ void adfh_patch(const FusedArgs& a, int p, int j0) {
     const int sua = (sl.x >> 16) & 0xff, sub = (sl.x >> 24) & 0xff;
     const int sda = sl.y & 0xff, sdb = (sl.y >> 8) & 0xff;
     const int cu = (sl.y >> 16) & 3, cd = (sl.y >> 18) & 3;
-    // row offsets of this thread's items: node columns (slot s, level kk) and edge
+    // row indices of this thread's items: node columns (slot s, level kk) and edge
     // columns (edge q, level kk), i = t + r * NT, s or q = i / KC, kk = i % KC
-    size_t nrow[NI], erow[NV];
+    uint32_t nrow[NI], erow[NV];
 #pragma unroll
     for (int r = 0; r < NI; ++r) {
         const int i = t + r * NT, s = i / KC;
-        nrow[r] = s < U ? (size_t)G(a.tab.ep.pnodes)[noff + s] * L : 0;
+        nrow[r] = (s < U ? (uint32_t)G(a.tab.ep.pnodes)[noff + s] * (uint32_t)L : 0u) + i % KC;
     }
 #pragma unroll
     for (int r = 0; r < NV; ++r) {
         const int i = t + r * NT, qq = i / KC;
-        erow[r] = qq < cnt ? (size_t)G(a.tab.ep.elist)[first + qq] * L : 0;
+        erow[r] = (qq < cnt ? (uint32_t)G(a.tab.ep.elist)[first + qq] * (uint32_t)L : 0u) + i % KC;
     }
     double pT[NI][KT], pO[NI][KT], pv[NV];
 #define FCT_PREFETCH(K0)                                                                    \
@@ -677,13 +691,13 @@ __device__ __forceinline__ void adfh_patch(const FusedArgs& a, int p, int j0) {
             const int i = t + r * NT, s = i / KC, k = (K0) + i % KC;                        \
             const bool ok = s < U && k < L;                                                 \
             _Pragma("unroll") for (int jj = 0; jj < KT; ++jj) {                             \
-                pT[r][jj] = ok ? G(a.T[j0 + jj])[nrow[r] + k] : 0.0;                        \
-                pO[r][jj] = ok ? G(a.Told[j0 + jj])[nrow[r] + k] : 0.0;                     \
+                pT[r][jj] = ok ? (G(a.T[j0 + jj]) + (K0))[opaque32(nrow[r])] : 0.0;              \
+                pO[r][jj] = ok ? (G(a.Told[j0 + jj]) + (K0))[opaque32(nrow[r])] : 0.0;           \
             }                                                                               \
         }                                                                                   \
         _Pragma("unroll") for (int r = 0; r < NV; ++r) {                                    \
             const int i = t + r * NT, qq = i / KC, k = (K0) + i % KC;                       \
-            pv[r] = (qq < cnt && k < L) ? G(a.vflux)[erow[r] + k] : 0.0;                    \
+            pv[r] = (qq < cnt && k < L) ? (G(a.vflux) + (K0))[opaque32(erow[r])] : 0.0;          \
         }                                                                                   \
     } while (0)
     FCT_PREFETCH(klo);
@@ -758,7 +772,7 @@ __device__ __forceinline__ void adfh_patch(const FusedArgs& a, int p, int j0) {
                 if (k >= rr.x && k < rr.y) {
 #pragma unroll
                     for (int jj = 0; jj < KT; ++jj)
-                        G(a.adfh + (size_t)(j0 + jj) * m.D * L)[erow[r] + k] = vo[jj][kk][qq];
+                        (G(a.adfh + (size_t)(j0 + jj) * m.D * L) + k0)[opaque32(erow[r])] = vo[jj][kk][qq];
                 }
             }
         }
@@ -1474,21 +1488,23 @@ __global__ void FCT_OCC(8) kb_adfh(const FusedArgs* __restrict__ d,
     adfh_group<NS, EPW>(a, g, w - g * a.K);
 }
 
-// adf_h over edge patches; KT tracers from slot j0 of the launch's tracer chunk
-// at most 128 registers per thread
+// adf_h over edge patches; KT tracers from slot j0 of the launch's tracer chunk. At most
+// 128 registers per thread, 168 in the one-tracer kernel with a thread per edge: its 40 KB
+// of LDS allow four workgroups per CU, but at 128 registers it spills 22 of them.
 template <int KT, int KC, int TPE>
-__global__ void __launch_bounds__(FCT_EP * TPE) __attribute__((amdgpu_waves_per_eu(4)))
-ke_adfh(FusedArgs a, int j0) {
-    adfh_patch<KT, KC, TPE>(a, (int)block_tile(a.remap), j0);
+__global__ void __launch_bounds__(FCT_EP * TPE) __attribute__((amdgpu_waves_per_eu(KT == 1 && KC == 8 && TPE == 1 ? 3 : 4)))
+ke_adfh(FusedArgs a, int j0, int nseg) {
+    const int b = (int)block_tile(a.remap), p = b / nseg;
+    adfh_patch<KT, KC, TPE>(a, p, j0, b - p * nseg, nseg);
 }
-// batched form: per workgroup (instance, patch | first tracer << 24)
+// batched form: per workgroup (instance, patch | first tracer << 24 | segment << 27)
 template <int KT, int KC, int TPE>
 __global__ void __launch_bounds__(FCT_EP * TPE) __attribute__((amdgpu_waves_per_eu(4)))
-kbe_adfh(const FusedArgs* __restrict__ d, const int2* __restrict__ blk, int remap) {
+kbe_adfh(const FusedArgs* __restrict__ d, const int2* __restrict__ blk, int remap, int nseg) {
     const int2 e = blk[block_tile(remap)];
     const int inst = __builtin_amdgcn_readfirstlane(e.x);
-    const int pj = __builtin_amdgcn_readfirstlane(e.y);
-    adfh_patch<KT, KC, TPE>(d[inst], pj & 0xffffff, pj >> 24);
+    const unsigned pj = (unsigned)__builtin_amdgcn_readfirstlane(e.y);
+    adfh_patch<KT, KC, TPE>(d[inst], (int)(pj & 0xffffffu), (int)(pj >> 24) & 7, (int)(pj >> 27), nseg);
 }
 
 #define FCT_NODE_KERNELS(PASS, OCC)                                                     \
@@ -1631,6 +1647,22 @@ static inline unsigned blocks_for(int64_t waves, int wpb) {
     return (unsigned)((waves + wpb - 1) / wpb);
 }
 
+// A patch's level chunks are dealt to several workgroups until a launch has about 2048 of
+// them (two to three are resident per CU, so four rounds of the chip): on the pi mesh 35
+// workgroups walking six chunks each took 95 us of a 108 us step, one chunk per
+// workgroup 12 us; at icosa-7 (1350 patches) two segments give 1044 us per step against
+// 1059 with one, and with 2048 patches or more the segments only repeat the patch's table
+// loads. A launch that has fewer chunks than the chip has CUs goes to the wavefront-per-
+// edge kernel instead (0 segments): icosa-4 x 48 33.8 against 38.7 us per step with one
+// tracer, pi 45 against 50; icosa-5 (510 chunks) 60 against 62 with one tracer and 89
+// against 88 with two, where the lines cross.
+int adfh_segments(int64_t patches, int L, int kc) {
+    const int chunks = (L + kc - 1) / kc;
+    if (patches <= 0 || patches * chunks < 256) return 0;
+    const int64_t n = (2048 + patches - 1) / patches;
+    return (int)(n > chunks ? chunks : n);
+}
+
 // node pass `stage` (1, 3 or 4) over the first `count` nodes of the node list with the
 // tracers taken two per wavefront (and a last one alone when K is odd)
 template <int DM>
@@ -1688,14 +1720,14 @@ static void launch_single(const FusedArgs& fa, const FusedTuning& t, hipStream_t
             }
             break;
         case 2:
-            if (t.adfh_kc && fa.tab.ep.np) {
-                const dim3 g(fa.tab.ep.np);
+            if (const int nseg = t.adfh_kc ? adfh_segments(fa.tab.ep.np, m.L, t.adfh_kc) : 0) {
+                const dim3 g((unsigned)(fa.tab.ep.np * nseg));
                 for (int j = 0; j < fa.K; j += 2) {
                     const bool two = fa.K - j >= 2;
 #define FCT_KE(KC, TPE)                                                                         \
     do {                                                                                        \
-        if (two) hipLaunchKernelGGL((ke_adfh<2, KC, TPE>), g, dim3(FCT_EP * TPE), 0, s, fa, j); \
-        else hipLaunchKernelGGL((ke_adfh<1, KC, TPE>), g, dim3(FCT_EP * TPE), 0, s, fa, j);     \
+        if (two) hipLaunchKernelGGL((ke_adfh<2, KC, TPE>), g, dim3(FCT_EP * TPE), 0, s, fa, j, nseg); \
+        else hipLaunchKernelGGL((ke_adfh<1, KC, TPE>), g, dim3(FCT_EP * TPE), 0, s, fa, j, nseg);     \
     } while (0)
                     if (t.adfh_kc == 4) {
                         if (t.adfh_tpe == 1) FCT_KE(4, 1);
@@ -1894,9 +1926,9 @@ static void launch_batch_t(const BatchGroup& g, const FusedTuning& t, hipStream_
 #define FCT_KBE(KC, TPE)                                                                            \
     do {                                                                                            \
         if (g.nb_e2) hipLaunchKernelGGL((kbe_adfh<2, KC, TPE>), dim3(g.nb_e2), dim3(FCT_EP * TPE), 0, s, \
-                                        g.desc, g.blk_e2, t.remap());                               \
+                                        g.desc, g.blk_e2, t.remap(), g.nseg2);                               \
         if (g.nb_e1) hipLaunchKernelGGL((kbe_adfh<1, KC, TPE>), dim3(g.nb_e1), dim3(FCT_EP * TPE), 0, s, \
-                                        g.desc, g.blk_e1, t.remap());                               \
+                                        g.desc, g.blk_e1, t.remap(), g.nseg1);                               \
     } while (0)
         if (t.adfh_kc == 4) {
             if (t.adfh_tpe == 1) FCT_KBE(4, 1);

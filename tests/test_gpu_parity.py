@@ -457,3 +457,28 @@ def test_tracers_share_wavefronts(nl, K, torch_dev):
         plan.lib.fct_plan_set_tuning(plan.ptr, _lib.FCT_TUNE_PAIR_TRACERS, 1)
     for a, b in zip(paired, single):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("level,nl,K", [(3, 48, 1), (4, 48, 2), (5, 19, 1), (5, 25, 3), (5, 48, 2),
+                                        (6, 33, 1)])
+def test_adfh_segments_and_small_meshes(level, nl, K, torch_dev):
+    """The adf_h pass either side of the rule that sends a mesh of few edge patches to the
+    wavefront-per-edge kernel and splits the patches' levels over workgroups (level 4 x 48:
+    126 chunks, waves; level 5 x 19 and x 25: 255 to 340, the line; level 5 x 48: one
+    chunk per workgroup; level 6 x 33: several chunks), bitwise to the oracle, alone and
+    in a batch."""
+    from fesom_jax_amd.batch import FctBatch, Instance
+    from fesom_jax_amd.inputs import make_case
+    from fesom_jax_amd.meshgen import icosahedral_mesh
+    m = icosahedral_mesh(level, nl, seed=81)
+    c = make_case(m, seed=82, dt=2700.0, tracers=("T", "S", "T")[:K])
+    want = [_oracle(m, c, j) for j in range(K)]
+    insts = [Instance.from_case(m, c, torch_dev) for _ in range(2)]
+    insts[0].step_alone()
+    alone = insts[0].T()
+    batch = FctBatch(insts[1:])
+    batch.step()
+    for j in range(K):
+        assert np.array_equal(alone[j].cpu().numpy(), want[j]), j
+        assert np.array_equal(insts[1].T()[j].cpu().numpy(), want[j]), j
+    batch.close()
