@@ -815,10 +815,8 @@ int launch_backward(const DevMesh& m, const AdjointWork& w, const fct_step_args*
         if (split) {
             if ((rc = launch_lo(m, &explicit_part, j, w.vflux, w.LOx, nullptr, nullptr, s)))
                 return rc;
-            if (hipMemcpyAsync(w.LO, w.LOx, NL * sizeof(double), hipMemcpyDeviceToDevice, s) !=
-                hipSuccess)
-                return set_error(FCT_E_HIP, "adjoint tape copy failed");
-            if ((rc = launch_vert_impl(m, a->w_i, a->hnode_new, a->dt, w.LO, w.sh_x, w.sh_n, s)))
+            if ((rc = launch_vert_impl(m, a->w_i, a->hnode_new, a->dt, w.LOx, w.LO, w.sh_x,
+                                       w.sh_n, s)))
                 return rc;
         } else if ((rc = launch_lo(m, a, j, w.vflux, w.LO, nullptr, nullptr, s))) {
             return rc;

@@ -837,8 +837,9 @@ int fct_forward_ex(fct_plan* p, const fct_step_args* a, int32_t path, void* stre
     int rc = check_args(p, a);
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
-    const bool fused_ok = a->w_i == nullptr && p->m.L <= 128 && p->tab.dm > 0;
-    if (path == FCT_PATH_FUSED && !fused_ok)
+    // (asked for by name, the fused path still refuses w_i, as it always has)
+    const bool fused_ok = p->m.L <= 128 && p->tab.dm > 0;
+    if (path == FCT_PATH_FUSED && (!fused_ok || a->w_i))
         return set_error(FCT_E_UNSUPPORTED,
                          "fused path needs w_i == NULL, nl <= 128 and node degree <= 8");
     if (path == FCT_PATH_PHASED || (path == FCT_PATH_AUTO && !fused_ok))

@@ -160,9 +160,17 @@ int launch_vflux(const DevMesh& m, const fct_step_args* a, double* vflux, hipStr
 int launch_lo(const DevMesh& m, const fct_step_args* a, int j, const double* vflux,
               double* LO, double* scr0, double* scr1, hipStream_t s);
 int launch_grad(const DevMesh& m, const fct_step_args* a, int j, double* tr, hipStream_t s);
-// adv_tra_vert_impl of X in place (cp, dp: [N*L] scratch)
+// adv_tra_vert_impl of X into out (X itself allowed; cp, dp: [N*L] scratch)
 int launch_vert_impl(const DevMesh& m, const double* w_i, const double* hnn, double dt,
-                     double* X, double* cp, double* dp, hipStream_t s);
+                     const double* X, double* out, double* cp, double* dp, hipStream_t s);
+
+// The same through LDS (fct_column.hip), for the nl that fit (vimpl_fits), and its form
+// for K tracer slots [K][N][L] of which only wet layers hold values, in place.
+bool vimpl_fits(int L);
+int launch_vimpl(const DevMesh& m, const double* w_i, const double* hnn, double dt,
+                 const double* X, double* out, hipStream_t s);
+int launch_vimpl_wet(const DevMesh& m, const double* w_i, const double* hnn, double dt, double* X,
+                     int K, hipStream_t s);
 int launch_pm(const DevMesh& m, const fct_step_args* a, int j, const double* vflux,
               const double* LO, const double* tr, double* gnode, double* adfh, double* adfv,
               double* tvmax, double* tvmin, double* fplus, double* fminus, hipStream_t s);

@@ -22,6 +22,8 @@
 //   kf_pass1  (node) : LO and the node-averaged gradient gnode (kl_pass1 over a node list)
 //                      (compute_fct_lo :298-313, tracer_gradient_elements :316-326,
 //                       _node_avg_grad :329-341)
+//   k_vimpl   (column): with the implicit split w_i, LO solved for the implicit vertical
+//                      advection (:487-529, fct_column.hip)
 //   kf_adfh   (edge) : adf_h = MFCT high order - upwind low order, once per edge-level
 //                      (:96-105, :196-225, fill_up_dn_grad :344-368)
 //   kf_pass2  (node) : cluster bounds, P+/P-, limiter factors (zalesak_limit :389-451),
@@ -130,6 +132,7 @@ struct FusedArgs {
     const double* uv;
     const double* helem;
     const double* w_e;
+    const double* w_i;     // optional implicit part: adf_v takes w_e + w_i
     const double* hnode;
     const double* hnn;
     const double* Z3d;     // optional
@@ -832,6 +835,7 @@ __device__ __forceinline__ void adfv_inputs(const FusedArgs& a, int n, double (&
         const int kc = k < L ? k : L - 1;
         const size_t i = b0 + kc;
         W[s] = G(a.w_e)[i];
+        if (a.w_i) W[s] = W[s] + G(a.w_i)[i];
         const double2 aa = ldv(m.aav, i);
         ar[s] = aa.x;
         avc[s] = aa.y;
@@ -1794,7 +1798,10 @@ static int launch_fused_t(FusedArgs& fa, const fct_step_args* a, int kw, const F
             const int jj = j0 + (j < K ? j : 0);
             fa.T[j] = a->T[jj]; fa.Told[j] = a->T_old[jj]; fa.Tnew[j] = a->T_new[jj];
         }
-        for (int stage = 1; stage <= 4; ++stage) launch_single<NS, DM>(fa, t, s, stage);
+        launch_single<NS, DM>(fa, t, s, 1);
+        if (a->w_i && (rc = launch_vimpl_wet(fa.m, a->w_i, a->hnode_new, a->dt, fa.LO, K, s)))
+            return rc;
+        for (int stage = 2; stage <= 4; ++stage) launch_single<NS, DM>(fa, t, s, stage);
         if ((rc = check_launch("fused passes"))) return rc;
     }
     return FCT_OK;
@@ -1811,7 +1818,7 @@ static void base_args(FusedArgs& fa, const DevMesh& m, const NodeTab& tab, const
                       const fct_step_args* a, const FusedTuning& tune, double* vflux, double* LO,
                       double* gnode, double* adfh, double* pf, double* adfv) {
     fa.m = m; fa.tab = tab; fa.vflux = vflux; fa.ekr = ekr; fa.uv = a->uv; fa.helem = a->helem;
-    fa.w_e = a->w_e; fa.hnode = a->hnode; fa.hnn = a->hnode_new; fa.Z3d = a->Z3d;
+    fa.w_e = a->w_e; fa.w_i = a->w_i; fa.hnode = a->hnode; fa.hnn = a->hnode_new; fa.Z3d = a->Z3d;
     fa.zbar3 = a->zbar3; fa.dt = a->dt; fa.remap = tune.remap(); fa.K = 0;
     fa.LO = LO; fa.gnode = (double2*)gnode; fa.adfh = adfh; fa.pf = pf; fa.adfv = adfv;
 }

@@ -86,8 +86,9 @@ k_lo(DevMesh m, const double* __restrict__ vflux, const double* __restrict__ T,
     LO[i] = (in_layer(nr, k) && hn > 0.0 && a > 0.0) ? lo : 0.0;
 }
 
-// adv_tra_vert_impl + ops.tdma (tracer_adv.py:487-529, ops.py:121-168); one thread
-// per node column, updates X in place. cp/dp are [N][L] scratch.
+// adv_tra_vert_impl + ops.tdma (tracer_adv.py:487-529, ops.py:121-168) for columns that
+// do not fit LDS (fct_column.hip has the others); one thread per node column, updates X in
+// place. cp/dp are [N][L] scratch.
 __global__ void __launch_bounds__(256)
 k_vert_impl(DevMesh m, const double* __restrict__ w_i, const double* __restrict__ hnn,
             double dt, double* __restrict__ X, double* __restrict__ cp,
@@ -661,16 +662,16 @@ int launch_lo(const DevMesh& m, const fct_step_args* a, int j, const double* vfl
                a->hnode_new, a->dt, LO);
     int rc = check_launch("k_lo");
     if (rc) return rc;
-    if (a->w_i) {
-        FCT_LAUNCH(k_vert_impl, (int64_t)m.N, s, m, a->w_i, a->hnode_new, a->dt, LO, scr0, scr1);
-        rc = check_launch("k_vert_impl");
-    }
-    return rc;
+    return a->w_i ? launch_vert_impl(m, a->w_i, a->hnode_new, a->dt, LO, LO, scr0, scr1, s) : FCT_OK;
 }
 
 int launch_vert_impl(const DevMesh& m, const double* w_i, const double* hnn, double dt,
-                     double* X, double* cp, double* dp, hipStream_t s) {
-    FCT_LAUNCH(k_vert_impl, (int64_t)m.N, s, m, w_i, hnn, dt, X, cp, dp);
+                     const double* X, double* out, double* cp, double* dp, hipStream_t s) {
+    if (vimpl_fits(m.L)) return launch_vimpl(m, w_i, hnn, dt, X, out, s);
+    if (X != out && hipMemcpyAsync(out, X, (size_t)m.N * m.L * sizeof(double),
+                                   hipMemcpyDeviceToDevice, s) != hipSuccess)
+        return set_error(FCT_E_HIP, "adv_tra_vert_impl: copy of the tracer failed");
+    FCT_LAUNCH(k_vert_impl, (int64_t)m.N, s, m, w_i, hnn, dt, out, cp, dp);
     return check_launch("k_vert_impl");
 }
 
@@ -779,10 +780,8 @@ int launch_stage(const DevMesh& m, const StageScratch& w, int stage, const doubl
             FCT_LAUNCH(k_st_f2d, nl, s, m, in[0], in[1], in[2], in[3], in[4], in[5], dt, out[0]);
             break;
         case FCT_STAGE_ADV_TRA_VERT_IMPL: {
-            if (nl > 0 && hipMemcpyAsync(out[0], in[1], (size_t)nl * sizeof(double),
-                                         hipMemcpyDeviceToDevice, s) != hipSuccess)
-                return set_error(FCT_E_HIP, "adv_tra_vert_impl: copy of T failed");
-            FCT_LAUNCH(k_vert_impl, (int64_t)m.N, s, m, in[0], in[2], dt, out[0], w.pf, w.mf);
+            const int rc = launch_vert_impl(m, in[0], in[2], dt, in[1], out[0], w.pf, w.mf, s);
+            if (rc) return rc;
             break;
         }
         default:

@@ -482,3 +482,52 @@ def test_adfh_segments_and_small_meshes(level, nl, K, torch_dev):
         assert np.array_equal(alone[j].cpu().numpy(), want[j]), j
         assert np.array_equal(insts[1].T()[j].cpu().numpy(), want[j]), j
     batch.close()
+
+
+@pytest.mark.parametrize("level,nl,degree8,scattered,K", [
+    (3, 23, 0, False, 1), (4, 48, 0, True, 2), (4, 64, 20, False, 3), (4, 65, 0, False, 2),
+    (4, 70, 20, False, 2), (3, 128, 0, True, 1)])
+@pytest.mark.parametrize("moving", [False, True])
+def test_implicit_split_takes_the_fused_path(level, nl, degree8, scattered, K, moving, torch_dev):
+    """With w_i the default path runs the fused passes and the LDS column solve; same bits
+    as the phased path and the oracle, for one- and two-slot columns (nl at and either
+    side of 64, the largest 128), 6- and 8-slot tables, scattered numbering, odd tracer
+    counts, the static and the moving stencil. The dry lanes of w_i hold values the
+    scheme must not read into the wet ones."""
+    from fesom_jax_amd.inputs import make_case
+    from fesom_jax_amd.meshgen import icosahedral_mesh, shuffled
+    from fesom_jax_amd.tracer_adv import get_plan
+    m = icosahedral_mesh(level, nl, seed=91, degree8=degree8)
+    if scattered:
+        m = shuffled(m, 92)
+    c = sharp_case(m, make_case(m, seed=93, dt=2700.0), 1.5)
+    c["T"] = [c["T"][0] * (1.0 + 0.1 * j) for j in range(K)]
+    c["T_old"] = [c["T_old"][0]] * K
+    rng = np.random.default_rng(94)
+    kw = {"w_i": 0.3 * np.abs(c["w_e"]).max() * rng.standard_normal(m.area.shape)}
+    if moving:
+        zb = m.zbar_3d_n * (1.0 + 0.01 * rng.random(m.zbar_3d_n.shape))
+        kw["Z3d"] = np.concatenate([0.5 * (zb[:, :-1] + zb[:, 1:]), zb[:, -1:]], axis=1)
+        kw["zbar3"] = zb
+    assert get_plan(m, torch_dev).fused_available
+    got = _gpu_step(m, c, torch_dev, path="auto", **kw)
+    ph = _gpu_step(m, c, torch_dev, path="phased", **kw)
+    for j in range(K):
+        assert np.array_equal(got[j], ph[j]), j
+        assert np.array_equal(got[j], _oracle(m, c, j, **kw)), j
+
+
+def test_column_solve_sizes(torch_dev):
+    """The LDS column solve at the edges of its workgroups: fewer columns than one
+    workgroup takes, a remainder, and an nl that leaves room for few columns."""
+    from fesom_jax_amd.meshgen import icosahedral_mesh
+    from fesom_jax_amd.tracer_adv import adv_tra_vert_impl
+    import torch
+    for level, nl, lf in ((2, 5, 0.3), (2, 17, 0.9), (3, 300, 0.3), (2, 1000, 0.6)):
+        m = icosahedral_mesh(level, nl, seed=95, land_fraction=lf, min_levels=2, polar_cap_deg=60.0)
+        rng = np.random.default_rng(96)
+        w_i, T = 1e-4 * rng.standard_normal(m.area.shape), rng.standard_normal(m.area.shape)
+        h = np.where(m.node_layer_mask, 50.0, 0.0)
+        t = lambda a: torch.from_numpy(a).to(torch_dev)
+        got = adv_tra_vert_impl(m, t(w_i), t(T), t(h), dt=2700.0).cpu().numpy()
+        assert np.array_equal(got, O.adv_tra_vert_impl(m, w_i, T, h, dt=2700.0)), (level, nl)
