@@ -688,15 +688,20 @@ int fct_plan_create(const fct_mesh_desc* d, fct_plan** out) {
     // node passes: for nl > 64 shallow columns, then deep ones; for nl <= 64 every column
     // is shallow (the list lets two tracers share a wavefront); each set in visit order
     std::vector<int> h_nlist;
-    if (dm && L > 64) {
+    const bool by_degree = dm == 8 && N >= FCT_SIX_NODES;
+    auto shallow = [&](int n) { return L <= 64 || d->nlevels_nod2D[n] - 1 < 64; };
+    auto six = [&](int n) {
+        return h_eoff[n + 1] - h_eoff[n] <= 6 && h_noff[n + 1] - h_noff[n] <= 6;
+    };
+    if (dm && (L > 64 || dm == 6 || by_degree || !local_ids)) {
         for (int n : visit)
-            if (d->nlevels_nod2D[n] - 1 < 64) h_nlist.push_back(n);
+            if (shallow(n) && (!by_degree || six(n))) h_nlist.push_back(n);
+        p->tab.nsix = dm == 6 || by_degree ? (int)h_nlist.size() : 0;
+        for (int n : visit)
+            if (by_degree && shallow(n) && !six(n)) h_nlist.push_back(n);
         p->tab.nshallow = (int)h_nlist.size();
         for (int n : visit)
-            if (d->nlevels_nod2D[n] - 1 >= 64) h_nlist.push_back(n);
-    } else if (dm == 6 || (dm && !local_ids)) {
-        h_nlist = visit;
-        p->tab.nshallow = N;
+            if (!shallow(n)) h_nlist.push_back(n);
     }
     if (dm && D && ((rc = dev_upload(p, &p->tab.ep.ptab, loc.ptab.data(), loc.ptab.size())) ||
                     (rc = dev_upload(p, &p->tab.ep.pnodes, loc.pnodes.data(), loc.pnodes.size())) ||

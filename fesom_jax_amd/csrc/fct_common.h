@@ -76,6 +76,12 @@ struct EdgePatches {
                                   //  (d_a, d_b) as bytes | cu << 16 | cd << 18
 };
 
+// On an 8-slot mesh the passes of the nodes with 7 or 8 neighbours are launches of their
+// own (three to five microseconds each) once two tracers share the wavefronts of the
+// others: icosa-7 x 70 with 1 % of such nodes, K = 2, 1.69 -> 1.59 ms per step; at 7,169
+// nodes (icosa-5 x 48) 92 us without the split, 98 with it.
+constexpr int FCT_SIX_NODES = 16384;
+
 // Per-node stencil table of the fused path (dm slots per node).
 struct NodeTab {
     int dm = 0;               // slots per node (6 or 8); 0 = mesh not supported
@@ -86,11 +92,14 @@ struct NodeTab {
                               //  edge's triangles as bytes lo1|hi1|lo2|hi2, layer range of
                               //  element slot q as bytes lo|hi), edges in reference order
     const int4* elem;         // [N*dm] (element, v0, v1, v2), increasing element id
-    // nl > 64 only: the nodes whose wet layers end above level 64 (`nshallow` of them, in
-    // node order), then the others; passes 2 and 3 take each set in a launch of its own,
-    // the first with one 64-level slot per wavefront and fewer registers
+    // Node list of the passes: the nodes whose wet layers end above level 64 (`nshallow` of
+    // them; for nl <= 64 all), in visit order, then the others; the passes take each set
+    // in a launch of its own, the first with one 64-level slot per wavefront and fewer
+    // registers. The first `nsix` shallow nodes have at most six slots each and may run
+    // two tracers per wavefront: all of them on a 6-slot mesh; on an 8-slot mesh of at
+    // least FCT_SIX_NODES nodes those with up to six neighbours come first (else 0).
     const int* nlist = nullptr;
-    int nshallow = 0;
+    int nshallow = 0, nsix = 0;
     // slots past a node's counts repeat its first slot, so a kernel can load every slot
     // without waiting for the counts
     EdgePatches ep;           // edge patches of the adf_h patch kernel

@@ -267,8 +267,13 @@ __device__ __forceinline__ void vflux_group(const FusedArgs& a, int g) {
 // ---------------------------------------------------------------------------
 // pass 1 of node n, tracer j: LO and gnode
 // ---------------------------------------------------------------------------
-template <int NS, int DM>
-__device__ __forceinline__ void pass1_body(const FusedArgs& a, int n, int j, int4 hd) {
+// One node's loops run over DM slots of its ST-slot table row. On an 8-slot mesh most nodes
+// have 5 or 6 neighbours: those take the 6-slot loops (a wave-uniform branch), which leaves
+// out the loads of two repeated slots (icosa-7 x 70 with 1 % of nodes at 8, two tracers:
+// pass 1 293 -> 268 us, pass 2 364 -> 333, pass 3 262 -> 260).
+template <int NS, int DM, int ST>
+__device__ __forceinline__ void pass1_slots(const FusedArgs& a, int n, int j, int4 hd,
+                                            double (*s_nb)[ST + 1][64]) {
     const DevMesh& m = a.m;
     const int L = m.L;
     const int2 nr = make_int2(hd.x, hd.y), cnt = make_int2(hd.z & 0xff, hd.w);   // levels, counts
@@ -283,11 +288,10 @@ __device__ __forceinline__ void pass1_body(const FusedArgs& a, int n, int j, int
     int4 el[DM];
 #pragma unroll
     for (int q = 0; q < DM; ++q) {
-        es[q] = ldc(a.tab.edge, (size_t)n * DM + q);
-        el[q] = ldc(a.tab.elem, (size_t)n * DM + q);
+        es[q] = ldc(a.tab.edge, (size_t)n * ST + q);
+        el[q] = ldc(a.tab.elem, (size_t)n * ST + q);
     }
     // per wavefront: the neighbour columns at the lane's level, then the node's own
-    __shared__ double s_nb[4][DM + 1][64];
     double* nb = &s_nb[threadIdx.x >> 6][0][lane_id()];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
@@ -322,12 +326,12 @@ __device__ __forceinline__ void pass1_body(const FusedArgs& a, int n, int j, int
             hn = G(a.hnn)[i]; hnd = G(a.hnode)[i];
             // the element vertices are the node and edge neighbours: the gradient below
             // reads them back from the lane's own LDS row by slot code (bits 16.. of the
-            // element-slot word: 4 bits per vertex, DM = the node) instead of loading
+            // element-slot word: 4 bits per vertex, ST = the node) instead of loading
             // them again
             if (gslot) {
 #pragma unroll
                 for (int q = 0; q < DM; ++q) nb[q * 64] = To[q];
-                nb[DM * 64] = Tk;
+                nb[ST * 64] = Tk;
             }
         }
         if (NS == 1) {
@@ -390,11 +394,18 @@ __device__ __forceinline__ void pass1_body(const FusedArgs& a, int n, int j, int
     }
 }
 
+template <int NS, int DM>
+__device__ __forceinline__ void pass1_body(const FusedArgs& a, int n, int j, int4 hd) {
+    __shared__ double s_nb[4][DM + 1][64];
+    if (DM > 6 && (hd.z & 0xff) <= 6 && hd.w <= 6) pass1_slots<NS, 6, DM>(a, n, j, hd, s_nb);
+    else pass1_slots<NS, DM, DM>(a, n, j, hd, s_nb);
+}
+
 // Pass 1 of a shallow node (wet layers end above level 64, one 64-level slot) for its KT
 // tracers in one wavefront: the tracer-independent loads (the edge fluxes, w, area,
 // areasvol, hnode, hnode_new) are made once; per tracer the arithmetic is pass1_body's.
 // KT is a compile-time count so that the tracer pointers are read at constant offsets.
-template <int DM, int KT>
+template <int DM, int KT, int ST>
 __device__ __forceinline__ void pass1_shallow_all(const FusedArgs& a, int n, int4 hd, int j0) {
     const DevMesh& m = a.m;
     const int L = m.L;
@@ -406,10 +417,10 @@ __device__ __forceinline__ void pass1_shallow_all(const FusedArgs& a, int n, int
     int4 el[DM];
 #pragma unroll
     for (int q = 0; q < DM; ++q) {
-        es[q] = ldc(a.tab.edge, (size_t)n * DM + q);
-        el[q] = ldc(a.tab.elem, (size_t)n * DM + q);
+        es[q] = ldc(a.tab.edge, (size_t)n * ST + q);
+        el[q] = ldc(a.tab.elem, (size_t)n * ST + q);
     }
-    __shared__ double s_nb[4][DM + 1][64];
+    __shared__ double s_nb[4][ST + 1][64];
     double* nb = &s_nb[threadIdx.x >> 6][0][lane_id()];
     const int k = lane_id();
     const bool rd = k < kneed;
@@ -439,7 +450,7 @@ __device__ __forceinline__ void pass1_shallow_all(const FusedArgs& a, int n, int
             if (gslot) {
 #pragma unroll
                 for (int q = 0; q < DM; ++q) nb[q * 64] = To[q];
-                nb[DM * 64] = Tk;
+                nb[ST * 64] = Tk;
             }
         }
         const double Tm = wave_prev(Tk, Tk);
@@ -894,8 +905,8 @@ __device__ __forceinline__ void adfv_column(const FusedArgs& a, int n, int2 nr,
 // ---------------------------------------------------------------------------
 // pass 2 of node n, tracer j: cluster bounds, P+/P-, limiter factors
 // ---------------------------------------------------------------------------
-template <int NS, int DM>
-__device__ __forceinline__ void pass2_body(const FusedArgs& a, int n, int j, int2 nr, int2 cnt) {
+template <int NS, int DM, int ST>
+__device__ __forceinline__ void pass2_slots(const FusedArgs& a, int n, int j, int2 nr, int2 cnt) {
     const DevMesh& m = a.m;
     const int L = m.L;
     const size_t jo = (size_t)j * m.N * L;
@@ -909,7 +920,7 @@ __device__ __forceinline__ void pass2_body(const FusedArgs& a, int n, int j, int
     const int kneed = nr.y + 1 < L ? nr.y + 1 : L;
     int4 es[DM];
 #pragma unroll
-    for (int q = 0; q < DM; ++q) es[q] = ldc(a.tab.edge, (size_t)n * DM + q);
+    for (int q = 0; q < DM; ++q) es[q] = ldc(a.tab.edge, (size_t)n * ST + q);
     double Tc[NS], Ac[NS], LOc[NS], tvx[NS], tvn[NS], ap[NS], am[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
@@ -1013,10 +1024,18 @@ __device__ __forceinline__ void pass2_body(const FusedArgs& a, int n, int j, int
     }
 }
 
+template <int NS, int DM>
+__device__ __forceinline__ void pass2_body(const FusedArgs& a, int n, int j, int2 nr, int2 cnt) {
+    // (two copies of the two-slot body in one kernel put its arrays into scratch memory:
+    // 221 against 62 us for the deep columns of icosa-7 x 70, one tracer)
+    if (NS == 1 && DM > 6 && cnt.x <= 6 && cnt.y <= 6) pass2_slots<NS, 6, DM>(a, n, j, nr, cnt);
+    else pass2_slots<NS, DM, DM>(a, n, j, nr, cnt);
+}
+
 // Pass 2 of a shallow node (one 64-level slot) for its KT tracers in one wavefront: w,
 // area, areasvol, the stencil depths and hnode_new are loaded once; per tracer the
 // arithmetic is pass2_body's.
-template <int DM, int KT>
+template <int DM, int KT, int ST>
 __device__ __forceinline__ void pass2_shallow_all(const FusedArgs& a, int n, int2 nr, int2 cnt, int j0) {
     constexpr int NS = 1;
     const DevMesh& m = a.m;
@@ -1042,7 +1061,7 @@ __device__ __forceinline__ void pass2_shallow_all(const FusedArgs& a, int n, int
         const int kneed = nr.y + 1 < L ? nr.y + 1 : L;
         int4 es[DM];
 #pragma unroll
-        for (int q = 0; q < DM; ++q) es[q] = ldc(a.tab.edge, (size_t)n * DM + q);
+        for (int q = 0; q < DM; ++q) es[q] = ldc(a.tab.edge, (size_t)n * ST + q);
         double Tc[NS], Ac[NS], LOc[NS], tvx[NS], tvn[NS], ap[NS], am[NS];
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
@@ -1158,8 +1177,8 @@ __device__ __forceinline__ void pass2_task(const FusedArgs& a, int n, int j) {
 // ---------------------------------------------------------------------------
 // pass 3 of node n, tracer j: limited fluxes, divergence, reconstruction
 // ---------------------------------------------------------------------------
-template <int NS, int DM>
-__device__ __forceinline__ void pass3_body(const FusedArgs& a, int n, int j, int2 nr, int2 cnt) {
+template <int NS, int DM, int ST>
+__device__ __forceinline__ void pass3_slots(const FusedArgs& a, int n, int j, int2 nr, int2 cnt) {
     const DevMesh& m = a.m;
     const int L = m.L;
     const auto T = G(a.T[j]);
@@ -1170,7 +1189,7 @@ __device__ __forceinline__ void pass3_body(const FusedArgs& a, int n, int j, int
     const int kneed = nr.y + 1 < L ? nr.y + 1 : L;
     int4 es[DM];
 #pragma unroll
-    for (int q = 0; q < DM; ++q) es[q] = ldc(a.tab.edge, (size_t)n * DM + q);
+    for (int q = 0; q < DM; ++q) es[q] = ldc(a.tab.edge, (size_t)n * ST + q);
     // adf_v at the node's interfaces (k <= nzmax) as pass 2 computed it
     const auto Fv = G(a.adfv + jo);
     double Tc[NS], fvc[NS], Pc[NS], Mc[NS], acc[NS];
@@ -1256,17 +1275,23 @@ __device__ __forceinline__ void pass3_body(const FusedArgs& a, int n, int j, int
     for (int k = 64 * NS + lane_id(); k < L; k += 64) Tn[b0 + k] = T[b0 + k] + 0.0;
 }
 
+template <int NS, int DM>
+__device__ __forceinline__ void pass3_body(const FusedArgs& a, int n, int j, int2 nr, int2 cnt) {
+    if (DM > 6 && cnt.x <= 6 && cnt.y <= 6) pass3_slots<NS, 6, DM>(a, n, j, nr, cnt);
+    else pass3_slots<NS, DM, DM>(a, n, j, nr, cnt);
+}
+
 // Pass 3 of a shallow node (one 64-level slot) for its KT tracers in one wavefront:
 // areasvol, hnode_new and hnode are loaded once; per tracer the arithmetic is
 // pass3_body's.
-template <int DM, int KT>
+template <int DM, int KT, int ST>
 __device__ __forceinline__ void pass3_shallow_all(const FusedArgs& a, int n, int2 nr, int2 cnt, int j0) {
     constexpr int NS = 1;
     const DevMesh& m = a.m;
     const int L = m.L;
     int4 es[DM];
 #pragma unroll
-    for (int q = 0; q < DM; ++q) es[q] = ldc(a.tab.edge, (size_t)n * DM + q);
+    for (int q = 0; q < DM; ++q) es[q] = ldc(a.tab.edge, (size_t)n * ST + q);
     const int kl = lane_id();
     const bool wetl = in_layer(nr, kl);
     double av_s = 0.0, hn_s = 0.0, hnd_s = 0.0;
@@ -1383,11 +1408,10 @@ __device__ __forceinline__ void pass3_task(const FusedArgs& a, int n, int j) {
 // fluxes of ttfAB (adv_flux_hor :96-105, adv_flux_ver :108-120), flux2dtracer
 // (:123-139) and ale_reconstruct (:142-151); every lane of T_new is written
 // ---------------------------------------------------------------------------
-template <int NS, int DM>
-__device__ __forceinline__ void upwind_task(const FusedArgs& a, int n, int j) {
+template <int NS, int DM, int ST>
+__device__ __forceinline__ void upwind_slots(const FusedArgs& a, int n, int j, int4 hd) {
     const DevMesh& m = a.m;
     const int L = m.L;
-    const int4 hd = ldc(a.tab.hdr, n);
     const int2 nr = make_int2(hd.x, hd.y), cnt = make_int2(hd.z & 0xff, hd.w);
     const auto T = G(a.T[j]);
     const auto To = G(a.Told[j]);
@@ -1395,7 +1419,7 @@ __device__ __forceinline__ void upwind_task(const FusedArgs& a, int n, int j) {
     const size_t b0 = (size_t)n * L;
     int4 es[DM];
 #pragma unroll
-    for (int q = 0; q < DM; ++q) es[q] = ldc(a.tab.edge, (size_t)n * DM + q);
+    for (int q = 0; q < DM; ++q) es[q] = ldc(a.tab.edge, (size_t)n * ST + q);
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         const int k = 64 * s + lane_id();
@@ -1450,6 +1474,13 @@ __device__ __forceinline__ void upwind_task(const FusedArgs& a, int n, int j) {
         const double dT = hn > 0.0 ? del / safe_hn : 0.0;
         Tn[i] = Ti + dT;
     }
+}
+
+template <int NS, int DM>
+__device__ __forceinline__ void upwind_task(const FusedArgs& a, int n, int j) {
+    const int4 hd = ldc(a.tab.hdr, n);
+    if (DM > 6 && (hd.z & 0xff) <= 6) upwind_slots<NS, 6, DM>(a, n, j, hd);
+    else upwind_slots<NS, DM, DM>(a, n, j, hd);
 }
 
 // ---------------------------------------------------------------------------
@@ -1573,30 +1604,30 @@ FCT_BATCH_LIST_KERNEL(pass3, 8, 6, (pass3_body<NSB, DM>(a, n, w - t * a.K, make_
 #undef FCT_BATCH_LIST_KERNEL
 
 // one wavefront per shallow node for KT tracers from slot j0
-template <int DM, int KT>
+template <int DM, int KT, int ST = DM>
 __global__ void FCT_OCC(DM == 6 ? 6 : 4) kl_pass2_all(FusedArgs a, int count, int j0) {
     int w;
     if (!single_wave((int64_t)count, a.remap, w)) return;
     const int n = ldc(a.tab.nlist, (size_t)w);
     const int4 hd = ldc(a.tab.hdr, n);
-    pass2_shallow_all<DM, KT>(a, n, make_int2(hd.x, hd.y), make_int2(hd.z & 0xff, hd.w), j0);
+    pass2_shallow_all<DM, KT, ST>(a, n, make_int2(hd.x, hd.y), make_int2(hd.z & 0xff, hd.w), j0);
 }
 
-template <int DM, int KT>
+template <int DM, int KT, int ST = DM>
 __global__ void FCT_OCC(DM == 6 ? 7 : 4) kl_pass3_all(FusedArgs a, int count, int j0) {
     int w;
     if (!single_wave((int64_t)count, a.remap, w)) return;
     const int n = ldc(a.tab.nlist, (size_t)w);
     const int4 hd = ldc(a.tab.hdr, n);
-    pass3_shallow_all<DM, KT>(a, n, make_int2(hd.x, hd.y), make_int2(hd.z & 0xff, hd.w), j0);
+    pass3_shallow_all<DM, KT, ST>(a, n, make_int2(hd.x, hd.y), make_int2(hd.z & 0xff, hd.w), j0);
 }
 
-template <int DM, int KT>
+template <int DM, int KT, int ST = DM>
 __global__ void FCT_OCC(DM == 6 ? 5 : 4) kl_pass1_all(FusedArgs a, int count, int j0) {
     int w;
     if (!single_wave((int64_t)count, a.remap, w)) return;
     const int n = ldc(a.tab.nlist, (size_t)w);
-    pass1_shallow_all<DM, KT>(a, n, ldc(a.tab.hdr, n), j0);
+    pass1_shallow_all<DM, KT, ST>(a, n, ldc(a.tab.hdr, n), j0);
 }
 
 // batched multi-tracer passes: waves over each instance's shallow node list; the block
@@ -1609,7 +1640,7 @@ __global__ void FCT_OCC(DM == 6 ? 5 : 4) kbp_pass1(const FusedArgs* __restrict__
     const FusedArgs& a = d[ij & 0xffff];
     if (w >= a.tab.nshallow) return;
     const int n = ldc(a.tab.nlist, (size_t)w);
-    pass1_shallow_all<DM, KT>(a, n, ldc(a.tab.hdr, n), ij >> 16);
+    pass1_shallow_all<DM, KT, DM>(a, n, ldc(a.tab.hdr, n), ij >> 16);
 }
 template <int DM, int KT>
 __global__ void FCT_OCC(DM == 6 ? 6 : 4) kbp_pass2(const FusedArgs* __restrict__ d,
@@ -1620,7 +1651,7 @@ __global__ void FCT_OCC(DM == 6 ? 6 : 4) kbp_pass2(const FusedArgs* __restrict__
     if (w >= a.tab.nshallow) return;
     const int n = ldc(a.tab.nlist, (size_t)w);
     const int4 hd = ldc(a.tab.hdr, n);
-    pass2_shallow_all<DM, KT>(a, n, make_int2(hd.x, hd.y), make_int2(hd.z & 0xff, hd.w), ij >> 16);
+    pass2_shallow_all<DM, KT, DM>(a, n, make_int2(hd.x, hd.y), make_int2(hd.z & 0xff, hd.w), ij >> 16);
 }
 template <int DM, int KT>
 __global__ void FCT_OCC(DM == 6 ? 7 : 4) kbp_pass3(const FusedArgs* __restrict__ d,
@@ -1631,7 +1662,7 @@ __global__ void FCT_OCC(DM == 6 ? 7 : 4) kbp_pass3(const FusedArgs* __restrict__
     if (w >= a.tab.nshallow) return;
     const int n = ldc(a.tab.nlist, (size_t)w);
     const int4 hd = ldc(a.tab.hdr, n);
-    pass3_shallow_all<DM, KT>(a, n, make_int2(hd.x, hd.y), make_int2(hd.z & 0xff, hd.w), ij >> 16);
+    pass3_shallow_all<DM, KT, DM>(a, n, make_int2(hd.x, hd.y), make_int2(hd.z & 0xff, hd.w), ij >> 16);
 }
 
 template <int NSB, int DM>
@@ -1669,59 +1700,68 @@ int adfh_segments(int64_t patches, int L, int kc) {
 
 // node pass `stage` (1, 3 or 4) over the first `count` nodes of the node list with the
 // tracers taken two per wavefront (and a last one alone when K is odd)
-template <int DM>
+template <int DM, int ST>
 static void launch_shallow_multi(const FusedArgs& fa, const FusedTuning& t, hipStream_t s,
                                  int stage, int count) {
     const dim3 blk(64 * t.wpb), g(blocks_for(count, t.wpb));
     for (int j0 = 0; j0 < fa.K; j0 += 2) {
         const bool two = fa.K - j0 >= 2;
         if (stage == 1) {
-            if (two) hipLaunchKernelGGL((kl_pass1_all<DM, 2>), g, blk, 0, s, fa, count, j0);
-            else hipLaunchKernelGGL((kl_pass1_all<DM, 1>), g, blk, 0, s, fa, count, j0);
+            if (two) hipLaunchKernelGGL((kl_pass1_all<DM, 2, ST>), g, blk, 0, s, fa, count, j0);
+            else hipLaunchKernelGGL((kl_pass1_all<DM, 1, ST>), g, blk, 0, s, fa, count, j0);
         } else if (stage == 3) {
-            if (two) hipLaunchKernelGGL((kl_pass2_all<DM, 2>), g, blk, 0, s, fa, count, j0);
-            else hipLaunchKernelGGL((kl_pass2_all<DM, 1>), g, blk, 0, s, fa, count, j0);
+            if (two) hipLaunchKernelGGL((kl_pass2_all<DM, 2, ST>), g, blk, 0, s, fa, count, j0);
+            else hipLaunchKernelGGL((kl_pass2_all<DM, 1, ST>), g, blk, 0, s, fa, count, j0);
         } else {
-            if (two) hipLaunchKernelGGL((kl_pass3_all<DM, 2>), g, blk, 0, s, fa, count, j0);
-            else hipLaunchKernelGGL((kl_pass3_all<DM, 1>), g, blk, 0, s, fa, count, j0);
+            if (two) hipLaunchKernelGGL((kl_pass3_all<DM, 2, ST>), g, blk, 0, s, fa, count, j0);
+            else hipLaunchKernelGGL((kl_pass3_all<DM, 1, ST>), g, blk, 0, s, fa, count, j0);
         }
     }
+}
+
+// node pass `stage` over the nodes [first, first + count) of the node list, every tracer
+// in a wavefront of its own
+template <int NSB, int DM>
+static void launch_list(const FusedArgs& fa, const FusedTuning& t, hipStream_t s, int stage,
+                        int first, int count) {
+    if (!count) return;
+    const dim3 blk(64 * t.wpb), g(blocks_for(node_waves(count, fa.K), t.wpb));
+    if (stage == 1) hipLaunchKernelGGL((kl_pass1<NSB, DM>), g, blk, 0, s, fa, first, count);
+    else if (stage == 3) hipLaunchKernelGGL((kl_pass2<NSB, DM>), g, blk, 0, s, fa, first, count);
+    else hipLaunchKernelGGL((kl_pass3<NSB, DM>), g, blk, 0, s, fa, first, count);
+}
+
+// node pass `stage` (1, 3 or 4): over the node list where there is one (shallow columns in
+// one-slot kernels, several tracers sharing a wavefront on the leading nodes of at most
+// six slots; then the deep columns), else over all nodes in id order
+template <int NS, int DM>
+static void launch_nodes(const FusedArgs& fa, const FusedTuning& t, hipStream_t s, int stage) {
+    const NodeTab& tb = fa.tab;
+    if constexpr (NS == 1) {      // every plan with nl > 64 has a list
+        if (!tb.nlist) {
+            const dim3 blk(64 * t.wpb), g(blocks_for(node_waves(fa.m.N, fa.K), t.wpb));
+            if (stage == 1) hipLaunchKernelGGL((kf_pass1<1, DM>), g, blk, 0, s, fa);
+            else if (stage == 3) hipLaunchKernelGGL((kf_pass2<1, DM>), g, blk, 0, s, fa);
+            else hipLaunchKernelGGL((kf_pass3<1, DM>), g, blk, 0, s, fa);
+            return;
+        }
+    }
+    const int n6 = fa.K >= 2 && t.pair ? tb.nsix : 0;
+    if (n6) launch_shallow_multi<6, DM>(fa, t, s, stage, n6);
+    launch_list<1, DM>(fa, t, s, stage, n6, tb.nshallow - n6);
+    if (NS == 2) launch_list<2, DM>(fa, t, s, stage, tb.nshallow, fa.m.N - tb.nshallow);
 }
 
 template <int NS, int DM>
 static void launch_single(const FusedArgs& fa, const FusedTuning& t, hipStream_t s, int stage) {
     const DevMesh& m = fa.m;
     const dim3 blk(64 * t.wpb);
-    const unsigned gn = blocks_for(node_waves(m.N, fa.K), t.wpb);
-    // several tracers share the tracer-independent loads of a shallow node in one
-    // wavefront (two at a time)
-    const bool multi = DM == 6 && fa.K >= 2 && t.pair && fa.tab.nlist;
     switch (stage) {
         case 0:
             if (t.vflux_epw == 2)
                 hipLaunchKernelGGL((kf_vflux<NS, 2>), dim3(blocks_for(vflux_waves(m.D, t), t.wpb)), blk, 0, s, fa);
             else
                 hipLaunchKernelGGL((kf_vflux<NS, 4>), dim3(blocks_for(vflux_waves(m.D, t), t.wpb)), blk, 0, s, fa);
-            break;
-        case 1:
-            if (NS == 1 && multi) {
-                // nl <= 64: every column is shallow
-                launch_shallow_multi<DM>(fa, t, s, 1, fa.tab.nshallow);
-            } else if (NS == 1 && fa.tab.nlist) {
-                // nl <= 64 in the list's (visit) order
-                hipLaunchKernelGGL((kl_pass1<1, DM>), dim3(gn), blk, 0, s, fa, 0, m.N);
-            } else if (NS == 2 && fa.tab.nlist) {
-                const int ns = fa.tab.nshallow, nd = m.N - fa.tab.nshallow;
-                if (ns && multi)
-                    launch_shallow_multi<DM>(fa, t, s, 1, ns);
-                else if (ns)
-                    hipLaunchKernelGGL((kl_pass1<1, DM>), dim3(blocks_for(node_waves(ns, fa.K), t.wpb)),
-                                       blk, 0, s, fa, 0, ns);
-                if (nd) hipLaunchKernelGGL((kl_pass1<2, DM>), dim3(blocks_for(node_waves(nd, fa.K), t.wpb)),
-                                           blk, 0, s, fa, ns, nd);
-            } else {
-                hipLaunchKernelGGL((kf_pass1<NS, DM>), dim3(gn), blk, 0, s, fa);
-            }
             break;
         case 2:
             if (const int nseg = t.adfh_kc ? adfh_segments(fa.tab.ep.np, m.L, t.adfh_kc) : 0) {
@@ -1749,38 +1789,9 @@ static void launch_single(const FusedArgs& fa, const FusedTuning& t, hipStream_t
             else
                 hipLaunchKernelGGL((kf_adfh<NS, 2>), dim3(blocks_for(adfh_waves(m.D, fa.K, t), t.wpb)), blk, 0, s, fa);
             break;
-        case 3:
-        case 4: {
-            const NodeTab& tb = fa.tab;
-            if (NS == 1 && multi) {
-                launch_shallow_multi<DM>(fa, t, s, stage, tb.nshallow);
-            } else if (NS == 1 && tb.nlist) {
-                if (stage == 3) hipLaunchKernelGGL((kl_pass2<1, DM>), dim3(gn), blk, 0, s, fa, 0, m.N);
-                else hipLaunchKernelGGL((kl_pass3<1, DM>), dim3(gn), blk, 0, s, fa, 0, m.N);
-            } else if (NS == 2 && tb.nlist) {
-                const int ns = tb.nshallow, nd = m.N - tb.nshallow;
-                const unsigned g1 = blocks_for(node_waves(ns, fa.K), t.wpb);
-                const unsigned g2 = blocks_for(node_waves(nd, fa.K), t.wpb);
-                if (stage == 3) {
-                    if (ns && multi)
-                        launch_shallow_multi<DM>(fa, t, s, 3, ns);
-                    else if (ns)
-                        hipLaunchKernelGGL((kl_pass2<1, DM>), dim3(g1), blk, 0, s, fa, 0, ns);
-                    if (nd) hipLaunchKernelGGL((kl_pass2<2, DM>), dim3(g2), blk, 0, s, fa, ns, nd);
-                } else {
-                    if (ns && multi)
-                        launch_shallow_multi<DM>(fa, t, s, 4, ns);
-                    else if (ns)
-                        hipLaunchKernelGGL((kl_pass3<1, DM>), dim3(g1), blk, 0, s, fa, 0, ns);
-                    if (nd) hipLaunchKernelGGL((kl_pass3<2, DM>), dim3(g2), blk, 0, s, fa, ns, nd);
-                }
-            } else if (stage == 3) {
-                hipLaunchKernelGGL((kf_pass2<NS, DM>), dim3(gn), blk, 0, s, fa);
-            } else {
-                hipLaunchKernelGGL((kf_pass3<NS, DM>), dim3(gn), blk, 0, s, fa);
-            }
+        default:
+            launch_nodes<NS, DM>(fa, t, s, stage);
             break;
-        }
     }
 }
 

@@ -531,3 +531,21 @@ def test_column_solve_sizes(torch_dev):
         t = lambda a: torch.from_numpy(a).to(torch_dev)
         got = adv_tra_vert_impl(m, t(w_i), t(T), t(h), dt=2700.0).cpu().numpy()
         assert np.array_equal(got, O.adv_tra_vert_impl(m, w_i, T, h, dt=2700.0)), (level, nl)
+
+
+@pytest.mark.parametrize("nl,K", [(48, 2), (70, 3)])
+def test_mixed_degree_large_mesh(nl, K, torch_dev):
+    """An 8-slot mesh above the size from which nodes with up to six neighbours share
+    wavefronts between tracers and the others run in launches of their own: bitwise to
+    the phased path, shallow and deep columns, even and odd tracer counts."""
+    from fesom_jax_amd.inputs import make_case_device
+    from fesom_jax_amd.meshgen import icosahedral_mesh
+    from fesom_jax_amd.tracer_adv import advect_fct
+    import torch
+    m = icosahedral_mesh(6, nl, seed=97, degree8=60)
+    assert m.nod2D >= 16384 and np.bincount(m.edges.reshape(-1)).max() == 8
+    c = make_case_device(m, torch_dev, seed=98, tracers=("T", "S", "T")[:K])
+    args = (m, c["uv"], c["w_e"], c["helem"], c["hnode"], c["hnode_new"], c["T"], c["T_old"])
+    for a, b in zip(advect_fct(*args, dt=2700.0, path="fused"),
+                    advect_fct(*args, dt=2700.0, path="phased")):
+        assert torch.equal(a[0], b[0])
