@@ -76,9 +76,12 @@ struct fct_plan {
     // fpf holds the limiter factors as (plus, minus) pairs; fadfv the vertical
     // antidiffusive flux pass 2 computes and pass 3 reads
     double *fLO = nullptr, *fgnode = nullptr, *fadfh = nullptr, *fpf = nullptr, *fadfv = nullptr;
-    // adjoint workspace (allocated on the first fct_backward)
-    bool adj_ready = false;
+    // adjoint workspace (allocated on the first fct_backward): the column kernels' where
+    // the mesh has node tables and nl <= 128, else the flat kernels'
+    bool adj_ready = false, adj_cols = false;
     AdjointWork aw{};
+    AdjointCols ac{};
+    double* adj_LOx = nullptr;
     std::vector<int> host_edge_tri, host_updn;   // [2D] each, -1 sentinels (adjoint lists)
     // implicit vertical diffusion scratch (allocated on the first call)
     double* vd_scratch = nullptr;
@@ -281,29 +284,12 @@ int ensure_phased(fct_plan* p) {
     return FCT_OK;
 }
 
-// Adjoint workspace: the phased tape plus cotangent scratch and the element-side lists
-// (element -> (edge, up/down role) for the interior edges' gradient triangles, element
-// -> (edge, side) for the edges' two triangles), in increasing edge order.
-int ensure_adjoint(fct_plan* p) {
-    if (p->adj_ready) return FCT_OK;
-    int rc = ensure_phased(p);
-    if (rc) return rc;
+// Element-side lists of the adjoint (element -> (edge, up/down role) for the interior
+// edges' gradient triangles, element -> (edge, side) for the edges' two triangles), in
+// increasing edge order.
+int upload_element_lists(fct_plan* p, const int** ud_off, const int** ud_list, const int** et_off,
+                         const int** et_list) {
     const DevMesh& m = p->m;
-    const size_t NL = (size_t)m.N * m.L, DL = (size_t)m.D * m.L, EL = (size_t)m.E * m.L;
-    AdjointWork& w = p->aw;
-    w.vflux = p->vflux; w.LO = p->LO; w.trxy = p->trxy; w.gnode = p->gnode; w.adfh = p->adfh;
-    w.adfv = p->adfv; w.tvmax = p->tvmax; w.tvmin = p->tvmin; w.fplus = p->fplus;
-    w.fminus = p->fminus; w.pf = p->pf; w.mf = p->mf;
-    double** node[] = {&w.gLO, &w.gx, &w.ghsc, &w.g_pf, &w.g_mf, &w.g_fp, &w.g_fm, &w.g_fmax,
-                       &w.g_fmin, &w.g_adfv, &w.gA, &w.g_fv, &w.g_tvx, &w.g_tvn, &w.sh_x,
-                       &w.sh_n, &w.g_div, &w.gw};
-    for (double** q : node)
-        if ((rc = dev_alloc(p, q, NL))) return rc;
-    if ((rc = dev_alloc(p, &w.g_num, 2 * NL)) || (rc = dev_alloc(p, &w.g_adfh, DL)) ||
-        (rc = dev_alloc(p, &w.eA, 2 * DL)) || (rc = dev_alloc(p, &w.eT, 2 * DL)) ||
-        (rc = dev_alloc(p, &w.eud, 4 * DL)) || (rc = dev_alloc(p, &w.g_vf, DL)) ||
-        (rc = dev_alloc(p, &w.g_tr, 2 * EL)))
-        return rc;
     const std::vector<int>& ud = p->host_updn;
     const std::vector<int>& et = p->host_edge_tri;
     std::vector<int> ud_cnt(m.E + 1, 0), et_cnt(m.E + 1, 0);
@@ -328,10 +314,123 @@ int ensure_adjoint(fct_plan* p) {
             if (el >= 0) et_ent[ep[el]++] = 2 * e + side;
         }
     }
-    if ((rc = dev_upload(p, &w.ud_off, ud_cnt.data(), ud_cnt.size())) ||
-        (rc = dev_upload(p, &w.ud_ent, ud_ent.data(), ud_ent.size())) ||
-        (rc = dev_upload(p, &w.et_off, et_cnt.data(), et_cnt.size())) ||
-        (rc = dev_upload(p, &w.et_ent, et_ent.data(), et_ent.size())))
+    int rc;
+    if ((rc = dev_upload(p, ud_off, ud_cnt.data(), ud_cnt.size())) ||
+        (rc = dev_upload(p, ud_list, ud_ent.data(), ud_ent.size())) ||
+        (rc = dev_upload(p, et_off, et_cnt.data(), et_cnt.size())) ||
+        (rc = dev_upload(p, et_list, et_ent.data(), et_ent.size())))
+        return rc;
+    return FCT_OK;
+}
+
+bool adjoint_by_columns(const fct_plan* p) { return p->tab.dm > 0 && p->m.L <= 128; }
+
+// Rings of the column adjoint: each node's neighbours in an order in which every triangle
+// around the node joins a slot to the next one (the last to the first), with that
+// triangle's layer range lo|hi << 8 (0: no triangle there; a triangle of no layers gets
+// 0x0101, which is empty too). A closed fan that leaves table slots free repeats its first
+// neighbour behind its last; other free slots repeat the last one.
+int upload_rings(fct_plan* p, const int2** out, bool* ok) {
+    const int N = p->m.N, dm = p->tab.dm;
+    std::vector<int4> hdr(N), edge((size_t)N * dm);
+    HIPCHK(hipMemcpy(hdr.data(), p->tab.hdr, hdr.size() * sizeof(int4), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(edge.data(), p->tab.edge, edge.size() * sizeof(int4), hipMemcpyDeviceToHost));
+    std::vector<int2> ring((size_t)N * dm);
+    *ok = true;
+    for (int n = 0; n < N; ++n) {
+        const int4* es = &edge[(size_t)n * dm];
+        const int de = hdr[n].z & 0xff, ne = hdr[n].w;
+        int2* r = &ring[(size_t)n * dm];
+        int nb[8][2], rg[8][2], cnt[8] = {};     // per slot: the slots its triangles join it to
+        for (int q = 0; q < ne; ++q) {
+            const unsigned w = (unsigned)es[q].w;
+            int c[2], k = 0;
+            for (int i = 0; i < 3; ++i) {
+                const int v = (int)(w >> (16 + 4 * i)) & 0xf;
+                if (v != dm && k < 2) c[k++] = v;
+            }
+            int range = (int)(w & 0xffff);
+            if (!range) range = 0x0101;
+            if (k != 2 || cnt[c[0]] == 2 || cnt[c[1]] == 2) { *ok = false; return FCT_OK; }
+            for (int i = 0; i < 2; ++i) {
+                nb[c[i]][cnt[c[i]]] = c[1 - i];
+                rg[c[i]][cnt[c[i]]++] = range;
+            }
+        }
+        bool used[8] = {};
+        int len = 0;
+        auto walk = [&](int q) {      // from slot q along unused triangles
+            int from = -1;
+            for (;;) {
+                used[q] = true;
+                if (len == dm) { *ok = false; return; }
+                r[len].x = es[q].y;
+                r[len++].y = 0;
+                int next = -1;
+                for (int i = 0; i < cnt[q]; ++i)
+                    if (nb[q][i] != from && !used[nb[q][i]]) { next = nb[q][i]; r[len - 1].y = rg[q][i]; break; }
+                if (next < 0) return;
+                from = q;
+                q = next;
+            }
+        };
+        for (int pass = 0; pass < 2 && *ok; ++pass)       // open fans first, then a closed one
+            for (int q = 0; q < de && *ok; ++q) {
+                if (used[q] || (pass == 0 && cnt[q] == 2)) continue;
+                const int start = len;
+                walk(q);
+                if (pass == 0 || !*ok) continue;
+                // close it: the last slot's triangle with the first
+                int last = -1;
+                for (int i = 0; i < de; ++i)
+                    if (es[i].y == r[len - 1].x) last = i;
+                for (int i = 0; i < 2; ++i)
+                    if (nb[last][i] == q) r[len - 1].y = rg[last][i];
+                if (start == 0 && len == dm) break;       // wraps round the table
+                if (len == dm) { *ok = false; break; }
+                r[len++] = make_int2(r[start].x, 0);
+            }
+        if (!*ok) return FCT_OK;
+        for (int q = len; q < dm; ++q) r[q] = make_int2(len ? r[len - 1].x : n, 0);
+    }
+    return dev_upload(p, out, ring.data(), ring.size());
+}
+
+// Adjoint workspace: of the column kernels, or of the flat ones with their phased tape.
+int ensure_adjoint(fct_plan* p) {
+    if (p->adj_ready) return FCT_OK;
+    int rc;
+    const DevMesh& m = p->m;
+    const size_t NL = (size_t)m.N * m.L, DL = (size_t)m.D * m.L, EL = (size_t)m.E * m.L;
+    bool rings = adjoint_by_columns(p);
+    if (rings && (rc = upload_rings(p, &p->ac.ring, &rings))) return rc;
+    p->adj_cols = rings;
+    if (rings) {
+        AdjointCols& c = p->ac;
+        if ((rc = dev_alloc(p, &c.node, NL * adjoint_cols_node())) ||
+            (rc = dev_alloc(p, &c.edge_up, (size_t)m.D * (m.L <= 64 ? 1 : 2))) ||
+            (rc = dev_alloc(p, &c.edge, DL * adjoint_cols_edge())) ||
+            (rc = dev_alloc(p, &c.elem, EL * adjoint_cols_elem())) ||
+            (rc = upload_element_lists(p, &c.ud_off, &c.ud_ent, &c.et_off, &c.et_ent)))
+            return rc;
+        p->adj_ready = true;
+        return FCT_OK;
+    }
+    if ((rc = ensure_phased(p))) return rc;
+    AdjointWork& w = p->aw;
+    w.vflux = p->vflux; w.LO = p->LO; w.trxy = p->trxy; w.gnode = p->gnode; w.adfh = p->adfh;
+    w.adfv = p->adfv; w.tvmax = p->tvmax; w.tvmin = p->tvmin; w.fplus = p->fplus;
+    w.fminus = p->fminus; w.pf = p->pf; w.mf = p->mf;
+    double** node[] = {&w.gLO, &w.gx, &w.ghsc, &w.g_pf, &w.g_mf, &w.g_fp, &w.g_fm, &w.g_fmax,
+                       &w.g_fmin, &w.g_adfv, &w.gA, &w.g_fv, &w.g_tvx, &w.g_tvn, &w.sh_x,
+                       &w.sh_n, &w.g_div, &w.gw};
+    for (double** q : node)
+        if ((rc = dev_alloc(p, q, NL))) return rc;
+    if ((rc = dev_alloc(p, &w.g_num, 2 * NL)) || (rc = dev_alloc(p, &w.g_adfh, DL)) ||
+        (rc = dev_alloc(p, &w.eA, 2 * DL)) || (rc = dev_alloc(p, &w.eT, 2 * DL)) ||
+        (rc = dev_alloc(p, &w.eud, 4 * DL)) || (rc = dev_alloc(p, &w.g_vf, DL)) ||
+        (rc = dev_alloc(p, &w.g_tr, 2 * EL)) ||
+        (rc = upload_element_lists(p, &w.ud_off, &w.ud_ent, &w.et_off, &w.et_ent)))
         return rc;
     p->adj_ready = true;
     return FCT_OK;
@@ -1422,6 +1521,14 @@ int fct_backward(fct_plan* p, const fct_step_args* a, const fct_adjoint_args* g,
     int rc = ensure_adjoint(p);
     if (rc) return rc;
     const size_t NL = (size_t)p->m.N * p->m.L;
+    if (p->adj_cols) {
+        if (a->w_i && !p->adj_LOx && (rc = dev_alloc(p, &p->adj_LOx, NL * p->kw))) return rc;
+        FusedTape t;
+        t.kw = p->kw; t.vflux = p->vflux; t.LO = p->fLO; t.LOx = p->adj_LOx; t.gnode = p->fgnode;
+        t.adfh = p->fadfh; t.pf = p->fpf; t.adfv = p->fadfv;
+        return launch_backward_cols(p->m, p->tab, p->ekr, t, p->ac, p->tune, a, g->g_T_new, g->g_T,
+                                    g->g_T_old, g->g_uv, g->g_w_e, g->g_w_i, (hipStream_t)stream);
+    }
     if (a->w_i && !p->aw.LOx &&
         ((rc = dev_alloc(p, &p->aw.LOx, NL)) || (rc = dev_alloc(p, &p->aw.gwi, NL))))
         return rc;

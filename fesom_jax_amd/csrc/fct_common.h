@@ -174,12 +174,15 @@ int launch_vert_impl(const DevMesh& m, const double* w_i, const double* hnn, dou
                      const double* X, double* out, double* cp, double* dp, hipStream_t s);
 
 // The same through LDS (fct_column.hip), for the nl that fit (vimpl_fits), and its form
-// for K tracer slots [K][N][L] of which only wet layers hold values, in place.
+// for K tracer slots [K][N][L] of which only wet layers hold values (out may be X), and
+// the reverse mode of the latter for one tracer (nl <= 128).
 bool vimpl_fits(int L);
 int launch_vimpl(const DevMesh& m, const double* w_i, const double* hnn, double dt,
                  const double* X, double* out, hipStream_t s);
-int launch_vimpl_wet(const DevMesh& m, const double* w_i, const double* hnn, double dt, double* X,
-                     int K, hipStream_t s);
+int launch_vimpl_wet(const DevMesh& m, const double* w_i, const double* hnn, double dt,
+                     const double* X, double* out, int K, hipStream_t s);
+int launch_vimpl_reverse(const DevMesh& m, const double* w_i, const double* hnn, double dt,
+                         const double* X, double* gX, double* gwi, hipStream_t s);
 int launch_pm(const DevMesh& m, const fct_step_args* a, int j, const double* vflux,
               const double* LO, const double* tr, double* gnode, double* adfh, double* adfv,
               double* tvmax, double* tvmin, double* fplus, double* fminus, hipStream_t s);
@@ -224,6 +227,28 @@ struct AdjointWork {
 int launch_backward(const DevMesh& m, const AdjointWork& w, const fct_step_args* a,
                     const double* const* g_out, double* const* gT, double* const* gTold,
                     double* g_uv, double* g_w, double* g_wi, hipStream_t s);
+
+// The fused path's workspace as the adjoint's tape (kw tracer slots each): LO, node
+// gradients, adf_h, factors and adf_v of one step; LOx (implicit split) is LO before the
+// column solve.
+struct FusedTape {
+    int kw = 1;
+    double *vflux = nullptr, *LO = nullptr, *LOx = nullptr, *gnode = nullptr, *adfh = nullptr;
+    double *pf = nullptr, *adfv = nullptr;
+};
+// Workspace of the column adjoint (fct_adjoint_cols.hip): one tracer's cotangents, in
+// adjoint_cols_node() * N*L, ..._edge() * D*L and ..._elem() * E*L doubles, the sign
+// bits of the edges' flux (one word per 64 levels), the nodes' rings and the element-side
+// lists.
+struct AdjointCols {
+    double *node = nullptr, *edge = nullptr, *elem = nullptr;
+    uint64_t* edge_up = nullptr;
+    const int2* ring = nullptr;
+    const int *ud_off = nullptr, *ud_ent = nullptr, *et_off = nullptr, *et_ent = nullptr;
+};
+size_t adjoint_cols_node();
+size_t adjoint_cols_edge();
+size_t adjoint_cols_elem();
 
 // Launch-shape knobs of the fused path (fct_plan_set_tuning / fct_batch_set_tuning);
 // results do not depend on them.
@@ -283,6 +308,19 @@ int adfh_segments(int64_t patches, int L, int kc);
 int launch_fused(const DevMesh& m, const NodeTab& tab, const int2* ekr, const fct_step_args* a,
                  int kw, const FusedTuning& tune, double* vflux, double* LO, double* gnode,
                  double* adfh, double* pf, double* adfv, hipStream_t s);
+
+// The first passes of the fused step (edge flux at j0 = 0, LO, the implicit split's
+// solve, adf_h, limiter factors) for tracers j0 .. j0 + K - 1 (K <= tape.kw), fct_fused.hip.
+int launch_tape(const DevMesh& m, const NodeTab& tab, const int2* ekr, const fct_step_args* a,
+                int j0, int K, const FusedTuning& tune, const FusedTape& tape, hipStream_t s);
+
+// One step's backward on that tape (fct_adjoint_cols.hip; meshes with node tables,
+// nl <= 128).
+int launch_backward_cols(const DevMesh& m, const NodeTab& tab, const int2* ekr,
+                         const FusedTape& tape, const AdjointCols& w, const FusedTuning& tune,
+                         const fct_step_args* f, const double* const* g_out, double* const* gT,
+                         double* const* gTold, double* g_uv, double* g_w, double* g_wi,
+                         hipStream_t s);
 
 // Upwind-only step (fct_fused.hip).
 int launch_upwind(const DevMesh& m, const NodeTab& tab, const int2* ekr, const fct_step_args* a,

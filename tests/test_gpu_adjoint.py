@@ -221,3 +221,43 @@ def test_adjoint_split_pi(pi_mesh, pi_case, torch_dev):
     opts = dict(w_i=w_i, Z3d=Z3d, zbar3=zb3)
     _compare("pi split", _gpu(pi_mesh, c, Ts, Tos, gs, torch_dev, **opts),
              _oracle(pi_mesh, c, Ts, Tos, gs, **opts))
+
+
+@pytest.mark.parametrize("level,nl,degree8,scattered,K,split", [
+    (2, 12, 0, False, 1, False), (3, 64, 0, True, 2, False), (3, 65, 0, False, 2, True),
+    (4, 70, 20, False, 1, True), (4, 48, 20, True, 3, False), (3, 128, 0, False, 1, True),
+    (3, 23, 0, False, 5, True)])
+def test_column_adjoint_forms(level, nl, degree8, scattered, K, split, torch_dev):
+    """The wavefront-per-column backward over the meshes it takes: nl at and either side
+    of the 64-lane slot and at its largest, 6- and 8-slot tables, scattered numbering,
+    more tracers than the plan has slots (5 of 4), with the limiter active; the oracle's
+    cotangents to the module's tolerance."""
+    from fesom_jax_amd.inputs import make_case
+    from fesom_jax_amd.meshgen import icosahedral_mesh, shuffled
+    m = icosahedral_mesh(level, nl, seed=101, degree8=degree8)
+    if scattered:
+        m = shuffled(m, 102)
+    c = sharp_case(m, make_case(m, seed=103, dt=2700.0), 1.5)
+    Ts = [c["T"][0] * (1.0 + 0.1 * j) for j in range(K)]
+    Tos = [c["T_old"][0] + 0.2 * j for j in range(K)]
+    opts = {}
+    if split:
+        w_i, Z3d, zb3 = _split(m, c, 104)
+        opts = dict(w_i=w_i, Z3d=Z3d, zbar3=zb3)
+    gs = _cot(m, K, 105)
+    _compare(f"icosa{level} nl{nl}", _gpu(m, c, Ts, Tos, gs, torch_dev, **opts),
+             _oracle(m, c, Ts, Tos, gs, **opts))
+
+
+def test_flat_adjoint_of_long_columns(torch_dev):
+    """Meshes that the column kernels do not take (nl > 128) keep the flat backward."""
+    from fesom_jax_amd.inputs import make_case
+    from fesom_jax_amd.meshgen import icosahedral_mesh
+    m = icosahedral_mesh(2, 130, seed=106)
+    c = sharp_case(m, make_case(m, seed=107, dt=2700.0), 1.5)
+    w_i, Z3d, zb3 = _split(m, c, 108)
+    gs = _cot(m, 2, 109)
+    Ts, Tos = [c["T"][0], 1.1 * c["T"][0]], [c["T_old"][0]] * 2
+    for opts in ({}, dict(w_i=w_i, Z3d=Z3d, zbar3=zb3)):
+        _compare("icosa2 nl130", _gpu(m, c, Ts, Tos, gs, torch_dev, **opts),
+                 _oracle(m, c, Ts, Tos, gs, **opts))
