@@ -1093,7 +1093,7 @@ extern "C" {
 int fct_impl_vert_diff(fct_plan* p, const fct_vdiff_args* a, void* stream) {
     int rc = check_vdiff(p, a);
     if (rc) return rc;
-    if (!p->vd_scratch) {
+    if (!p->vd_scratch && !vdiff_fits(p->m.L)) {
         int cus = 0;
         HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device));
         int grid = 0;
@@ -1107,6 +1107,7 @@ int fct_impl_vert_diff(fct_plan* p, const fct_vdiff_args* a, void* stream) {
 int fct_impl_vert_diff_static(fct_plan* p, const fct_vdiff_args* a, void* stream) {
     int rc = check_vdiff(p, a);
     if (rc) return rc;
+    if (vdiff_fits(p->m.L)) return run_vdiff(p, a, 0, nullptr, (hipStream_t)stream);
     // workgroups: as many as the fixed scratch has slots for, at most the resident count
     const size_t slot = vdiff_scratch_doubles(p->m.L, 1);
     const size_t slots = (size_t)FCT_VDIFF_STATIC_BYTES / sizeof(double) / slot;

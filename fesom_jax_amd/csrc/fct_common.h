@@ -380,6 +380,9 @@ struct VdiffCall {
     int floor_j = -1;               // index within the call, -1 = none
     double floor_v = 0.0;
 };
+// Whether columns of L levels fit LDS; launch_vdiff then needs no scratch (and ignores
+// max_grid and scratch).
+bool vdiff_fits(int L);
 // Workgroups the GPU holds at once over every kernel variant (cus compute units).
 int vdiff_max_grid(int cus, int* out);
 size_t vdiff_scratch_doubles(int L, int grid);

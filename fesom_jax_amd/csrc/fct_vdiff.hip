@@ -3,7 +3,8 @@
 // the optional lower bound on wet layers that the step applies to salinity right after
 // it (step.py:456).
 //
-// Mapping: a workgroup is one 64-lane wavefront; lane = node column. The Thomas
+// Columns that fit LDS (nl up to about 980) take k_vdiff_lds below; k_vdiff is for longer
+// ones. Its mapping: a workgroup is one 64-lane wavefront; lane = node column. The Thomas
 // recurrence (ops.py:121-168) runs down each lane's column in the reference's operation
 // order, over the rows [0, Lw) where Lw is the deepest bottom in the wavefront (rows
 // further down are dry in every lane and solve to +0 in the reference too). The inputs
@@ -20,7 +21,8 @@
 #include <mutex>
 #include <vector>
 
-#include "fct_common.h"
+#include "fct_column.h"
+#include "fct_wave.h"
 
 namespace fct {
 namespace {
@@ -378,6 +380,169 @@ int vd_launch(const VdArgs& a, int grid, hipStream_t s) {
     return check_launch("k_vdiff");
 }
 
+// ---- columns that fit LDS --------------------------------------------------------------
+// The same rows and recurrence, C columns per workgroup, cp and dp in LDS (fct_column.hip).
+// Rows are formed by one wavefront per column with lane = level, four columns' loads at
+// once, k-1 and k+1 values by lane shifts; a column whose wet layers reach lane 63 goes
+// level by level with loads of its neighbours instead. icosa-8 x 70, two tracers: 1005 us
+// by k_vdiff (64-byte pieces of rows, one wavefront per SIMD, cp and dp through memory),
+// 685 here (494 without the recurrence: what remains is phases that four workgroups per
+// CU do not overlap), 718 with one thread per value and neighbour loads, 954 with the neighbours through LDS
+// (three more barriers, 130 registers).
+// One row's inputs -> the row in LDS (tracer_diff.py:84-125).
+template <int K, bool SW>
+__device__ __forceinline__ void vd_row(const VdArgs& a, double* s, int S, bool surf, bool bot,
+                                       double kc, double kn, double ac, double an, double av,
+                                       double h, double zm, double zc, double zn,
+                                       const double (&tm)[K], const double (&tc)[K],
+                                       const double (&tn)[K], const double (&wc)[K],
+                                       const double (&wn)[K], const double (&bc)[K]) {
+    const double dZu = nz_safe(zm - zc), dZd = nz_safe(zc - zn);
+    const double sav = av > 0.0 ? av : 1.0;
+    const double af = -kc * a.dt / dZu * (ac / sav);
+    const double an_sav = an / sav;
+    const double cf = -kn * a.dt / dZd * an_sav;
+    const double ca = surf ? 0.0 : af, cc = bot ? 0.0 : cf;
+    s[0] = ca;
+    s[S] = -ca - cc + h;
+    s[2 * S] = cc;
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        double rhs = ca * (tc[j] - tm[j]) + cc * (tc[j] - tn[j]);
+        if (a.bc[j]) rhs = rhs + (surf ? bc[j] : 0.0);
+        if (SW && a.sw[j]) rhs = rhs + (wc[j] - wn[j] * an_sav) * a.dt;
+        s[(3 + j) * S] = rhs;
+    }
+}
+
+constexpr int VD_Q = 4;       // columns per wavefront at most
+template <int K, bool Z3D, bool SW>
+__global__ void __launch_bounds__(256) k_vdiff_lds(DevMesh m, VdArgs a, int C) {
+    extern __shared__ double sh[];
+    const int L = m.L, P = (L + 1) | 1, S = C * P;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = blockIdx.x * C;
+    const int nc = min(C, m.N - n0);
+    const gp<const double> Zp = glb(a.Zp);
+    int2 nr[VD_Q];
+    double tc[VD_Q][K];
+    {
+        double kc[VD_Q], ac[VD_Q], av[VD_Q], h[VD_Q], zc[VD_Q], wc[VD_Q][K], bc[VD_Q][K];
+        const double zs = Z3D ? 0.0 : Zp[min(lane, L - 1)];
+#pragma unroll
+        for (int q = 0; q < VD_Q; ++q) {
+            const int c = wv + 4 * q;
+            nr[q] = c < nc ? m.nlev[n0 + c] : make_int2(0, 0);
+        }
+#pragma unroll
+        for (int q = 0; q < VD_Q; ++q) {
+            const int c = wv + 4 * q;
+            const size_t i = (size_t)(n0 + (c < nc ? c : 0)) * L + lane;
+            const bool rd = c < nc && lane < L, on = rd && lane <= nr[q].y && lane >= nr[q].x;
+            kc[q] = ac[q] = av[q] = h[q] = 0.0;
+            zc[q] = zs;
+#pragma unroll
+            for (int j = 0; j < K; ++j) {
+                tc[q][j] = rd ? glb(a.T[j])[i] : 0.0;
+                wc[q][j] = bc[q][j] = 0.0;
+            }
+            if (on) {      // wet layers and the bottom interface
+                kc[q] = glb(a.Kv)[i];
+                ac[q] = glb(a.area)[i];
+                av[q] = glb(a.av)[i];
+                h[q] = glb(a.hnn)[i];
+#pragma unroll
+                for (int j = 0; j < K; ++j) {
+                    if (SW && a.sw[j]) wc[q][j] = glb(a.sw[j])[i];
+                    if (a.bc[j]) bc[q][j] = glb(a.bc[j])[n0 + c];
+                }
+            }
+            if (Z3D && rd) zc[q] = glb(a.Z3d)[i];
+        }
+#pragma unroll
+        for (int q = 0; q < VD_Q; ++q) {
+            // all lanes active; levels past the column are not used (a column with
+            // nr.y > 63 is redone below)
+            const double kn = wave_next(kc[q], 0.0), an = wave_next(ac[q], 0.0);
+            const double zm = wave_prev(zc[q], zc[q]), zn = wave_next(zc[q], 0.0);
+            double tm[K], tn[K], wn[K];
+#pragma unroll
+            for (int j = 0; j < K; ++j) {
+                tm[j] = wave_prev(tc[q][j], tc[q][j]);
+                tn[j] = wave_next(tc[q][j], 0.0);
+                wn[j] = SW ? wave_next(wc[q][j], 0.0) : 0.0;
+            }
+            const int c = wv + 4 * q;
+            if (c < nc && in_layer(nr[q], lane))
+                vd_row<K, SW>(a, sh + c * P + lane, S, lane == nr[q].x, lane == nr[q].y - 1, kc[q],
+                              kn, ac[q], an, av[q], h[q], zm, zc[q], lane + 1 < L ? zn : 0.0, tm,
+                              tc[q], tn, wc[q], wn, bc[q]);
+        }
+    }
+#pragma unroll 1
+    for (int c = wv; c < nc; c += 4) {
+        const int2 r = m.nlev[n0 + c];
+        if (r.y <= 63) continue;
+        const size_t b0 = (size_t)(n0 + c) * L;
+        for (int k = 63 + lane; k < r.y; k += 64) {
+            if (k < r.x) continue;
+            const bool nx = k + 1 < L;
+            const size_t i = b0 + k, in = nx ? i + 1 : i, im = i - 1;
+            double tm[K], t0[K], tn[K], w0[K], wn[K], bc[K];
+#pragma unroll
+            for (int j = 0; j < K; ++j) {
+                tm[j] = glb(a.T[j])[im]; t0[j] = glb(a.T[j])[i]; tn[j] = nx ? glb(a.T[j])[in] : 0.0;
+                w0[j] = wn[j] = 0.0;
+                if (SW && a.sw[j]) { w0[j] = glb(a.sw[j])[i]; wn[j] = nx ? glb(a.sw[j])[in] : 0.0; }
+                bc[j] = a.bc[j] ? glb(a.bc[j])[n0 + c] : 0.0;
+            }
+            const double zm = Z3D ? glb(a.Z3d)[im] : Zp[k - 1], zc = Z3D ? glb(a.Z3d)[i] : Zp[k];
+            const double zn = !nx ? 0.0 : (Z3D ? glb(a.Z3d)[in] : Zp[k + 1]);
+            vd_row<K, SW>(a, sh + c * P + k, S, k == r.x, k == r.y - 1, glb(a.Kv)[i],
+                          nx ? glb(a.Kv)[in] : 0.0, glb(a.area)[i], nx ? glb(a.area)[in] : 0.0,
+                          glb(a.av)[i], glb(a.hnn)[i], zm, zc, zn, tm, t0, tn, w0, wn, bc);
+        }
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < nc * K) {
+        const int c = (int)threadIdx.x / K, j = (int)threadIdx.x - c * K;
+        const int2 r = m.nlev[n0 + c];
+        double* A = sh + c * P;
+        thomas_column(A, A + S, A + 2 * S, A + (3 + j) * S, r.x, r.y);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < VD_Q; ++q) {
+        const int c = wv + 4 * q;
+        if (c >= nc) break;
+        const size_t b0 = (size_t)(n0 + c) * L;
+        for (int k = lane; k < L; k += 64) {
+            const bool wet = in_layer(nr[q], k);
+#pragma unroll
+            for (int j = 0; j < K; ++j) {
+                const double t = k < 64 ? tc[q][j] : glb(a.T[j])[b0 + k];
+                double out = t + (wet ? sh[(3 + j) * S + c * P + k] : 0.0);
+                if (j == a.floor_j && wet) out = out < a.floor_v ? a.floor_v : out;
+                glb(a.Tn[j])[b0 + k] = out;
+            }
+        }
+    }
+}
+
+template <int K, bool Z3D, bool SW>
+int vd_lds_launch(const DevMesh& m, const VdArgs& a, hipStream_t s) {
+    const int C = std::min(vi_columns(m.L, 3 + K), 4 * VD_Q);
+    const size_t lds = ((size_t)(3 + K) * C * vi_pitch(m.L) + VI_SLACK) * sizeof(double);
+    k_vdiff_lds<K, Z3D, SW><<<dim3((m.N + C - 1) / C), dim3(256), lds, s>>>(m, a, C);
+    return check_launch("k_vdiff_lds");
+}
+
+template <int K>
+int vd_lds_dispatch(const DevMesh& m, const VdArgs& a, bool z3d, bool sw, hipStream_t s) {
+    if (z3d) return sw ? vd_lds_launch<K, true, true>(m, a, s) : vd_lds_launch<K, true, false>(m, a, s);
+    return sw ? vd_lds_launch<K, false, true>(m, a, s) : vd_lds_launch<K, false, false>(m, a, s);
+}
+
 template <int K>
 int vd_dispatch(const VdArgs& a, bool z3d, bool sw, int grid, hipStream_t s) {
     if (z3d) return sw ? vd_launch<K, true, true>(a, grid, s) : vd_launch<K, true, false>(a, grid, s);
@@ -391,6 +556,8 @@ int vd_resident_k(bool z3d, bool sw, int cus, int* out) {
 }
 
 }  // namespace
+
+bool vdiff_fits(int L) { return vi_columns(L, 5) >= 1; }
 
 int vdiff_max_grid(int cus, int* out) {
     int best = 0;
@@ -435,6 +602,9 @@ int launch_vdiff(const DevMesh& m, const VdiffCall& c, int max_grid, double* scr
         sw = sw || c.sw[j] != nullptr;
     }
     if (a.nblk == 0) return FCT_OK;
+    if (vdiff_fits(m.L))
+        return c.K == 1 ? vd_lds_dispatch<1>(m, a, c.Z3d != nullptr, sw, s)
+                        : vd_lds_dispatch<2>(m, a, c.Z3d != nullptr, sw, s);
     const int grid = std::min(a.nblk, max_grid);
     return c.K == 1 ? vd_dispatch<1>(a, c.Z3d != nullptr, sw, grid, s)
                     : vd_dispatch<2>(a, c.Z3d != nullptr, sw, grid, s);

@@ -156,3 +156,28 @@ def test_rejects_bad_arguments(pi_mesh, pi_case, torch_dev):
     with pytest.raises(ValueError):
         diffuse_tracers(m, [T0], Kv, t(c["hnode_new"]),
                         out=[t(np.asfortranarray(c["T"][0])).t().contiguous().t()])
+
+
+@pytest.mark.parametrize("level,nl,K,moving", [(2, 3, 1, False), (3, 63, 2, True), (3, 64, 1, False),
+                                               (3, 65, 2, False), (3, 66, 2, True), (3, 128, 1, True),
+                                               (2, 500, 2, False), (1, 1300, 2, True)])
+def test_column_sizes(level, nl, K, moving, torch_dev):
+    """The LDS solve at the edges of its mapping: nl either side of the 64 lanes (columns
+    that end at lane 63 and past it), few columns per workgroup, a remainder of columns,
+    and an nl whose columns do not fit LDS (the kernel with memory scratch)."""
+    from fesom_jax_amd.meshgen import icosahedral_mesh
+    from fesom_jax_amd.tracer_diff import diffuse_tracers
+    m = icosahedral_mesh(level, nl, seed=111, min_levels=2, polar_cap_deg=60.0)
+    t = _t(torch_dev)
+    rng = np.random.default_rng(112)
+    h = np.where(m.node_layer_mask, 5.0 + 40.0 * rng.random(m.area.shape), 0.0)
+    Ts = [10.0 + rng.standard_normal(m.area.shape) for _ in range(K)]
+    Kv = _kv(m, 113)
+    bc, sw = _forcing(m, 114)
+    Z3d = np.concatenate([m.Z, m.Z[-1:]])[None, :] * (1.0 + 0.05 * rng.random((m.nod2D, 1)))
+    Z = dict(Z3d=Z3d) if moving else {}
+    got = diffuse_tracers(m, [t(T) for T in Ts], t(Kv), t(h), dt=2700.0, bc_surf=[t(bc)] * K,
+                          sw_3d=[t(sw)] + [None] * (K - 1), **{k: t(v) for k, v in Z.items()})
+    for j in range(K):
+        _eq(got[j], VD.impl_vert_diff_one(m, Ts[j], Kv, h, dt=2700.0, bc_surf=bc,
+                                          sw_3d=sw if j == 0 else None, **Z), (nl, j))
