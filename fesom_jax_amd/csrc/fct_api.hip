@@ -89,6 +89,7 @@ struct fct_plan {
     // sea-ice FCT workspace and element table (allocated on the first call)
     double* ice_work = nullptr;
     double* ice_tab = nullptr;
+    char* ice_slots = nullptr;
 };
 
 namespace {
@@ -995,11 +996,15 @@ int fct_ice_fct_solve(fct_plan* p, const fct_ice_args* a, void* stream) {
             (rc = dev_alloc(p, &tab, ice_table_doubles(E))) ||
             (rc = dev_alloc(p, &work, ice_workspace_doubles(p->m.N))))
             return rc;
+        char* slots = nullptr;
+        if (p->tab.dm && (rc = dev_alloc(p, &slots, ice_slot_bytes(p->m.N, p->tab.dm)))) return rc;
         HIPCHK(hipMemcpy(sq, h.data(), (size_t)E * sizeof(double), hipMemcpyHostToDevice));
         // built once, on the null stream, and waited for: later calls may use any stream
         if ((rc = launch_ice_tables(p->m, sq, tab, nullptr))) return rc;
+        if (slots && (rc = launch_ice_slots(p->m, p->tab, slots, nullptr))) return rc;
         HIPCHK(hipDeviceSynchronize());
         p->ice_tab = tab;
+        p->ice_slots = slots;
         p->ice_work = work;
     }
     IceCall c;
@@ -1010,7 +1015,8 @@ int fct_ice_fct_solve(fct_plan* p, const fct_ice_args* a, void* stream) {
     c.v = a->v_ice;
     c.X[0] = a->a_ice; c.X[1] = a->m_ice; c.X[2] = a->m_snow;
     c.out[0] = a->a_new; c.out[1] = a->m_new; c.out[2] = a->ms_new;
-    return launch_ice_fct(p->m, c, p->ice_work, p->ice_tab, (hipStream_t)stream);
+    return launch_ice_fct(p->m, c, p->ice_work, p->ice_tab, p->tab.dm, p->ice_slots,
+                          (hipStream_t)stream);
 }
 
 int fct_compute_w(fct_plan* p, const double* uv, const double* helem, double* w,

@@ -353,8 +353,12 @@ size_t ice_table_doubles(int E);
 // coefficients, area, sq[e] = sqrt(elem_area[e] / 2e8) computed on the host, correctly
 // rounded), built once per plan into `tab`
 int launch_ice_tables(const DevMesh& m, const double* sq, double* tab, hipStream_t s);
-int launch_ice_fct(const DevMesh& m, const IceCall& c, double* work, const double* tab,
-                   hipStream_t s);
+// slot tables of a mesh with node tables (dm slots), ice_slot_bytes of them at `mem`
+size_t ice_slot_bytes(int N, int dm);
+int launch_ice_slots(const DevMesh& m, const NodeTab& tab, void* mem, hipStream_t s);
+// dm = 0: over the element lists, else over the slot tables
+int launch_ice_fct(const DevMesh& m, const IceCall& c, double* work, const double* tab, int dm,
+                   void* slots, hipStream_t s);
 
 // Vertical velocity from continuity (fct_ale.hip).
 // the FCT's edge volume flux alone (kf_vflux) into vflux [D][L]; fused node tables only

@@ -4,20 +4,26 @@
 //
 // Mapping: one thread per node and all three tracers per thread (the problem is 2-D;
 // the tracers share every geometry load). Each node gathers over its elements in
-// increasing element id (the node -> element CSR), which is the order of the
-// reference's scatter-add over (element, vertex); sums over an element's three
-// vertices run ((x0 + x1) + x2). Six launches: the inputs packed per node, then five
-// gather passes over the elements around every node: right-hand side + low-order
-// solve, two high-order corrections (the second also stores each node's gamma * X + d,
-// the vertex value of the antidiffusive fluxes), fluxes + bounds + ratios, limited
-// fluxes + update.
+// increasing element id, which is the order of the reference's scatter-add over (element,
+// vertex); sums over an element's three vertices run ((x0 + x1) + x2). Six launches: the
+// inputs packed per node, then five gather passes over the elements around every node:
+// right-hand side + low-order solve, two high-order corrections (the second also stores
+// each node's gamma * X + d, the vertex value of the antidiffusive fluxes), fluxes +
+// bounds + ratios, limited fluxes + update.
 //
-// Layout: every gather is per-lane scattered, so the passes are bound by the number
-// of gather instructions. The three tracers of a node sit together (dv4, the fourth
-// slot carrying the node's inverse area where a pass needs it), (u, v) as a pair, and
-// an element's vertices, open flag, gradient coefficients, volume and diffusion factor
-// in one iv4 and four dv2: a vertex costs two loads for all three tracers instead
-// of three, an element five instead of twelve.
+// On meshes with the fused node tables (ki_*) a node's neighbours and elements come from
+// tables with one row per slot ([slot][node], whole lines read), so that all its gathers
+// leave together: the vertices of its elements are its neighbours (six gathers instead of
+// eighteen), kept in the thread's own LDS column and picked by a 4-bit code per vertex. What
+// bounded the walk over the element lists (k_ice_*, kept for other meshes) was the chain
+// list entry -> element -> vertices, six times over: icosa-8 surface 371 us, 188 here
+// (ki_hi 22, at the 19 us its 200 bytes per node take; ki_rhs 50, ki_ratio 42 and ki_apply
+// 43 against 35, 22 and 21: they hold 200 registers of gathered values, so eight wavefronts
+// per CU; capped to 168 registers they spill and take twice as long).
+//
+// Layout: the three tracers of a node sit together (dv4, the fourth slot carrying the
+// node's inverse area where a pass needs it), (u, v) as a pair, and an element's gradient
+// coefficients, volume and diffusion factor in four dv2.
 
 #include <hip/hip_runtime.h>
 
@@ -366,12 +372,349 @@ __global__ void __launch_bounds__(256) k_ice_apply(IceArgs a) {
     for (int t = 0; t < ICE_K; ++t) glb(a.out[t])[n] = comp(xl, t) + acc[t];
 }
 
+// ---------------------------------------------------------------------------
+// slot tables (meshes with node tables): neighbours, elements and vertex codes per slot
+// ---------------------------------------------------------------------------
+struct IceSlots {
+    int N;
+    const int* nbr;             // [DM][N] node of the slot
+    const int* eid;             // [DM][N] element of the slot, increasing id
+    const unsigned short* code; // [DM][N] 4 bits per vertex: the slot it is, or DM the node
+                                // itself; bit 12: an open element (padding slots: not)
+    const unsigned short* open; // [N] node open (ulevels_nod2D <= 1)
+    const double* inv;          // [N] 1 / surface area
+    const double* vol;          // [E]
+};
+constexpr int ICE_TB = 128;     // threads per workgroup of the slot passes
+
+__global__ void __launch_bounds__(256) ki_slots(int N, int L, int dm, const int4* __restrict__ hdr,
+                                                const int4* __restrict__ edge,
+                                                const int4* __restrict__ elem,
+                                                const int2* __restrict__ elev,
+                                                const double* __restrict__ area, int* __restrict__ nbr,
+                                                int* __restrict__ eid, unsigned short* __restrict__ code,
+                                                unsigned short* __restrict__ open,
+                                                double* __restrict__ inv) {
+    const int n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= N) return;
+    const int4 h = hdr[n];
+    for (int q = 0; q < dm; ++q) {
+        const int4 es = edge[(size_t)n * dm + q];
+        const int e = elem[(size_t)n * dm + q].x;
+        nbr[(size_t)q * N + n] = es.y;
+        eid[(size_t)q * N + n] = e;
+        const bool on = q < h.w && elev[e].x == 0;
+        code[(size_t)q * N + n] = (unsigned short)((((unsigned)es.w >> 16) & 0xfffu) | (on ? 0x1000u : 0u));
+    }
+    open[n] = h.x == 0;
+    const double ar = area[(size_t)n * L];
+    inv[n] = 1.0 / (ar > 0 ? ar : 1.0);
+}
+
+// The thread's LDS column: row r of its DM neighbours' (and, last, its own) values.
+template <int DM>
+struct IceCol {
+    double* p;
+    __device__ __forceinline__ double& at(int row, int slot) const {
+        return p[(size_t)(row * (DM + 1) + slot) * ICE_TB];
+    }
+};
+__device__ __forceinline__ int vslot(unsigned c, int i) { return (int)(c >> (4 * i)) & 0xf; }
+template <int DM>
+__device__ __forceinline__ int own_vertex(unsigned c) {
+    return vslot(c, 0) == DM ? 0 : (vslot(c, 1) == DM ? 1 : 2);
+}
+template <int DM>
+__device__ __forceinline__ void slots_of(const IceSlots& t, int n, int (&nb)[DM], unsigned (&cd)[DM]) {
+#pragma unroll
+    for (int q = 0; q < DM; ++q) {
+        nb[q] = glb(t.nbr)[(size_t)q * t.N + n];
+        cd[q] = glb(t.code)[(size_t)q * t.N + n];
+    }
+}
+
+template <int DM>
+__global__ void __launch_bounds__(ICE_TB) ki_rhs(IceArgs a, IceSlots t) {
+    __shared__ double sh[5 * (DM + 1) * ICE_TB];
+    const int n = blockIdx.x * ICE_TB + threadIdx.x;
+    if (n >= a.N) return;
+    const IceCol<DM> col{sh + threadIdx.x};
+    int nb[DM], el[DM];
+    unsigned cd[DM];
+    slots_of<DM>(t, n, nb, cd);
+#pragma unroll
+    for (int q = 0; q < DM; ++q) el[q] = glb(t.eid)[(size_t)q * t.N + n];
+    const dv4 xn = glb(a.X)[n];
+    {
+        dv4 x[DM + 1];
+        dv2 w[DM + 1];
+#pragma unroll
+        for (int q = 0; q < DM; ++q) { x[q] = glb(a.X)[nb[q]]; w[q] = glb(a.uv)[nb[q]]; }
+        x[DM] = xn;
+        w[DM] = glb(a.uv)[n];
+#pragma unroll
+        for (int q = 0; q <= DM; ++q) {
+            col.at(0, q) = x[q].x; col.at(1, q) = x[q].y; col.at(2, q) = x[q].z;
+            col.at(3, q) = w[q].x; col.at(4, q) = w[q].y;
+        }
+    }
+    double rhs[ICE_K] = {0.0, 0.0, 0.0}, mm[ICE_K] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < DM; ++s) {
+        const size_t e = (size_t)el[s];
+        const dv2 g0 = glb(a.eg)[4 * e], g1 = glb(a.eg)[4 * e + 1];
+        const dv2 g2 = glb(a.eg)[4 * e + 2], g3 = glb(a.eg)[4 * e + 3];
+        const int v[3] = {vslot(cd[s], 0), vslot(cd[s], 1), vslot(cd[s], 2)};
+        const int q = own_vertex<DM>(cd[s]);
+        const bool on = cd[s] & 0x1000u;
+        const double dx[3] = {g0.x, g0.y, g1.x}, dy[3] = {g1.y, g2.x, g2.y};
+        const double dxq = q == 0 ? dx[0] : (q == 1 ? dx[1] : dx[2]);
+        const double dyq = q == 0 ? dy[0] : (q == 1 ? dy[1] : dy[2]);
+        const double vol = g3.x;
+        double U[3], V[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) { U[i] = col.at(3, v[i]); V[i] = col.at(4, v[i]); }
+        const double um = sum3(U[0], U[1], U[2]), vm = sum3(V[0], V[1], V[2]);
+        const double diff = a.diff * g3.y;
+        const double udn_q = um * dxq + vm * dyq;
+        double ent[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const double ta = (dxq * (um + U[j]) + dyq * (vm + V[j])) / 12.0;
+            const double tb = diff * (dxq * dx[j] + dyq * dy[j]);
+            const double udn_j = um * dx[j] + vm * dy[j];
+            const double tc = 0.5 * a.dt * (udn_q * udn_j) / 9.0;
+            ent[j] = vol * a.dt * (ta - tb - tc);
+        }
+#pragma unroll
+        for (int k = 0; k < ICE_K; ++k) {
+            const double x0 = col.at(k, v[0]), x1 = col.at(k, v[1]), x2 = col.at(k, v[2]);
+            const double c = (ent[0] * x0 + ent[1] * x1) + ent[2] * x2;
+            rhs[k] = rhs[k] + (on ? c : 0.0);
+            mm[k] = mm[k] + (on ? mm_term(vol, comp(xn, k), x0, x1, x2) : 0.0);
+        }
+    }
+    const double inv = glb(t.inv)[n];
+    const bool nc = glb(t.open)[n];
+    double xl[ICE_K], d[ICE_K];
+#pragma unroll
+    for (int k = 0; k < ICE_K; ++k) {
+        const double x = comp(xn, k);
+        xl[k] = nc ? (rhs[k] + a.gamma * mm[k]) * inv + (1.0 - a.gamma) * x : x;
+        d[k] = nc ? rhs[k] * inv : 0.0;
+    }
+    glb(a.rhs)[n] = dv4{rhs[0], rhs[1], rhs[2], 0.0};
+    glb(a.xl)[n] = dv4{xl[0], xl[1], xl[2], inv};
+    glb(a.d0)[n] = dv4{d[0], d[1], d[2], 0.0};
+}
+
+template <int DM>
+__global__ void __launch_bounds__(ICE_TB) ki_hi(IceArgs a, IceSlots t, const dv4* din, dv4* dout,
+                                                dv4* wout) {
+    __shared__ double sh[3 * (DM + 1) * ICE_TB];
+    const int n = blockIdx.x * ICE_TB + threadIdx.x;
+    if (n >= a.N) return;
+    const IceCol<DM> col{sh + threadIdx.x};
+    int nb[DM];
+    unsigned cd[DM];
+    double vol[DM];
+    slots_of<DM>(t, n, nb, cd);
+#pragma unroll
+    for (int q = 0; q < DM; ++q) vol[q] = glb(t.vol)[glb(t.eid)[(size_t)q * t.N + n]];
+    const dv4 dv = glb(din)[n], r = glb(a.rhs)[n];
+    {
+        dv4 x[DM];
+#pragma unroll
+        for (int q = 0; q < DM; ++q) x[q] = glb(din)[nb[q]];
+#pragma unroll
+        for (int q = 0; q < DM; ++q) { col.at(0, q) = x[q].x; col.at(1, q) = x[q].y; col.at(2, q) = x[q].z; }
+        col.at(0, DM) = dv.x; col.at(1, DM) = dv.y; col.at(2, DM) = dv.z;
+    }
+    double mm[ICE_K] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < DM; ++s) {
+        const bool on = cd[s] & 0x1000u;
+        const int v0 = vslot(cd[s], 0), v1 = vslot(cd[s], 1), v2 = vslot(cd[s], 2);
+#pragma unroll
+        for (int k = 0; k < ICE_K; ++k)
+            mm[k] = mm[k] + (on ? mm_term(vol[s], comp(dv, k), col.at(k, v0), col.at(k, v1), col.at(k, v2))
+                                : 0.0);
+    }
+    const double inv = glb(t.inv)[n];
+    const bool nc = glb(t.open)[n];
+    double dn[ICE_K];
+#pragma unroll
+    for (int k = 0; k < ICE_K; ++k) {
+        const double d = comp(dv, k);
+        dn[k] = nc ? d + (comp(r, k) - mm[k]) * inv : d;
+    }
+    if (dout) glb(dout)[n] = dv4{dn[0], dn[1], dn[2], 0.0};
+    if (wout) {
+        const dv4 x = glb(a.X)[n];
+        glb(wout)[n] = dv4{a.gamma * x.x + dn[0], a.gamma * x.y + dn[1], a.gamma * x.z + dn[2], inv};
+    }
+}
+
+// pp4, pm4: the ratios of the three tracers per node
+template <int DM>
+__global__ void __launch_bounds__(ICE_TB) ki_ratio(IceArgs a, IceSlots t, dv4* pp4, dv4* pm4) {
+    __shared__ double sh[3 * (DM + 1) * ICE_TB];
+    const int n = blockIdx.x * ICE_TB + threadIdx.x;
+    if (n >= a.N) return;
+    const IceCol<DM> col{sh + threadIdx.x};
+    int nb[DM];
+    unsigned cd[DM];
+    double vol[DM];
+    slots_of<DM>(t, n, nb, cd);
+#pragma unroll
+    for (int q = 0; q < DM; ++q) vol[q] = glb(t.vol)[glb(t.eid)[(size_t)q * t.N + n]];
+    const dv4 xn = glb(a.X)[n], xln = glb(a.xl)[n], wn = glb(a.w)[n];
+    dv4 xv[DM], lv[DM], wv[DM];
+#pragma unroll
+    for (int q = 0; q < DM; ++q) { xv[q] = glb(a.X)[nb[q]]; lv[q] = glb(a.xl)[nb[q]]; wv[q] = glb(a.w)[nb[q]]; }
+    const double inv = xln.w;
+    const bool nc = glb(t.open)[n];
+    double p[ICE_K], m[ICE_K];
+#pragma unroll
+    for (int k = 0; k < ICE_K; ++k) {
+#pragma unroll
+        for (int q = 0; q < DM; ++q) {
+            const double x = comp(xv[q], k), l = comp(lv[q], k);
+            col.at(0, q) = comp(wv[q], k);
+            col.at(1, q) = fmax(l, x);
+            col.at(2, q) = fmin(l, x);
+        }
+        const double xl = comp(xln, k);
+        col.at(0, DM) = comp(wn, k);
+        col.at(1, DM) = fmax(xl, comp(xn, k));
+        col.at(2, DM) = fmin(xl, comp(xn, k));
+        double fp = 0.0, fm = 0.0, hi = -INFINITY, lo = INFINITY;
+#pragma unroll
+        for (int s = 0; s < DM; ++s) {
+            const int v0 = vslot(cd[s], 0), v1 = vslot(cd[s], 1), v2 = vslot(cd[s], 2);
+            const bool on = cd[s] & 0x1000u;
+            // ice_flux with the node's own value as w[q]
+            const double su = sum3(col.at(0, v0), col.at(0, v1), col.at(0, v2)) - 3.0 * comp(wn, k);
+            const double f = on ? -su * (vol[s] * inv) / 12.0 : 0.0;
+            fp = fp + fmax(f, 0.0);
+            fm = fm + fmin(f, 0.0);
+            const double eh = fmax(fmax(col.at(1, v0), col.at(1, v1)), col.at(1, v2));
+            const double el = fmin(fmin(col.at(2, v0), col.at(2, v1)), col.at(2, v2));
+            hi = on ? fmax(hi, eh) : hi;
+            lo = on ? fmin(lo, el) : lo;
+        }
+        const double h = isfinite(hi) ? hi : 0.0, l = isfinite(lo) ? lo : 0.0;
+        const double tmax = h - xl, tmin = l - xl;
+        p[k] = fp > 0.0 ? min1(tmax / (fp > ICE_FLUX_EPS ? fp : ICE_FLUX_EPS)) : 0.0;
+        m[k] = fm < 0.0 ? min1(tmin / (fm < -ICE_FLUX_EPS ? fm : -ICE_FLUX_EPS)) : 0.0;
+        p[k] = nc ? p[k] : 0.0;
+        m[k] = nc ? m[k] : 0.0;
+    }
+    glb(pp4)[n] = dv4{p[0], p[1], p[2], 0.0};
+    glb(pm4)[n] = dv4{m[0], m[1], m[2], 0.0};
+}
+
+template <int DM>
+__global__ void __launch_bounds__(ICE_TB) ki_apply(IceArgs a, IceSlots t, const dv4* pp4,
+                                                   const dv4* pm4) {
+    __shared__ double sh[4 * (DM + 1) * ICE_TB];
+    const int n = blockIdx.x * ICE_TB + threadIdx.x;
+    if (n >= a.N) return;
+    const IceCol<DM> col{sh + threadIdx.x};
+    int nb[DM];
+    unsigned cd[DM];
+    double vol[DM];
+    slots_of<DM>(t, n, nb, cd);
+#pragma unroll
+    for (int q = 0; q < DM; ++q) vol[q] = glb(t.vol)[glb(t.eid)[(size_t)q * t.N + n]];
+    const dv4 wn = glb(a.w)[n], ppn = glb(pp4)[n], pmn = glb(pm4)[n], xl = glb(a.xl)[n];
+    dv4 wv[DM], pv[DM], mv[DM];
+#pragma unroll
+    for (int q = 0; q < DM; ++q) { wv[q] = glb(a.w)[nb[q]]; pv[q] = glb(pp4)[nb[q]]; mv[q] = glb(pm4)[nb[q]]; }
+#pragma unroll
+    for (int q = 0; q < DM; ++q) col.at(3, q) = wv[q].w;
+    col.at(3, DM) = wn.w;
+#pragma unroll
+    for (int k = 0; k < ICE_K; ++k) {
+#pragma unroll
+        for (int q = 0; q < DM; ++q) {
+            col.at(0, q) = comp(wv[q], k);
+            col.at(1, q) = comp(pv[q], k);
+            col.at(2, q) = comp(mv[q], k);
+        }
+        col.at(0, DM) = comp(wn, k);
+        col.at(1, DM) = comp(ppn, k);
+        col.at(2, DM) = comp(pmn, k);
+        double acc = 0.0;
+#pragma unroll
+        for (int s = 0; s < DM; ++s) {
+            const int v[3] = {vslot(cd[s], 0), vslot(cd[s], 1), vslot(cd[s], 2)};
+            const bool on = cd[s] & 0x1000u;
+            double w[3];
+#pragma unroll
+            for (int j = 0; j < 3; ++j) w[j] = col.at(0, v[j]);
+            const double su = sum3(w[0], w[1], w[2]);
+            // the element's factor takes each vertex's ratio by the sign of that vertex's
+            // flux (0 when the element is closed); only the node's own flux is divided
+            double ae = INFINITY, gq = 0.0;
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                const double g = -(su - 3.0 * w[j]) * (vol[s] * col.at(3, v[j]));
+                gq = v[j] == DM ? g : gq;
+                ae = fmin(ae, col.at(!on || ice_flux_nonneg(g) ? 1 : 2, v[j]));
+            }
+            acc = acc + (on ? (gq / 12.0) * ae : 0.0);
+        }
+        glb(a.out[k])[n] = comp(xl, k) + acc;
+    }
+}
+
+template <int DM>
+void ice_slot_passes(const IceArgs& a, const IceSlots& t, hipStream_t s) {
+    const dim3 grid((a.N + ICE_TB - 1) / ICE_TB), block(ICE_TB);
+    ki_rhs<DM><<<grid, block, 0, s>>>(a, t);
+    ki_hi<DM><<<grid, block, 0, s>>>(a, t, a.d0, a.d1, nullptr);
+    ki_hi<DM><<<grid, block, 0, s>>>(a, t, a.d1, nullptr, a.w);
+    // the ratios take the place of the right-hand side and of the first correction
+    ki_ratio<DM><<<grid, block, 0, s>>>(a, t, a.rhs, a.d1);
+    ki_apply<DM><<<grid, block, 0, s>>>(a, t, a.rhs, a.d1);
+}
+
 }  // namespace
 
 // rhs, xl, d0, d1, w, X as dv4, (u, v) as dv2, pp and pm: 32 doubles per node
 size_t ice_workspace_doubles(int N) { return (size_t)32 * N; }
 // el (iv4) and eg (four dv2): 10 doubles per element
 size_t ice_table_doubles(int E) { return (size_t)10 * E; }
+// inverse areas, then neighbours and elements (int), codes and open flags (16 bits)
+size_t ice_slot_bytes(int N, int dm) { return (size_t)N * (8 + 8 * dm + 2 * (dm + 1)); }
+
+namespace {
+IceSlots slots_at(const DevMesh& m, int dm, void* mem) {
+    IceSlots t{};
+    const size_t N = (size_t)m.N;
+    char* p = static_cast<char*>(mem);
+    t.N = m.N;
+    t.vol = m.earea;
+    t.inv = reinterpret_cast<double*>(p);
+    t.nbr = reinterpret_cast<int*>(p + 8 * N);
+    t.eid = t.nbr + N * dm;
+    t.code = reinterpret_cast<unsigned short*>(p + 8 * N + 8 * N * dm);
+    t.open = t.code + N * dm;
+    return t;
+}
+}  // namespace
+
+int launch_ice_slots(const DevMesh& m, const NodeTab& tab, void* mem, hipStream_t s) {
+    if (m.N == 0) return FCT_OK;
+    const IceSlots t = slots_at(m, tab.dm, mem);
+    ki_slots<<<(m.N + 255) / 256, 256, 0, s>>>(m.N, m.L, tab.dm, tab.hdr, tab.edge, tab.elem, m.elev,
+                                              m.area, const_cast<int*>(t.nbr), const_cast<int*>(t.eid),
+                                              const_cast<unsigned short*>(t.code),
+                                              const_cast<unsigned short*>(t.open),
+                                              const_cast<double*>(t.inv));
+    return check_launch("ki_slots");
+}
 
 int launch_ice_tables(const DevMesh& m, const double* sq, double* tab, hipStream_t s) {
     if (m.E == 0) return FCT_OK;
@@ -381,8 +724,8 @@ int launch_ice_tables(const DevMesh& m, const double* sq, double* tab, hipStream
     return check_launch("k_ice_tables");
 }
 
-int launch_ice_fct(const DevMesh& m, const IceCall& c, double* work, const double* tab,
-                   hipStream_t s) {
+int launch_ice_fct(const DevMesh& m, const IceCall& c, double* work, const double* tab, int dm,
+                   void* slots, hipStream_t s) {
     if (m.N == 0) return FCT_OK;
     IceArgs a{};
     a.N = m.N;
@@ -410,6 +753,12 @@ int launch_ice_fct(const DevMesh& m, const IceCall& c, double* work, const doubl
     a.pm = work + 29 * N;
     const dim3 grid((m.N + 255) / 256), block(256);
     k_ice_pack<<<grid, block, 0, s>>>(m.N, c.X[0], c.X[1], c.X[2], c.u, c.v, X, uv);
+    if (dm) {
+        const IceSlots t = slots_at(m, dm, slots);
+        if (dm == 6) ice_slot_passes<6>(a, t, s);
+        else ice_slot_passes<8>(a, t, s);
+        return check_launch("ki");
+    }
     k_ice_rhs<<<grid, block, 0, s>>>(a, m.area, m.L);
     k_ice_hi<<<grid, block, 0, s>>>(a, a.d0, a.d1, nullptr);
     k_ice_hi<<<grid, block, 0, s>>>(a, a.d1, a.d0, a.w);

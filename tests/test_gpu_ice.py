@@ -114,3 +114,20 @@ def test_ice_numpy_in_numpy_out_and_errors(pi_mesh, torch_dev):
                            ms_new=torch.empty_like(ins[0]).data_ptr())
     rc = plan.lib.fct_ice_fct_solve(plan.ptr, ctypes.byref(args), None)
     assert rc == _lib.FCT_E_INVALID
+
+
+@pytest.mark.parametrize("level,degree8,scattered", [(1, 0, False), (3, 0, True), (4, 25, False),
+                                                     (5, 100, True)])
+def test_ice_slot_tables(level, degree8, scattered, torch_dev):
+    """The slot-table passes bitwise on 6- and 8-slot meshes, coastal nodes with free slots,
+    closed elements (cavities), scattered numbering, fewer nodes than a workgroup."""
+    from fesom_jax_amd.inputs import make_ice_case
+    from fesom_jax_amd.meshgen import icosahedral_mesh, shuffled
+    m = icosahedral_mesh(level, 12, seed=121, degree8=degree8, land_fraction=0.4)
+    if scattered:
+        m = shuffled(m, 122)
+    cfg = I.IceConfig(ice_dt=4000.0)
+    c = make_ice_case(m, seed=123, speed=0.5)
+    for mesh in (m, _shelf(m)):
+        for g, w in zip(_gpu(cfg, mesh, c, torch_dev), _want(cfg, mesh, c)):
+            assert np.array_equal(g, w)
