@@ -72,10 +72,6 @@ struct ColArgs {
     double2* eg;
     double* g_vf;
     uint64_t* edge_up;
-    // [N*DM] a node's neighbours in the order in which its triangles join them: (neighbour,
-    // layer range lo|hi of the triangle between it and the next slot, the last slot's next
-    // being the first; empty if there is none)
-    const int2* ring;
     double2* g_tr;                // [E][L]
     double *gw, *gwi;             // every lane; may be null
     const int *ud_off, *ud_ent, *et_off, *et_ent;
@@ -131,7 +127,8 @@ __device__ __forceinline__ void limit_body(const ColArgs& a, int n) {
 #pragma unroll
     for (int q = 0; q < DM; ++q) {
         es[q] = ldc(a.tab.edge, (size_t)n * DM + q);
-        rg[q] = ldc(a.ring, (size_t)n * DM + q);
+        const int4 r = ldc(a.tab.ring, (size_t)n * DM + q);
+        rg[q] = make_int2(r.x, r.w & 0xffff);
     }
     double Tc[NS], Ac[NS], LOc[NS], tvx[NS], tvn[NS], ap[NS], am[NS], hp[NS], hm[NS];
     double P[NS], M[NS], fv[NS], gx[NS], cx[NS], cn[NS];
@@ -489,9 +486,12 @@ __device__ __forceinline__ void vertex_body(const ColArgs& a, int n) {
     const int4 hd = ldc(a.tab.hdr, n);
     const int2 nr = make_int2(hd.x, hd.y);
     const size_t b0 = (size_t)n * L;
-    int2 rg[DM];
+    int2 rg[DM];      // ring: neighbour, layer range of the triangle to the next slot
 #pragma unroll
-    for (int q = 0; q < DM; ++q) rg[q] = ldc(a.ring, (size_t)n * DM + q);
+    for (int q = 0; q < DM; ++q) {
+        const int4 r = ldc(a.tab.ring, (size_t)n * DM + q);
+        rg[q] = make_int2(r.x, r.w & 0xffff);
+    }
     double gLO[NS], gt[NS], Tc[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
@@ -990,7 +990,6 @@ int launch_backward_cols(const DevMesh& m, const NodeTab& tab, const int2* ekr, 
     a.eg = reinterpret_cast<double2*>(w.edge);
     a.g_vf = w.edge + 2 * DL;
     a.edge_up = w.edge_up;
-    a.ring = w.ring;
     a.g_tr = reinterpret_cast<double2*>(w.elem);
     a.gw = g_w;
     a.gwi = f->w_i ? (g_wi ? g_wi : own_wi) : nullptr;

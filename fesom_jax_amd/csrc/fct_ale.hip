@@ -9,18 +9,18 @@
 // C loop (for nz = nzmax-1 .. nzmin: w[nz] += w[nz+1]), run by one lane per column on
 // the columns staged in LDS.
 //
-// Two forms of the divergence. k_compute_w evaluates each (edge, side) term from the
-// triangles' uv and helem, so every edge term is computed at both ends of the edge.
-// k_compute_w_vf (meshes with the fused node tables) takes the terms from the FCT's
-// edge volume flux, computed once per edge by kf_vflux:
-//   term(e, k) = (v1 dx1 - u1 dy1) h1 - (v2 dx2 - u2 dy2) h2 = -vflux(e, k)
-// exactly: x - y = -(y - x) and (-x) h = -(x h) in IEEE arithmetic, and a masked
-// triangle gives +0 in both. The two can differ only in the sign of a zero, which a
-// sum that starts at +0.0 absorbs, so both kernels give the same bits.
+// Two forms of the divergence, term by term the same arithmetic in the same order.
+// k_compute_w evaluates each (edge, side) from the edge's two triangles, so that a node
+// loads every triangle around it twice. k_compute_w_tab (meshes whose nodes have rings)
+// loads each of the node's triangles once. icosa-8 x 70: 869 us with the edge terms computed
+// once per edge into memory and gathered from there (edge flux 436, gather 471, both slots
+// of every column loaded), 478 here against 278 for the compulsory bytes at the rate of a
+// copy; with (u, v, helem) taken from LDS rows by slot and four columns summed per
+// workgroup 890.
 
 #include <hip/hip_runtime.h>
 
-#include "fct_common.h"
+#include "fct_wave.h"
 
 namespace fct {
 namespace {
@@ -29,10 +29,6 @@ template <class T>
 using gp = __attribute__((address_space(1))) T*;
 template <class T>
 __device__ __forceinline__ gp<T> glb(T* p) { return (gp<T>)p; }
-// wave-uniform loads of mesh tables through the constant address space (scalar loads)
-__device__ __forceinline__ int ldc(const int* p, size_t i) {
-    return ((__attribute__((address_space(4))) const int*)p)[i];
-}
 
 // stage 2 and 3 of both kernels for node n (valid: n < nod2D), whose divergence is div.
 // Blocks are FCT_W_WPB wavefronts, one node each; every thread reaches the barriers.
@@ -87,46 +83,94 @@ __device__ __forceinline__ void finish_w(const DevMesh& m, int n, bool valid, in
     }
 }
 
-// divergence from the edge volume flux (see the top of the file); the node's edge slots
-// come from the fused node table, in the same 2e+side order as the CSR list
+// divergence from the node's own triangles (see the top of the file): the ring gives each
+// edge's two triangles at fixed slots; the terms go through the lane's LDS column into the
+// node table's 2e+side order, which is that of the CSR list. A workgroup's C columns are
+// summed up together, one per lane of its first wavefront.
 template <int NS, int DM>
-__global__ void __launch_bounds__(256) k_compute_w_vf(DevMesh m, NodeTab tab,
-                                                      const int2* ekr_, const double* vflux_,
-                                                      double* w_) {
-    const int lane = threadIdx.x & 63;
-    // the node index is wave-uniform: scalar registers, so the table loads are scalar
-    const int n0 = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
-    const bool valid = n0 < m.N;
-    const int n = valid ? n0 : m.N - 1;
-    const int L = m.L;
-    const auto vflux = glb(vflux_);
-    const int* ekr = reinterpret_cast<const int*>(ekr_);
-    const int* ent = reinterpret_cast<const int*>(tab.edge);
-    const int cnt = ldc(reinterpret_cast<const int*>(tab.hdr), 4 * (size_t)n + 2) & 0xff;
-    int code[DM], lo[DM], hi[DM];
+__global__ void __launch_bounds__(256) k_compute_w_tab(DevMesh m, NodeTab tab, int C, int remap,
+                                                       const double* uv_, const double* helem_,
+                                                       double* w_) {
+    extern __shared__ double s_w[];       // C columns of nl | 1, then the waves' terms
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int L = m.L, P = L | 1;
+    const int n0 = (int)block_tile(remap) * C;
+    const int nc = min(C, m.N - n0);
+    double* term = s_w + C * P + wv * DM * 64 + lane;
+#pragma unroll 1
+    for (int c = wv; c < nc; c += 4) {
+        const int n = n0 + c;
+        const int4 hd = ldc(tab.hdr, n);
+        int4 r[DM];
+        double4 cr[DM];
 #pragma unroll
-    for (int q = 0; q < DM; ++q) {
-        code[q] = ldc(ent, 4 * ((size_t)n * DM + q));
-        lo[q] = ldc(ekr, 2 * (size_t)(code[q] >> 1));
-        hi[q] = ldc(ekr, 2 * (size_t)(code[q] >> 1) + 1);
-    }
-    double div[NS];
+        for (int q = 0; q < DM; ++q) r[q] = ldc(tab.ring, (size_t)n * DM + q);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        const int k = lane + 64 * s;
-        const int kc = k < L ? k : L - 1;
-        double vf[DM];
+        for (int q = 0; q < DM; ++q) cr[q] = ldc(m.cross, r[q].z < 0 ? 0 : r[q].z >> 1);
 #pragma unroll
-        for (int q = 0; q < DM; ++q) vf[q] = vflux[(size_t)(code[q] >> 1) * L + kc];
-        double d = 0.0;
+        for (int s = 0; s < NS; ++s) {
+            const int k = lane + 64 * s;
+            double d = 0.0;
+            if (k < hd.y) {      // no triangle reaches below the node's wet layers
+                double2 w[DM];
+                double h[DM];
 #pragma unroll
-        for (int q = 0; q < DM; ++q) {
-            const bool use = q < cnt && k >= lo[q] && k < hi[q];
-            d = d + (use ? ((code[q] & 1) ? vf[q] : -vf[q]) : 0.0);
+                for (int q = 0; q < DM; ++q) {
+                    const size_t i = (size_t)r[q].y * L + k;
+                    w[q] = ldv(reinterpret_cast<const double2*>(uv_), i);
+                    h[q] = G(helem_)[i];
+                }
+                bool in[DM];
+#pragma unroll
+                for (int q = 0; q < DM; ++q)
+                    in[q] = q > 0 && (r[q].w & FCT_RING_DUP) ? in[q > 0 ? q - 1 : 0] : in_bytes(r[q].w, 0, k);
+#pragma unroll
+                for (int q = 0; q < DM; ++q) {
+                    if (r[q].z < 0) continue;
+                    const int b = (q + DM - 1) % DM;
+                    const bool prev = r[q].w & FCT_RING_PREV;    // the edge's triangles: (b, q) or (q, b)
+                    const double xb = prev ? cr[q].x : cr[q].z, yb = prev ? cr[q].y : cr[q].w;
+                    const double xq = prev ? cr[q].z : cr[q].x, yq = prev ? cr[q].w : cr[q].y;
+                    const double tb = in[b] ? (w[b].y * xb - w[b].x * yb) * h[b] : 0.0;
+                    const double tq = in[q] ? (w[q].y * xq - w[q].x * yq) * h[q] : 0.0;
+                    const double t = prev ? tb + -tq : tq + -tb;   // sign * where(mask, term, 0)
+                    term[((r[q].w >> 16) & 0xf) * 64] = (r[q].z & 1) ? -t : t;
+                }
+#pragma unroll
+                for (int q = 0; q < DM; ++q)
+                    if (q < (hd.z & 0xff)) d = d + term[q * 64];
+            }
+            if (k < L) s_w[c * P + k] = d;
         }
-        div[s] = d;
     }
-    finish_w<NS>(m, n, valid, lane, div, w_);
+    __syncthreads();
+    if ((int)threadIdx.x < nc) {
+        const int zmin = m.nlev[n0 + threadIdx.x].x;
+        double* col = s_w + threadIdx.x * P;
+        double acc = col[L - 1];
+#pragma unroll 8
+        for (int k = L - 2; k >= zmin; --k) {
+            acc = acc + col[k];
+            col[k] = acc;
+        }
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int c = wv; c < nc; c += 4) {
+        const int2 nr = m.nlev[n0 + c];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const int k = lane + 64 * s;
+            if (k >= L) continue;
+            const size_t i = (size_t)(n0 + c) * L + k;
+            double v = 0.0;
+            if (k >= nr.x && k <= nr.y) {
+                const double a = G(m.area)[i];
+                v = s_w[c * P + k] / (a > 0.0 ? a : 1.0);
+            }
+            G(w_)[i] = v;
+        }
+    }
 }
 
 template <int NS>
@@ -193,18 +237,20 @@ int launch_compute_w(const DevMesh& m, const double* uv, const double* helem, do
     return check_launch("k_compute_w");
 }
 
-int launch_compute_w_vf(const DevMesh& m, const NodeTab& tab, const int2* ekr,
-                        const double* vflux, double* w, hipStream_t s) {
+int launch_compute_w_tab(const DevMesh& m, const NodeTab& tab, int remap, const double* uv,
+                         const double* helem, double* w, hipStream_t s) {
     if (m.N == 0) return FCT_OK;
-    const int wpb = FCT_W_WPB;
-    const dim3 grid((m.N + wpb - 1) / wpb), block(64 * wpb);
     if (m.L > 128) return set_error(FCT_E_UNSUPPORTED, "compute_w supports nl <= 128 (got %d)", m.L);
-    if (tab.dm == 6 && m.L <= 64) k_compute_w_vf<1, 6><<<grid, block, 0, s>>>(m, tab, ekr, vflux, w);
-    else if (tab.dm == 6) k_compute_w_vf<2, 6><<<grid, block, 0, s>>>(m, tab, ekr, vflux, w);
-    else if (tab.dm == 8 && m.L <= 64) k_compute_w_vf<1, 8><<<grid, block, 0, s>>>(m, tab, ekr, vflux, w);
-    else if (tab.dm == 8) k_compute_w_vf<2, 8><<<grid, block, 0, s>>>(m, tab, ekr, vflux, w);
-    else return set_error(FCT_E_UNSUPPORTED, "compute_w from vflux needs the fused node table");
-    return check_launch("k_compute_w_vf");
+    // columns per workgroup: icosa-8 x 70 took 590, 504, 478, 526 and 698 us with 4, 8, 16,
+    // 32 and 64 (fewer: the column sums of a workgroup are exposed; more: fewer workgroups)
+    const int C = 16;
+    const dim3 grid((m.N + C - 1) / C), block(256);
+    const size_t lds = ((size_t)C * (m.L | 1) + 4 * 64 * tab.dm) * sizeof(double);
+    if (tab.dm == 6 && m.L <= 64) k_compute_w_tab<1, 6><<<grid, block, lds, s>>>(m, tab, C, remap, uv, helem, w);
+    else if (tab.dm == 6) k_compute_w_tab<2, 6><<<grid, block, lds, s>>>(m, tab, C, remap, uv, helem, w);
+    else if (m.L <= 64) k_compute_w_tab<1, 8><<<grid, block, lds, s>>>(m, tab, C, remap, uv, helem, w);
+    else k_compute_w_tab<2, 8><<<grid, block, lds, s>>>(m, tab, C, remap, uv, helem, w);
+    return check_launch("k_compute_w_tab");
 }
 
 }  // namespace fct

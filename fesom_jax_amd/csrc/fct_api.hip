@@ -78,7 +78,7 @@ struct fct_plan {
     double *fLO = nullptr, *fgnode = nullptr, *fadfh = nullptr, *fpf = nullptr, *fadfv = nullptr;
     // adjoint workspace (allocated on the first fct_backward): the column kernels' where
     // the mesh has node tables and nl <= 128, else the flat kernels'
-    bool adj_ready = false, adj_cols = false;
+    bool adj_ready = false;
     AdjointWork aw{};
     AdjointCols ac{};
     double* adj_LOx = nullptr;
@@ -268,6 +268,73 @@ bool fused_mesh_ok(const fct_mesh_desc* d, const std::vector<int>& eoff,
     return true;
 }
 
+// Ring of node n (NodeTab::ring): from its table edges `es` (de of them; .x code, .y
+// neighbour, .w >> 16 the vertex slots of element slot q), its ne elements `els` and their
+// layer ranges (es[q].w, low 16 bits). False if the fans do not fit dm slots.
+bool node_ring(const fct_mesh_desc* d, int dm, int de, int ne, const int4* es, const int* els, int4* r) {
+    int nb[8][2], el[8][2], cnt[8] = {};      // per slot: the slots its triangles join it to
+    for (int q = 0; q < ne; ++q) {
+        const unsigned w = (unsigned)es[q].w;
+        int c[2], k = 0;
+        for (int i = 0; i < 3; ++i) {
+            const int v = (int)(w >> (16 + 4 * i)) & 0xf;
+            if (v != dm && k < 2) c[k++] = v;
+        }
+        if (k != 2 || cnt[c[0]] == 2 || cnt[c[1]] == 2) return false;
+        for (int i = 0; i < 2; ++i) {
+            nb[c[i]][cnt[c[i]]] = c[1 - i];
+            el[c[i]][cnt[c[i]]++] = q;
+        }
+    }
+    int slot[8], join[8], len = 0, closed = -1;   // join: element slot to the next, -1 none
+    bool used[8] = {};
+    for (int pass = 0; pass < 2; ++pass)          // open fans first, then a closed one
+        for (int q = 0; q < de; ++q) {
+            if (used[q] || (pass == 0 && cnt[q] == 2)) continue;
+            if (closed >= 0) return false;
+            const int start = len;
+            for (int at = q, from = -1; at >= 0;) {
+                used[at] = true;
+                slot[len] = at;
+                join[len] = -1;
+                int next = -1;
+                for (int i = 0; i < cnt[at] && next < 0; ++i)
+                    if (nb[at][i] != from && !used[nb[at][i]]) {
+                        next = nb[at][i];
+                        join[len] = el[at][i];
+                    }
+                ++len;
+                from = at;
+                at = next;
+            }
+            if (pass == 0) continue;
+            for (int i = 0; i < 2; ++i)           // the triangle between the last and the first
+                if (nb[slot[len - 1]][i] == q) join[len - 1] = el[slot[len - 1]][i];
+            if (start != 0) return false;         // (its first slot's previous is the last one)
+            closed = len;
+        }
+    auto range = [&](int q) {                     // never 0 for a triangle
+        const int w = es[q].w & 0xffff;
+        return w ? w : 0x0101;
+    };
+    for (int i = 0; i < dm; ++i) {
+        if (i >= len) {   // free slots: a closed ring's first neighbour and last triangle again
+            const int s = closed >= 0 ? slot[0] : (len ? slot[len - 1] : 0);
+            const int e = closed >= 0 ? els[join[closed - 1]] : (ne ? els[0] : 0);
+            r[i] = make_int4(es[s].y, e, -1, closed >= 0 ? FCT_RING_DUP : 0);
+            continue;
+        }
+        const int4 t = es[slot[i]];
+        // the edge's first triangle is the one before it in the ring, or the one behind
+        const int prev = i > 0 ? join[i - 1] : (closed >= 0 ? join[closed - 1] : -1);
+        const bool first_prev = prev >= 0 && els[prev] == d->edge_tri[2 * (t.x >> 1)];
+        r[i] = make_int4(t.y, join[i] >= 0 ? els[join[i]] : (ne ? els[0] : 0), t.x,
+                         (join[i] >= 0 ? range(join[i]) : 0) | (slot[i] << 16) |
+                             (first_prev ? FCT_RING_PREV : 0));
+    }
+    return true;
+}
+
 // Workspace of the phased path, allocated on the first call that takes it (the fused
 // path, which batches and most callers use, never needs it).
 int ensure_phased(fct_plan* p) {
@@ -324,78 +391,7 @@ int upload_element_lists(fct_plan* p, const int** ud_off, const int** ud_list, c
     return FCT_OK;
 }
 
-bool adjoint_by_columns(const fct_plan* p) { return p->tab.dm > 0 && p->m.L <= 128; }
-
-// Rings of the column adjoint: each node's neighbours in an order in which every triangle
-// around the node joins a slot to the next one (the last to the first), with that
-// triangle's layer range lo|hi << 8 (0: no triangle there; a triangle of no layers gets
-// 0x0101, which is empty too). A closed fan that leaves table slots free repeats its first
-// neighbour behind its last; other free slots repeat the last one.
-int upload_rings(fct_plan* p, const int2** out, bool* ok) {
-    const int N = p->m.N, dm = p->tab.dm;
-    std::vector<int4> hdr(N), edge((size_t)N * dm);
-    HIPCHK(hipMemcpy(hdr.data(), p->tab.hdr, hdr.size() * sizeof(int4), hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(edge.data(), p->tab.edge, edge.size() * sizeof(int4), hipMemcpyDeviceToHost));
-    std::vector<int2> ring((size_t)N * dm);
-    *ok = true;
-    for (int n = 0; n < N; ++n) {
-        const int4* es = &edge[(size_t)n * dm];
-        const int de = hdr[n].z & 0xff, ne = hdr[n].w;
-        int2* r = &ring[(size_t)n * dm];
-        int nb[8][2], rg[8][2], cnt[8] = {};     // per slot: the slots its triangles join it to
-        for (int q = 0; q < ne; ++q) {
-            const unsigned w = (unsigned)es[q].w;
-            int c[2], k = 0;
-            for (int i = 0; i < 3; ++i) {
-                const int v = (int)(w >> (16 + 4 * i)) & 0xf;
-                if (v != dm && k < 2) c[k++] = v;
-            }
-            int range = (int)(w & 0xffff);
-            if (!range) range = 0x0101;
-            if (k != 2 || cnt[c[0]] == 2 || cnt[c[1]] == 2) { *ok = false; return FCT_OK; }
-            for (int i = 0; i < 2; ++i) {
-                nb[c[i]][cnt[c[i]]] = c[1 - i];
-                rg[c[i]][cnt[c[i]]++] = range;
-            }
-        }
-        bool used[8] = {};
-        int len = 0;
-        auto walk = [&](int q) {      // from slot q along unused triangles
-            int from = -1;
-            for (;;) {
-                used[q] = true;
-                if (len == dm) { *ok = false; return; }
-                r[len].x = es[q].y;
-                r[len++].y = 0;
-                int next = -1;
-                for (int i = 0; i < cnt[q]; ++i)
-                    if (nb[q][i] != from && !used[nb[q][i]]) { next = nb[q][i]; r[len - 1].y = rg[q][i]; break; }
-                if (next < 0) return;
-                from = q;
-                q = next;
-            }
-        };
-        for (int pass = 0; pass < 2 && *ok; ++pass)       // open fans first, then a closed one
-            for (int q = 0; q < de && *ok; ++q) {
-                if (used[q] || (pass == 0 && cnt[q] == 2)) continue;
-                const int start = len;
-                walk(q);
-                if (pass == 0 || !*ok) continue;
-                // close it: the last slot's triangle with the first
-                int last = -1;
-                for (int i = 0; i < de; ++i)
-                    if (es[i].y == r[len - 1].x) last = i;
-                for (int i = 0; i < 2; ++i)
-                    if (nb[last][i] == q) r[len - 1].y = rg[last][i];
-                if (start == 0 && len == dm) break;       // wraps round the table
-                if (len == dm) { *ok = false; break; }
-                r[len++] = make_int2(r[start].x, 0);
-            }
-        if (!*ok) return FCT_OK;
-        for (int q = len; q < dm; ++q) r[q] = make_int2(len ? r[len - 1].x : n, 0);
-    }
-    return dev_upload(p, out, ring.data(), ring.size());
-}
+bool adjoint_by_columns(const fct_plan* p) { return p->tab.ring != nullptr && p->m.L <= 128; }
 
 // Adjoint workspace: of the column kernels, or of the flat ones with their phased tape.
 int ensure_adjoint(fct_plan* p) {
@@ -403,10 +399,7 @@ int ensure_adjoint(fct_plan* p) {
     int rc;
     const DevMesh& m = p->m;
     const size_t NL = (size_t)m.N * m.L, DL = (size_t)m.D * m.L, EL = (size_t)m.E * m.L;
-    bool rings = adjoint_by_columns(p);
-    if (rings && (rc = upload_rings(p, &p->ac.ring, &rings))) return rc;
-    p->adj_cols = rings;
-    if (rings) {
+    if (adjoint_by_columns(p)) {
         AdjointCols& c = p->ac;
         if ((rc = dev_alloc(p, &c.node, NL * adjoint_cols_node())) ||
             (rc = dev_alloc(p, &c.edge_up, (size_t)m.D * (m.L <= 64 ? 1 : 2))) ||
@@ -589,6 +582,8 @@ int fct_plan_create(const fct_mesh_desc* d, fct_plan** out) {
     if (dm && (L > 128 || !fused_mesh_ok(d, h_eoff, h_ecsr, h_noff, h_ncsr))) dm = 0;
     std::vector<int4> h_thdr;
     std::vector<int4> h_tedge, h_telem;
+    std::vector<int4> h_ring;
+    bool ring_ok = true;
     bool vertex_missing = false;   // an element vertex that is not an edge neighbour
     if (dm) {
         // levels at which the adf_h pass reads a node's averaged gradient gnode: the wet
@@ -615,6 +610,7 @@ int fct_plan_create(const fct_mesh_desc* d, fct_plan** out) {
         h_thdr.resize(N);
         h_tedge.assign((size_t)N * dm, make_int4(0, 0, 0, 0));
         h_telem.assign((size_t)N * dm, make_int4(0, 0, 0, 0));
+        h_ring.resize((size_t)N * dm);
         for (int n = 0; n < N; ++n) {
             const int de = h_eoff[n + 1] - h_eoff[n], ne = h_noff[n + 1] - h_noff[n];
             const int gl = g_lo[n] < g_hi[n] ? g_lo[n] : 0, gh = g_lo[n] < g_hi[n] ? g_hi[n] : 0;
@@ -669,6 +665,9 @@ int fct_plan_create(const fct_mesh_desc* d, fct_plan** out) {
             }
             for (int q = ne; q < dm && ne > 0; ++q)
                 h_telem[(size_t)n * dm + q] = h_telem[(size_t)n * dm];
+            ring_ok = ring_ok && !vertex_missing &&
+                      node_ring(d, dm, de, ne, &h_tedge[(size_t)n * dm], &h_ncsr[h_noff[n]],
+                                &h_ring[(size_t)n * dm]);
         }
         if (vertex_missing) dm = 0;   // the fused kernels read element vertices by slot
     }
@@ -815,6 +814,7 @@ int fct_plan_create(const fct_mesh_desc* d, fct_plan** out) {
                (!h_nlist.empty() && (rc = dev_upload(p, &p->tab.nlist, h_nlist.data(), h_nlist.size()))) ||
                (rc = dev_upload(p, &m.etr, h_etr.data(), h_etr.size())) ||
                (rc = dev_upload(p, &m.udv, h_udv.data(), h_udv.size())) ||
+               (ring_ok && (rc = dev_upload(p, &p->tab.ring, h_ring.data(), h_ring.size()))) ||
                (rc = dev_upload(p, &p->tab.edge, h_tedge.data(), h_tedge.size())) ||
                (rc = dev_upload(p, &p->tab.elem, h_telem.data(), h_telem.size())))) {
         free_plan(p);
@@ -1027,11 +1027,8 @@ int fct_compute_w(fct_plan* p, const double* uv, const double* helem, double* w,
         return set_error(FCT_E_INVALID, "current device %d is not the plan's device %d", cur,
                          p->device);
     const hipStream_t s = (hipStream_t)stream;
-    if (p->tune.w_vflux && p->tab.dm && p->m.L <= 128) {
-        // edge terms once per edge into the plan's vflux workspace, then summed per node
-        int rc = launch_vflux_fused(p->m, p->tab, p->ekr, uv, helem, p->tune, p->vflux, s);
-        return rc ? rc : launch_compute_w_vf(p->m, p->tab, p->ekr, p->vflux, w, s);
-    }
+    if (p->tune.w_vflux && p->tab.ring && p->m.L <= 128)
+        return launch_compute_w_tab(p->m, p->tab, p->tune.remap(), uv, helem, w, s);
     return launch_compute_w(p->m, uv, helem, w, s);
 }
 
@@ -1528,7 +1525,7 @@ int fct_backward(fct_plan* p, const fct_step_args* a, const fct_adjoint_args* g,
     int rc = ensure_adjoint(p);
     if (rc) return rc;
     const size_t NL = (size_t)p->m.N * p->m.L;
-    if (p->adj_cols) {
+    if (adjoint_by_columns(p)) {
         if (a->w_i && !p->adj_LOx && (rc = dev_alloc(p, &p->adj_LOx, NL * p->kw))) return rc;
         FusedTape t;
         t.kw = p->kw; t.vflux = p->vflux; t.LO = p->fLO; t.LOx = p->adj_LOx; t.gnode = p->fgnode;

@@ -82,6 +82,8 @@ struct EdgePatches {
 // nodes (icosa-5 x 48) 92 us without the split, 98 with it.
 constexpr int FCT_SIX_NODES = 16384;
 
+constexpr int FCT_RING_PREV = 1 << 20, FCT_RING_DUP = 1 << 21;
+
 // Per-node stencil table of the fused path (dm slots per node).
 struct NodeTab {
     int dm = 0;               // slots per node (6 or 8); 0 = mesh not supported
@@ -92,6 +94,14 @@ struct NodeTab {
                               //  edge's triangles as bytes lo1|hi1|lo2|hi2, layer range of
                               //  element slot q as bytes lo|hi), edges in reference order
     const int4* elem;         // [N*dm] (element, v0, v1, v2), increasing element id
+    // [N*dm] the node's edges in an order in which its triangles join consecutive slots (the
+    // last slot's next being the first): (neighbour, triangle between this slot and the
+    // next, edge code 2e+side, w). w: that triangle's layer range lo|hi << 8 (0: none), the
+    // edge's slot in `edge` << 16, FCT_RING_PREV if the edge's first triangle is the one
+    // before this slot. A closed ring with slots to spare repeats its first neighbour and
+    // its last triangle there (FCT_RING_DUP, edge code -1, range 0). NULL if a node's
+    // triangles form no such ring.
+    const int4* ring = nullptr;
     // Node list of the passes: the nodes whose wet layers end above level 64 (`nshallow` of
     // them; for nl <= 64 all), in visit order, then the others; the passes take each set
     // in a launch of its own, the first with one 64-level slot per wavefront and fewer
@@ -238,12 +248,10 @@ struct FusedTape {
 };
 // Workspace of the column adjoint (fct_adjoint_cols.hip): one tracer's cotangents, in
 // adjoint_cols_node() * N*L, ..._edge() * D*L and ..._elem() * E*L doubles, the sign
-// bits of the edges' flux (one word per 64 levels), the nodes' rings and the element-side
-// lists.
+// bits of the edges' flux (one word per 64 levels) and the element-side lists.
 struct AdjointCols {
     double *node = nullptr, *edge = nullptr, *elem = nullptr;
     uint64_t* edge_up = nullptr;
-    const int2* ring = nullptr;
     const int *ud_off = nullptr, *ud_ent = nullptr, *et_off = nullptr, *et_ent = nullptr;
 };
 size_t adjoint_cols_node();
@@ -263,7 +271,7 @@ struct FusedTuning {
                         // 0 = one wavefront per edge column (kf_adfh)
     int adfh_tpe = 1;   // edge-patch kernel: threads per edge (1, 2 or 4), which split
                         // the chunk's levels
-    int w_vflux = 1;    // compute_w from the edge volume flux (1) or per node (0)
+    int w_vflux = 1;    // compute_w over the node tables (1) or the edge lists (0)
     int pair = 1;       // two tracers: shallow node passes take both in one wavefront
     // the remap as the kernels take it: XCD count in the low 8 bits, chunk above
     int remap() const { return xcd | (xchunk << 8); }
@@ -361,12 +369,8 @@ int launch_ice_fct(const DevMesh& m, const IceCall& c, double* work, const doubl
                    void* slots, hipStream_t s);
 
 // Vertical velocity from continuity (fct_ale.hip).
-// the FCT's edge volume flux alone (kf_vflux) into vflux [D][L]; fused node tables only
-int launch_vflux_fused(const DevMesh& m, const NodeTab& tab, const int2* ekr, const double* uv,
-                       const double* helem, const FusedTuning& t, double* vflux, hipStream_t s);
-// compute_w's divergence from that edge flux (exactly minus the per-edge term)
-int launch_compute_w_vf(const DevMesh& m, const NodeTab& tab, const int2* ekr,
-                        const double* vflux, double* w, hipStream_t s);
+int launch_compute_w_tab(const DevMesh& m, const NodeTab& tab, int remap, const double* uv,
+                         const double* helem, double* w, hipStream_t s);
 int launch_compute_w(const DevMesh& m, const double* uv, const double* helem, double* w,
                      hipStream_t s);
 

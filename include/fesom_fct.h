@@ -117,9 +117,9 @@ enum {
     FCT_TUNE_ADFH_EDGES = 4,        /* edges per wavefront in the adf_h pass: 1 or 2 (2)   */
     FCT_TUNE_XCD_CHUNK = 5,         /* workgroups per range of one XCD under FCT_TUNE_XCD:
                                        0 = one range per XCD, else 1..2^20 (default 8)    */
-    FCT_TUNE_W_EDGE_FLUX = 6,       /* fct_compute_w: 1 = edge terms once per edge (the
-                                       step's edge flux pass), 0 = per node from the
-                                       triangles; same bits either way (default 1)        */
+    FCT_TUNE_W_EDGE_FLUX = 6,       /* fct_compute_w: 1 = over the node tables, each
+                                       triangle around a node loaded once, 0 = over the edge
+                                       lists; same bits either way (default 1)            */
     FCT_TUNE_PAIR_TRACERS = 7,      /* nl > 64, two tracers, node degree <= 6: 1 = the
                                        shallow columns' node passes take both tracers
                                        in one wavefront, 0 = one wavefront per tracer
@@ -234,9 +234,8 @@ int fct_ice_fct_solve(fct_plan* plan, const fct_ice_args* args, void* stream);
  * w = compute_w(mesh, uv, helem) (fesom_jax/ale.py:309-365), the w_e the step takes:
  * per-level edge divergence into the nodes, cumulative sum from the bottom, divided by
  * the interface area; zero outside each node's interfaces [nzmin, nzmax]. uv is
- * [elem2D][nl][2], helem [elem2D][nl], w [nod2D][nl] (device). nl <= 128. Uses the
- * plan's edge-flux workspace, as fct_forward does: calls on one plan are ordered on one
- * stream (they race if they overlap). No allocation. */
+ * [elem2D][nl][2], helem [elem2D][nl], w [nod2D][nl] (device). nl <= 128. Uses
+ * no workspace and allocates nothing. */
 int fct_compute_w(fct_plan* plan, const double* uv, const double* helem, double* w,
                   void* stream);
 

@@ -49,6 +49,31 @@ def test_compute_w_bitwise(which, form, pi_mesh, pi_case, torch_dev):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("level,nl,degree8,scattered,land", [
+    (1, 5, 0, False, 0.3), (2, 64, 0, True, 0.6), (2, 65, 0, False, 0.3),
+    (3, 128, 10, True, 0.5), (3, 40, 10, False, 0.7)])
+def test_compute_w_over_rings(level, nl, degree8, scattered, land, torch_dev):
+    """The divergence over the nodes' rings of triangles, bit for bit to the oracle: one
+    and two 64-lane slots at their edges, 6- and 8-slot tables, 42 nodes (a workgroup that
+    is not full), coasts (open fans, several at one node) and scattered numbering; NaN in
+    dry cells stays there."""
+    from fesom_jax_amd.ale import compute_w
+    from fesom_jax_amd.inputs import make_case
+    from fesom_jax_amd.meshgen import icosahedral_mesh, shuffled
+    m = icosahedral_mesh(level, nl, seed=45, degree8=degree8, land_fraction=land, min_levels=2,
+                         polar_cap_deg=60.0)
+    if scattered:
+        m = shuffled(m, 46)
+    c = make_case(m, seed=47, dt=2700.0)
+    want = O.compute_w(m, c["uv"], c["helem"])
+    uv, he = c["uv"].copy(), c["helem"].copy()
+    uv[~m.elem_layer_mask] = np.nan
+    he[~m.elem_layer_mask] = np.nan
+    t = _t(torch_dev)
+    got = compute_w(m, t(uv), t(he)).cpu().numpy()
+    assert np.array_equal(got, want)
+
+
 def test_compute_w_numpy_in_numpy_out(pi_mesh, pi_case, torch_dev):
     from fesom_jax_amd.ale import compute_w
     w = compute_w(pi_mesh, pi_case["uv"], pi_case["helem"])
