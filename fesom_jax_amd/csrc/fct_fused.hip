@@ -1342,6 +1342,134 @@ __device__ __forceinline__ void upwind_slots(const FusedArgs& a, int n, int j, i
     }
 }
 
+// The same over the node's ring (NodeTab::ring), one 64-level slot s: each triangle of the
+// node loaded once and its edges' volume fluxes formed here, for all K tracers, so that no
+// edge flux pass runs and no flux crosses memory; the levels above and below come from the
+// neighbouring lanes (and one uniform load where the slot ends). The first tracer's columns
+// are in flight with the triangles. The terms go through the lane's LDS column into the
+// table's 2e+side order. Bound by the vector memory path (six triangles of 24 B and twelve
+// tracer columns a node) at four wavefronts per SIMD: icosa-7 x 47 187 us, 251 with
+// the edge flux pass (158 + 100); 219 with the tracer's loads behind the fluxes, 258 at five
+// wavefronts (spills). icosa-7 x 70 289 -> 234 us; with both slots of a column in registers
+// 339.
+template <bool HALO, int DM, int ST>
+__device__ __forceinline__ void upwind_ring(const FusedArgs& a, int n, int4 hd, int s, double* term) {
+    const DevMesh& m = a.m;
+    const int L = m.L;
+    const int2 nr = make_int2(hd.x, hd.y);
+    const int k = 64 * s + lane_id();
+    const size_t i = (size_t)n * L + k;
+    const size_t up = (size_t)n * L + 64 * s - 1, dn = (size_t)n * L + 64 * s + 64;
+    const bool has_up = HALO && s > 0, has_dn = HALO && 64 * s + 64 < nr.y;
+    int4 r[DM];
+    double4 cr[DM];
+#pragma unroll
+    for (int q = 0; q < DM; ++q) r[q] = ldc(a.tab.ring, (size_t)n * ST + q);
+#pragma unroll
+    for (int q = 0; q < DM; ++q) cr[q] = ldc(m.cross, r[q].z < 0 ? 0 : r[q].z >> 1);
+    double Ti, Ai, T2[DM], A2[DM], Tu, Td;
+    auto load = [&](int j) {
+        const auto T = G(a.T[j]);
+        const auto To = G(a.Told[j]);
+        Ti = Ai = Tu = Td = 0.0;
+        if (k < L) {
+            Ti = T[i];
+            Ai = To[i];
+        }
+        if (has_up) Tu = ab2(To[up], T[up]);
+        if (has_dn) Td = ab2(To[dn], T[dn]);
+        if (k < nr.y) {
+#pragma unroll
+            for (int q = 0; q < DM; ++q) {
+                const size_t c = (size_t)r[q].x * L + k;
+                T2[q] = T[c];
+                A2[q] = To[c];
+            }
+        }
+    };
+    load(0);
+    double vf[DM];
+    {
+        double2 w[DM];
+        double h[DM];
+        bool in[DM];
+        if (k < nr.y) {
+#pragma unroll
+            for (int q = 0; q < DM; ++q) {
+                const size_t c = (size_t)r[q].y * L + k;
+                w[q] = ldv(reinterpret_cast<const double2*>(a.uv), c);
+                h[q] = G(a.helem)[c];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < DM; ++q)
+            in[q] = q > 0 && (r[q].w & FCT_RING_DUP) ? in[q > 0 ? q - 1 : 0] : in_bytes(r[q].w, 0, k);
+#pragma unroll
+        for (int q = 0; q < DM; ++q) {
+            const int b = (q + DM - 1) % DM;
+            const bool prev = r[q].w & FCT_RING_PREV;   // the edge's triangles: (b, q) or (q, b)
+            const double xb = prev ? cr[q].x : cr[q].z, yb = prev ? cr[q].y : cr[q].w;
+            const double xq = prev ? cr[q].z : cr[q].x, yq = prev ? cr[q].w : cr[q].y;
+            const double tb = in[b] ? (w[b].y * xb - w[b].x * yb) * h[b] : 0.0;
+            const double tq = in[q] ? (w[q].y * xq - w[q].x * yq) * h[q] : 0.0;
+            vf[q] = prev ? tq - tb : tb - tq;           // (the first triangle's term is negated)
+        }
+    }
+    // the node's own fields
+    double w0 = 0.0, a0 = 0.0, av = 0.0, hn = 0.0, hnd = 0.0;
+    const bool wet = in_layer(nr, k);
+    if (wet) {
+        const double2 aa = ldv(m.aav, i);
+        w0 = G(a.w_e)[i]; a0 = aa.x; av = aa.y;
+        hn = G(a.hnn)[i]; hnd = G(a.hnode)[i];
+    }
+    const double w1 = wave_next(w0, has_dn ? G(a.w_e)[dn] : 0.0);
+    const double a1 = wave_next(a0, has_dn ? G(m.area)[dn] : 0.0);
+#pragma unroll 1
+    for (int j = 0;;) {
+        const auto Tn = G(a.Tnew[j]);
+        const double A = ab2(Ai, Ti);
+        const double Am = wave_prev(A, has_up ? Tu : A);   // (level 0 takes itself)
+        const double Ap = wave_next(A, Td);
+        if (wet) {
+#pragma unroll
+            for (int q = 0; q < DM; ++q) {
+                if (r[q].z < 0) continue;
+                const double v = vf[q], far = ab2(A2[q], T2[q]);
+                const bool side = r[q].z & 1;
+                const double x1 = side ? far : A, x2 = side ? A : far;
+                const double aq = fabs(v);
+                const double f = -0.5 * (x1 * (v + aq) + x2 * (v - aq));
+                term[((r[q].w >> 16) & 0xf) * 64] = v != 0.0 ? (side ? -f : f) : 0.0;
+            }
+            double raw = 0.0;
+#pragma unroll
+            for (int q = 0; q < DM; ++q)
+                if (q < (hd.z & 0xff)) raw = raw + term[q * 64];
+            double fv0, fv1 = 0.0;
+            {
+                const double aw = fabs(w0);
+                fv0 = (-0.5 * (A * (w0 + aw) + Am * (w0 - aw))) * a0;
+            }
+            if (in_layer(nr, k + 1)) {
+                const double aw = fabs(w1);
+                fv1 = (-0.5 * (Ap * (w1 + aw) + A * (w1 - aw))) * a1;
+            }
+            const double safe_a = av > 0.0 ? av : 1.0, safe_hn = hn > 0.0 ? hn : 1.0;
+            const double dttf_v = (fv0 - fv1) * a.dt / safe_a;
+            const double dttf_h = raw * a.dt / safe_a;
+            double del = dttf_h + dttf_v;
+            del = del + Ti * (hnd - hn);
+            const double dT = hn > 0.0 ? del / safe_hn : 0.0;
+            Tn[i] = Ti + dT;
+        } else if (k < L) {
+            Tn[i] = Ti + 0.0;
+        }
+        if (++j == a.K) break;
+        load(j);
+    }
+}
+
 template <int NS, int DM>
 __device__ __forceinline__ void upwind_task(const FusedArgs& a, int n, int j) {
     const int4 hd = ldc(a.tab.hdr, n);
@@ -1437,6 +1565,28 @@ FCT_NODE_KERNELS(pass3, 6)
 // Passes 2 and 3 over `count` nodes of the node list from `first`, all of whose wet
 // layers fit NSB slots: shallow columns (NSB = 1) run with fewer registers per
 // wavefront and so more wavefronts per SIMD than the two-slot body needs.
+// (occupancy on 8-slot tables, 1 % of the nodes at 8: one slot 225 us at three wavefronts,
+// 235 at four, with spills; two slots 324 and 270)
+template <int NS, int DM>
+__global__ void FCT_OCC(DM == 8 && NS == 1 ? 3 : 4) kf_upwind_ring(FusedArgs a) {
+    __shared__ double s_term[4][DM][64];
+    int n;
+    if (!single_wave(a.m.N, a.remap, n)) return;
+    const int4 hd = ldc(a.tab.hdr, n);
+    double* term = &s_term[threadIdx.x >> 6][0][lane_id()];
+#pragma unroll 1
+    for (int s = 0; s < NS; ++s) {
+        if (NS > 1 && 64 * s >= hd.y) {       // nothing wet from here on
+            for (int j = 0; j < a.K; ++j)
+                for (int k = 64 * s + lane_id(); k < a.m.L; k += 64)
+                    G(a.Tnew[j])[(size_t)n * a.m.L + k] = G(a.T[j])[(size_t)n * a.m.L + k] + 0.0;
+            break;
+        }
+        if (DM > 6 && (hd.z & 0xff) <= 6) upwind_ring<(NS > 1), 6, DM>(a, n, hd, s, term);
+        else upwind_ring<(NS > 1), DM, DM>(a, n, hd, s, term);
+    }
+}
+
 #define FCT_LIST_KERNELS(PASS, OCC1, OCC2)                                                  template <int NSB, int DM>                                                              __global__ void FCT_OCC(DM == 6 ? (NSB == 1 ? OCC1 : OCC2) : 4)                              kl_##PASS(FusedArgs a, int first, int count) {                                          int w;                                                                                  if (!single_wave((int64_t)count * a.K, a.remap, w)) return;                              const int t = w / a.K;                                                                  const int n = ldc(a.tab.nlist, (size_t)first + t);                                      const int4 hd = ldc(a.tab.hdr, n);                                                      PASS##_body<NSB, DM>(a, n, w - t * a.K, make_int2(hd.x, hd.y),                                               make_int2(hd.z & 0xff, hd.w));                                 }
 
 FCT_LIST_KERNELS(pass2, 7, 4)
@@ -1747,7 +1897,8 @@ static int launch_upwind_t(FusedArgs& fa, const fct_step_args* a, const FusedTun
                            hipStream_t s) {
     const DevMesh& m = fa.m;
     fa.K = 1;
-    if (m.D) launch_single<NS, DM>(fa, t, s, 0);
+    // (meshes with a node whose triangles make no ring: fluxes once per edge into memory)
+    if (m.D && !fa.tab.ring) launch_single<NS, DM>(fa, t, s, 0);
     int rc = check_launch("kf_vflux");
     if (rc) return rc;
     for (int j0 = 0; j0 < a->ntracers; j0 += FCT_KCHUNK) {
@@ -1757,8 +1908,10 @@ static int launch_upwind_t(FusedArgs& fa, const fct_step_args* a, const FusedTun
             const int jj = j0 + (j < K ? j : 0);
             fa.T[j] = a->T[jj]; fa.Told[j] = a->T_old[jj]; fa.Tnew[j] = a->T_new[jj];
         }
-        const unsigned gn = blocks_for(node_waves(m.N, K), t.wpb);
-        hipLaunchKernelGGL((kf_upwind<NS, DM>), dim3(gn), dim3(64 * t.wpb), 0, s, fa);
+        if (fa.tab.ring)
+            hipLaunchKernelGGL((kf_upwind_ring<NS, DM>), dim3(blocks_for(m.N, t.wpb)), dim3(64 * t.wpb), 0, s, fa);
+        else
+            hipLaunchKernelGGL((kf_upwind<NS, DM>), dim3(blocks_for(node_waves(m.N, K), t.wpb)), dim3(64 * t.wpb), 0, s, fa);
         if ((rc = check_launch("kf_upwind"))) return rc;
     }
     return FCT_OK;

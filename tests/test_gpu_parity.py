@@ -325,6 +325,38 @@ def test_upwind_step_bitwise(which, pi_mesh, pi_case, icosa4_mesh, icosa4_case, 
         assert np.array_equal(got.cpu().numpy(), want), f"{which} tracer {j}"
 
 
+@pytest.mark.parametrize("level,nl,degree8,scattered,land,K", [
+    (1, 5, 0, False, 0.3, 1), (2, 64, 0, True, 0.6, 2), (2, 65, 0, False, 0.3, 5),
+    (3, 128, 10, True, 0.5, 2), (3, 40, 10, False, 0.7, 1)])
+def test_upwind_over_rings(level, nl, degree8, scattered, land, K, torch_dev):
+    """The upwind step over the nodes' rings of triangles, bit for bit to the oracle: one
+    and two 64-lane slots at their edges, 6- and 8-slot tables, a last workgroup that is
+    not full, coasts, scattered numbering, more tracers than a launch takes; NaN in the
+    triangles' dry cells stays there."""
+    import torch
+    from fesom_jax_amd import tracer_adv
+    from fesom_jax_amd.inputs import make_case
+    from fesom_jax_amd.meshgen import icosahedral_mesh, shuffled
+    m = icosahedral_mesh(level, nl, seed=25, degree8=degree8, land_fraction=land, min_levels=2,
+                         polar_cap_deg=60.0)
+    if scattered:
+        m = shuffled(m, 26)
+    c = make_case(m, seed=27, dt=2700.0)
+    Ts = [c["T"][0] * (1.0 + 0.1 * j) for j in range(K)]
+    Tos = [0.98 * x + 0.3 for x in Ts]
+    uv, he = c["uv"].copy(), c["helem"].copy()
+    uv[~m.elem_layer_mask] = np.nan
+    he[~m.elem_layer_mask] = np.nan
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(torch_dev)
+    got = tracer_adv._run(m, t(uv), t(c["w_e"]), t(he), t(c["hnode"]), t(c["hnode_new"]),
+                          [t(x) for x in Ts], [t(x) for x in Tos], c["dt"], None, None, None,
+                          None, tracer_adv._UPWIND)
+    for j in range(K):
+        want, _ = O.advect_one(m, c["uv"], c["w_e"], c["helem"], c["hnode"], c["hnode_new"],
+                               Ts[j], Tos[j], dt=c["dt"])
+        assert np.array_equal(got[j].cpu().numpy(), want), j
+
+
 def test_small_icosa_matches_loop_oracle(torch_dev):
     """Whole path on a 162-node sphere: the GPU equals the numpy oracle bit for bit and
     the independent C loop restatement (oracle/fct_loops.c) to 1e-11, smooth and with
