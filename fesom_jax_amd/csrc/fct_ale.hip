@@ -83,13 +83,62 @@ __device__ __forceinline__ void finish_w(const DevMesh& m, int n, bool valid, in
     }
 }
 
-// divergence from the node's own triangles (see the top of the file): the ring gives each
-// edge's two triangles at fixed slots; the terms go through the lane's LDS column into the
-// node table's 2e+side order, which is that of the CSR list. A workgroup's C columns are
-// summed up together, one per lane of its first wavefront.
+// divergence of node n from its own triangles (see the top of the file) into its LDS column:
+// the ring gives each edge's two triangles at fixed slots; the terms go through the lane's
+// LDS column into the node table's 2e+side order, which is that of the CSR list. On 8-slot
+// tables a node with up to six neighbours takes the 6-slot loops.
+template <int NS, int DM, int ST>
+__device__ __forceinline__ void ring_divergence(const DevMesh& m, const NodeTab& tab, int n, int4 hd,
+                                                const double* uv_, const double* helem_,
+                                                double* term, double* col) {
+    const int lane = threadIdx.x & 63, L = m.L;
+    int4 r[DM];
+    double4 cr[DM];
+#pragma unroll
+    for (int q = 0; q < DM; ++q) r[q] = ldc(tab.ring, (size_t)n * ST + q);
+#pragma unroll
+    for (int q = 0; q < DM; ++q) cr[q] = ldc(m.cross, r[q].z < 0 ? 0 : r[q].z >> 1);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        const int k = lane + 64 * s;
+        double d = 0.0;
+        if (k < hd.y) {      // no triangle reaches below the node's wet layers
+            double2 w[DM];
+            double h[DM];
+#pragma unroll
+            for (int q = 0; q < DM; ++q) {
+                const size_t i = (size_t)r[q].y * L + k;
+                w[q] = ldv(reinterpret_cast<const double2*>(uv_), i);
+                h[q] = G(helem_)[i];
+            }
+            bool in[DM];
+#pragma unroll
+            for (int q = 0; q < DM; ++q)
+                in[q] = q > 0 && (r[q].w & FCT_RING_DUP) ? in[q > 0 ? q - 1 : 0] : in_bytes(r[q].w, 0, k);
+#pragma unroll
+            for (int q = 0; q < DM; ++q) {
+                if (r[q].z < 0) continue;
+                const int b = (q + DM - 1) % DM;
+                const bool prev = r[q].w & FCT_RING_PREV;    // the edge's triangles: (b, q) or (q, b)
+                const double xb = prev ? cr[q].x : cr[q].z, yb = prev ? cr[q].y : cr[q].w;
+                const double xq = prev ? cr[q].z : cr[q].x, yq = prev ? cr[q].w : cr[q].y;
+                const double tb = in[b] ? (w[b].y * xb - w[b].x * yb) * h[b] : 0.0;
+                const double tq = in[q] ? (w[q].y * xq - w[q].x * yq) * h[q] : 0.0;
+                const double t = prev ? tb + -tq : tq + -tb;   // sign * where(mask, term, 0)
+                term[((r[q].w >> 16) & 0xf) * 64] = (r[q].z & 1) ? -t : t;
+            }
+#pragma unroll
+            for (int q = 0; q < DM; ++q)
+                if (q < (hd.z & 0xff)) d = d + term[q * 64];
+        }
+        if (k < L) col[k] = d;
+    }
+}
+
+// A workgroup's C columns are summed up together, one per lane of its first wavefront.
 template <int NS, int DM>
 __global__ void __launch_bounds__(256) k_compute_w_tab(DevMesh m, NodeTab tab, int C, int remap,
-                                                       const double* uv_, const double* helem_,
+                                                       const double* uv, const double* helem,
                                                        double* w_) {
     extern __shared__ double s_w[];       // C columns of nl | 1, then the waves' terms
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -99,49 +148,11 @@ __global__ void __launch_bounds__(256) k_compute_w_tab(DevMesh m, NodeTab tab, i
     double* term = s_w + C * P + wv * DM * 64 + lane;
 #pragma unroll 1
     for (int c = wv; c < nc; c += 4) {
-        const int n = n0 + c;
-        const int4 hd = ldc(tab.hdr, n);
-        int4 r[DM];
-        double4 cr[DM];
-#pragma unroll
-        for (int q = 0; q < DM; ++q) r[q] = ldc(tab.ring, (size_t)n * DM + q);
-#pragma unroll
-        for (int q = 0; q < DM; ++q) cr[q] = ldc(m.cross, r[q].z < 0 ? 0 : r[q].z >> 1);
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            const int k = lane + 64 * s;
-            double d = 0.0;
-            if (k < hd.y) {      // no triangle reaches below the node's wet layers
-                double2 w[DM];
-                double h[DM];
-#pragma unroll
-                for (int q = 0; q < DM; ++q) {
-                    const size_t i = (size_t)r[q].y * L + k;
-                    w[q] = ldv(reinterpret_cast<const double2*>(uv_), i);
-                    h[q] = G(helem_)[i];
-                }
-                bool in[DM];
-#pragma unroll
-                for (int q = 0; q < DM; ++q)
-                    in[q] = q > 0 && (r[q].w & FCT_RING_DUP) ? in[q > 0 ? q - 1 : 0] : in_bytes(r[q].w, 0, k);
-#pragma unroll
-                for (int q = 0; q < DM; ++q) {
-                    if (r[q].z < 0) continue;
-                    const int b = (q + DM - 1) % DM;
-                    const bool prev = r[q].w & FCT_RING_PREV;    // the edge's triangles: (b, q) or (q, b)
-                    const double xb = prev ? cr[q].x : cr[q].z, yb = prev ? cr[q].y : cr[q].w;
-                    const double xq = prev ? cr[q].z : cr[q].x, yq = prev ? cr[q].w : cr[q].y;
-                    const double tb = in[b] ? (w[b].y * xb - w[b].x * yb) * h[b] : 0.0;
-                    const double tq = in[q] ? (w[q].y * xq - w[q].x * yq) * h[q] : 0.0;
-                    const double t = prev ? tb + -tq : tq + -tb;   // sign * where(mask, term, 0)
-                    term[((r[q].w >> 16) & 0xf) * 64] = (r[q].z & 1) ? -t : t;
-                }
-#pragma unroll
-                for (int q = 0; q < DM; ++q)
-                    if (q < (hd.z & 0xff)) d = d + term[q * 64];
-            }
-            if (k < L) s_w[c * P + k] = d;
-        }
+        const int4 hd = ldc(tab.hdr, n0 + c);
+        if (DM > 6 && (hd.z & 0xff) <= 6)
+            ring_divergence<NS, 6, DM>(m, tab, n0 + c, hd, uv, helem, term, s_w + c * P);
+        else
+            ring_divergence<NS, DM, DM>(m, tab, n0 + c, hd, uv, helem, term, s_w + c * P);
     }
     __syncthreads();
     if ((int)threadIdx.x < nc) {
@@ -241,9 +252,11 @@ int launch_compute_w_tab(const DevMesh& m, const NodeTab& tab, int remap, const 
                          const double* helem, double* w, hipStream_t s) {
     if (m.N == 0) return FCT_OK;
     if (m.L > 128) return set_error(FCT_E_UNSUPPORTED, "compute_w supports nl <= 128 (got %d)", m.L);
-    // columns per workgroup: icosa-8 x 70 took 590, 504, 478, 526 and 698 us with 4, 8, 16,
-    // 32 and 64 (fewer: the column sums of a workgroup are exposed; more: fewer workgroups)
-    const int C = 16;
+    // Columns per workgroup. Fewer leave the column sums exposed, more leave fewer workgroups:
+    // icosa-8 x 70 took 590, 504, 478, 526 and 698 us with 4, 8, 16, 32 and 64; icosa-6 x 70
+    // (29 thousand nodes) 40, 37 and 42 with 4, 8 and 16; icosa-7 x 70 on an 8-slot table,
+    // whose term rows take more of the LDS, 154, 148 and 171.
+    const int C = tab.dm == 6 && m.N >= 65536 ? 16 : 8;
     const dim3 grid((m.N + C - 1) / C), block(256);
     const size_t lds = ((size_t)C * (m.L | 1) + 4 * 64 * tab.dm) * sizeof(double);
     if (tab.dm == 6 && m.L <= 64) k_compute_w_tab<1, 6><<<grid, block, lds, s>>>(m, tab, C, remap, uv, helem, w);
