@@ -7,7 +7,8 @@
 // (kl_*): columns whose wet layers fit 64 lanes in a one-slot kernel, which needs fewer
 // registers, the others in the two-slot kernel. With two tracers on a 6-slot mesh the
 // one-slot launches take one wavefront per node for both tracers (kl_pass*_all), so the
-// tracer-independent loads are made once. Task indices are wave-uniform (scalar
+// tracer-independent loads are made once; a column of at most 32 levels holds one tracer in
+// each half of that wavefront. Task indices are wave-uniform (scalar
 // registers); each node reads its stencil (incident edges in the reference's summation
 // order with the layer ranges of their triangles, incident triangles with their
 // vertices) from a per-node table with scalar loads, and then issues the loads of all
@@ -267,12 +268,32 @@ __device__ __forceinline__ void pass1_body(const FusedArgs& a, int n, int j, int
     else pass1_slots<NS, DM, DM>(a, n, j, hd, s_nb);
 }
 
+// The pointer of tracer slot j0 + jj; half-wavefront columns: of j0 in lanes 0-31 and of
+// j0 + 1 in lanes 32-63. (As a sum: a select became a per-lane index into the kernel's
+// arguments, which put all of them into scratch memory.)
+template <bool HALF, class T>
+__device__ __forceinline__ gptr<T> lane_tracer(T* const* p, int j0, int jj) {
+    if constexpr (HALF) {
+        const uint64_t p0 = (uint64_t)p[j0], p1 = (uint64_t)p[j0 + 1];
+        return (gptr<T>)(p0 + (uint64_t)(lane_id() >> 5) * (p1 - p0));
+    }
+    return G(p[j0 + jj]);
+}
+
 // Pass 1 of a shallow node (wet layers end above level 64, one 64-level slot) for its KT
 // tracers in one wavefront: the tracer-independent loads (the edge fluxes, w, area,
 // areasvol, hnode, hnode_new) are made once; per tracer the arithmetic is pass1_body's.
 // KT is a compile-time count so that the tracer pointers are read at constant offsets.
-template <int DM, int KT, int ST>
-__device__ __forceinline__ void pass1_shallow_all(const FusedArgs& a, int n, int4 hd, int j0) {
+// HALF: a column of at most 32 levels, interfaces included, with its two tracers in the
+// wavefront's halves: half the loads, divisions and stores of a column that leaves half of
+// the lanes empty, and the mesh tables stay wave-uniform. The passes cost per wavefront
+// instruction more than per byte, so short columns (57 % of the nodes at nl = 47, 20 % at
+// 70) gain: icosa-7 x 47, pass 1 217 -> 204 us, pass 2 273 -> 237, pass 3 222 -> 187;
+// icosa-9 x 70, 2735 -> 2730, 4277 -> 3998, 3537 -> 3410. Where the wet layers pass 31 one
+// tracer does not fit a half.
+template <int DM, int KT, int ST, bool HALF>
+__device__ __forceinline__ void pass1_shallow(const FusedArgs& a, int n, int4 hd, int j0,
+                                              double (*s_nb)[ST + 1][64]) {
     const DevMesh& m = a.m;
     const int L = m.L;
     const int2 nr = make_int2(hd.x, hd.y), cnt = make_int2(hd.z & 0xff, hd.w);
@@ -286,9 +307,8 @@ __device__ __forceinline__ void pass1_shallow_all(const FusedArgs& a, int n, int
         es[q] = ldc(a.tab.edge, (size_t)n * ST + q);
         el[q] = ldc(a.tab.elem, (size_t)n * ST + q);
     }
-    __shared__ double s_nb[4][ST + 1][64];
     double* nb = &s_nb[threadIdx.x >> 6][0][lane_id()];
-    const int k = lane_id();
+    const int k = col_lane<HALF>();
     const bool rd = k < kneed;
     const bool wet = in_layer(nr, k);
     const bool gslot = glo < ghi;
@@ -304,9 +324,9 @@ __device__ __forceinline__ void pass1_shallow_all(const FusedArgs& a, int n, int
     }
     const double w1 = wave_next(w0, 0.0), a1 = wave_next(a0, 0.0);
 #pragma unroll
-    for (int jj = 0; jj < KT; ++jj) {
-        const int j = j0 + jj;   // tracer slot
-        const auto T = G(a.T[j]);
+    for (int jj = 0; jj < (HALF ? 1 : KT); ++jj) {
+        const int j = j0 + (HALF ? lane_id() >> 5 : jj);   // tracer slot
+        const auto T = lane_tracer<HALF>(a.T, j0, jj);
         const size_t jo = (size_t)j * m.N * L;
         const double Tk = rd ? T[b0 + k] : 0.0;
         double To[DM] = {};
@@ -319,7 +339,7 @@ __device__ __forceinline__ void pass1_shallow_all(const FusedArgs& a, int n, int
                 nb[ST * 64] = Tk;
             }
         }
-        const double Tm = wave_prev(Tk, Tk);
+        const double Tm = HALF ? half_prev(Tk) : wave_prev(Tk, Tk);
         const double Tp = wave_next(Tk, 0.0);
         if (!wet) continue;
         double acc = 0.0;
@@ -367,6 +387,13 @@ __device__ __forceinline__ void pass1_shallow_all(const FusedArgs& a, int n, int
         const double d = den > 0.0 ? den : 1.0;
         if (k >= glo && k < ghi) stv(a.gnode, jo + i, make_double2(nx / d, ny / d));
     }
+}
+
+template <int DM, int KT, int ST>
+__device__ __forceinline__ void pass1_shallow_all(const FusedArgs& a, int n, int4 hd, int j0) {
+    __shared__ double s_nb[4][ST + 1][64];
+    if (KT == 2 && hd.y < 32) pass1_shallow<DM, KT, ST, true>(a, n, hd, j0, s_nb);
+    else pass1_shallow<DM, KT, ST, false>(a, n, hd, j0, s_nb);
 }
 
 template <int NS, int DM>
@@ -699,7 +726,7 @@ __device__ __forceinline__ double adfv_at(int k, int2 nr, double A1, double A, d
 // Also hands back areasvol at every level (loaded with the area, clamped like it).
 // The column's w, area, areasvol, depth Z at k and interface depth at every lane
 // (clamped below the last level): the tracer-independent inputs of adfv_column.
-template <int NS>
+template <int NS, bool HALF = false>
 __device__ __forceinline__ void adfv_inputs(const FusedArgs& a, int n, double (&W)[NS],
                                             double (&ar)[NS], double (&avc)[NS],
                                             double (&Zc)[NS], double (&zb)[NS]) {
@@ -708,7 +735,7 @@ __device__ __forceinline__ void adfv_inputs(const FusedArgs& a, int n, double (&
     const size_t b0 = (size_t)n * L;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        const int k = 64 * s + lane_id();
+        const int k = 64 * s + col_lane<HALF>();
         const int kc = k < L ? k : L - 1;
         const size_t i = b0 + kc;
         W[s] = G(a.w_e)[i];
@@ -727,7 +754,7 @@ __device__ __forceinline__ void adfv_inputs(const FusedArgs& a, int n, double (&
     }
 }
 
-template <int NS>
+template <int NS, bool HALF = false>
 __device__ __forceinline__ void adfv_compute(const FusedArgs& a, int2 nr,
                                              const double (&Tc)[NS], const double (&Ac)[NS],
                                              const double (&W)[NS], const double (&ar)[NS],
@@ -735,23 +762,23 @@ __device__ __forceinline__ void adfv_compute(const FusedArgs& a, int2 nr,
                                              double (&out)[NS]) {
     const int L = a.m.L;
     double Tm[NS], A1[NS];
-    col_prev<NS>(Tc, Tm, col_bcast0<NS>(Tc));
-    col_prev<NS>(Ac, A1, col_bcast0<NS>(Ac));
+    col_prev<NS, HALF>(Tc, Tm, col_bcast0<NS>(Tc));
+    col_prev<NS, HALF>(Ac, A1, col_bcast0<NS>(Ac));
     // The reference's stencil depths (_z_stencil, tracer_adv.py:228-238) clamp Z[k-1] and
     // Z[k-2] at the top and Z[k+1] at the bottom. qc is needed at levels nr.x+1 .. nr.y-1
     // only (qd at nr.x+2 reads nr.x+1, qu at nr.y-2 reads nr.y-1): there 1 <= k <= L-2,
     // no clamp applies, and Z[k-1] is the plain lane shift of Z.
     const double z0 = col_bcast0<NS>(Zc);
     double Zm1[NS], qc[NS], qu[NS], qd[NS];
-    col_prev<NS>(Zc, Zm1, z0);
+    col_prev<NS, HALF>(Zc, Zm1, z0);
 #pragma unroll
     for (int s = 0; s < NS; ++s)
         qc[s] = 64 * s <= nr.y ? (A1[s] - Ac[s]) / nz_safe(Zm1[s] - Zc[s]) : 0.0;
     col_next<NS>(qc, qu, 0.0);
-    col_prev<NS>(qc, qd, 0.0);
+    col_prev<NS, HALF>(qc, qd, 0.0);
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        const int k = 64 * s + lane_id();
+        const int k = 64 * s + col_lane<HALF>();
         out[s] = 0.0;
         if (k <= nr.y && k < L)
             out[s] = adfv_at(k, nr, A1[s], Ac[s], Tm[s], Tc[s], W[s], ar[s], Zc[s], Zm1[s],
@@ -901,28 +928,28 @@ __device__ __forceinline__ void pass2_body(const FusedArgs& a, int n, int j, int
 // Pass 2 of a shallow node (one 64-level slot) for its KT tracers in one wavefront: w,
 // area, areasvol, the stencil depths and hnode_new are loaded once; per tracer the
 // arithmetic is pass2_body's.
-template <int DM, int KT, int ST>
-__device__ __forceinline__ void pass2_shallow_all(const FusedArgs& a, int n, int2 nr, int2 cnt, int j0) {
+template <int DM, int KT, int ST, bool HALF>
+__device__ __forceinline__ void pass2_shallow(const FusedArgs& a, int n, int2 nr, int2 cnt, int j0) {
     constexpr int NS = 1;
     const DevMesh& m = a.m;
     const int L = m.L;
     double Ws[NS], ars[NS], avs[NS], Zcs[NS], zbs[NS];
-    adfv_inputs<NS>(a, n, Ws, ars, avs, Zcs, zbs);
+    adfv_inputs<NS, HALF>(a, n, Ws, ars, avs, Zcs, zbs);
     double hns[NS];
     {
-        const int kl = lane_id();
+        const int kl = col_lane<HALF>();
         hns[0] = in_layer(nr, kl) ? G(a.hnn)[(size_t)n * L + kl] : 0.0;
     }
 #pragma unroll
-    for (int jj = 0; jj < KT; ++jj) {
-        const int j = j0 + jj;   // tracer slot
+    for (int jj = 0; jj < (HALF ? 1 : KT); ++jj) {
+        const int j = j0 + (HALF ? lane_id() >> 5 : jj);   // tracer slot
         const size_t jo = (size_t)j * m.N * L;
         const size_t b0 = (size_t)n * L;
-        const auto Tb = G(a.T[j]);
+        const auto Tb = lane_tracer<HALF>(a.T, j0, jj);
         const auto LOb = G(a.LO + jo);
-        const auto Tr = G(Tb + b0);
-        const auto Or = G(a.Told[j] + b0);
-        const auto LOr = G(LOb + b0);
+        const auto Tr = Tb + b0;
+        const auto Or = lane_tracer<HALF>(a.Told, j0, jj) + b0;
+        const auto LOr = LOb + b0;
         const auto adfh = G(a.adfh + (size_t)j * m.D * L);
         const int kneed = nr.y + 1 < L ? nr.y + 1 : L;
         int4 es[DM];
@@ -934,7 +961,7 @@ __device__ __forceinline__ void pass2_shallow_all(const FusedArgs& a, int n, int
             Tc[s] = 0.0; Ac[s] = 0.0; LOc[s] = 0.0;
             tvx[s] = -INFINITY; tvn[s] = INFINITY; ap[s] = 0.0; am[s] = 0.0;
             if (64 * s >= kneed) continue;
-            const int k = 64 * s + lane_id();
+            const int k = 64 * s + col_lane<HALF>();
             const bool rd = k < kneed;
             const bool wet = in_layer(nr, k);
             // own column and the neighbours' LO, T and the edges' antidiffusive fluxes,
@@ -985,23 +1012,23 @@ __device__ __forceinline__ void pass2_shallow_all(const FusedArgs& a, int n, int
             }
         }
         double tvxm[NS], tvxp[NS], tvnm[NS], tvnp[NS];
-        col_prev<NS>(tvx, tvxm, col_bcast0<NS>(tvx));
+        col_prev<NS, HALF>(tvx, tvxm, col_bcast0<NS>(tvx));
         col_next<NS>(tvx, tvxp, 0.0);
-        col_prev<NS>(tvn, tvnm, col_bcast0<NS>(tvn));
+        col_prev<NS, HALF>(tvn, tvnm, col_bcast0<NS>(tvn));
         col_next<NS>(tvn, tvnp, 0.0);
         double fvc[NS], fvb[NS];
-        adfv_compute<NS>(a, nr, Tc, Ac, Ws, ars, Zcs, zbs, fvc);
+        adfv_compute<NS, HALF>(a, nr, Tc, Ac, Ws, ars, Zcs, zbs, fvc);
         col_next<NS>(fvc, fvb, 0.0);
         // for pass 3, which reads it instead of computing it again
         const auto Fv = G(a.adfv + jo);
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            const int k = 64 * s + lane_id();
+            const int k = 64 * s + col_lane<HALF>();
             if (k <= nr.y && k < L) Fv[b0 + k] = fvc[s];
         }
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            const int k = 64 * s + lane_id();
+            const int k = 64 * s + col_lane<HALF>();
             if (!in_layer(nr, k)) continue;
             const size_t i = b0 + k;
             const bool use_own = (k == nr.x) || (k == nr.y - 1);
@@ -1029,6 +1056,19 @@ __device__ __forceinline__ void pass2_shallow_all(const FusedArgs& a, int n, int
             // (plus, minus) factor pairs, interleaved: pass 3 reads both with one load
             stv(reinterpret_cast<double2*>(a.pf), jo + i, make_double2(fp, fm));
         }
+    }
+}
+
+template <int DM, int KT, int ST>
+__device__ __forceinline__ void pass2_shallow_all(const FusedArgs& a, int n, int2 nr, int2 cnt, int j0) {
+    if (KT == 2 && nr.y < 32) {
+        // (keeps the two bodies' common loads from being merged across the branch, which
+        // took the kernel's arguments through scratch memory: three times the pass's time)
+        asm volatile("" ::: "memory");
+        pass2_shallow<DM, KT, ST, true>(a, n, nr, cnt, j0);
+        asm volatile("" ::: "memory");
+    } else {
+        pass2_shallow<DM, KT, ST, false>(a, n, nr, cnt, j0);
     }
 }
 
@@ -1150,15 +1190,15 @@ __device__ __forceinline__ void pass3_body(const FusedArgs& a, int n, int j, int
 // Pass 3 of a shallow node (one 64-level slot) for its KT tracers in one wavefront:
 // areasvol, hnode_new and hnode are loaded once; per tracer the arithmetic is
 // pass3_body's.
-template <int DM, int KT, int ST>
-__device__ __forceinline__ void pass3_shallow_all(const FusedArgs& a, int n, int2 nr, int2 cnt, int j0) {
+template <int DM, int KT, int ST, bool HALF>
+__device__ __forceinline__ void pass3_shallow(const FusedArgs& a, int n, int2 nr, int2 cnt, int j0) {
     constexpr int NS = 1;
     const DevMesh& m = a.m;
     const int L = m.L;
     int4 es[DM];
 #pragma unroll
     for (int q = 0; q < DM; ++q) es[q] = ldc(a.tab.edge, (size_t)n * ST + q);
-    const int kl = lane_id();
+    const int kl = col_lane<HALF>();
     const bool wetl = in_layer(nr, kl);
     double av_s = 0.0, hn_s = 0.0, hnd_s = 0.0;
     if (wetl) {
@@ -1167,9 +1207,9 @@ __device__ __forceinline__ void pass3_shallow_all(const FusedArgs& a, int n, int
         hnd_s = G(a.hnode)[(size_t)n * L + kl];
     }
 #pragma unroll
-    for (int jj = 0; jj < KT; ++jj) {
-        const int j = j0 + jj;   // tracer slot
-        const auto T = G(a.T[j]);
+    for (int jj = 0; jj < (HALF ? 1 : KT); ++jj) {
+        const int j = j0 + (HALF ? lane_id() >> 5 : jj);   // tracer slot
+        const auto T = lane_tracer<HALF>(a.T, j0, jj);
         const size_t jo = (size_t)j * m.N * L;
         const double2* pm = reinterpret_cast<const double2*>(a.pf) + jo;   // (plus, minus) pairs
         const auto adfh = G(a.adfh + (size_t)j * m.D * L);
@@ -1182,7 +1222,7 @@ __device__ __forceinline__ void pass3_shallow_all(const FusedArgs& a, int n, int
         for (int s = 0; s < NS; ++s) {
             Tc[s] = 0.0; fvc[s] = 0.0; Pc[s] = 1.0; Mc[s] = 1.0; acc[s] = 0.0;
             if (64 * s >= kneed) continue;
-            const int k = 64 * s + lane_id();
+            const int k = 64 * s + col_lane<HALF>();
             const bool wet = in_layer(nr, k);
             // T on every level of the slot (one load for the wet levels and the dry ones
             // below, which are copied)
@@ -1215,12 +1255,12 @@ __device__ __forceinline__ void pass3_shallow_all(const FusedArgs& a, int n, int
             }
         }
         double Pm[NS], Mm[NS];
-        col_prev<NS>(Pc, Pm, col_bcast0<NS>(Pc));
-        col_prev<NS>(Mc, Mm, col_bcast0<NS>(Mc));
+        col_prev<NS, HALF>(Pc, Pm, col_bcast0<NS>(Pc));
+        col_prev<NS, HALF>(Mc, Mm, col_bcast0<NS>(Mc));
         double vl[NS];
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            const int k = 64 * s + lane_id();
+            const int k = 64 * s + col_lane<HALF>();
             vl[s] = 0.0;
             if (in_iface(nr, k) && k < L) {
                 const double f = fvc[s];
@@ -1233,10 +1273,10 @@ __device__ __forceinline__ void pass3_shallow_all(const FusedArgs& a, int n, int
         double vl1[NS];
         col_next<NS>(vl, vl1, 0.0);
         const auto LO = G(a.LO + jo);
-        const auto Tn = G(a.Tnew[j]);
+        const auto Tn = lane_tracer<HALF>(a.Tnew, j0, jj);
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            const int k = 64 * s + lane_id();
+            const int k = 64 * s + col_lane<HALF>();
             if (k >= L) continue;
             const size_t i = b0 + k;
             if (!in_layer(nr, k)) {
@@ -1257,8 +1297,14 @@ __device__ __forceinline__ void pass3_shallow_all(const FusedArgs& a, int n, int
             Tn[i] = Ti + dT;
         }
         // levels past the slots (a shallow column taking the one-slot body): dry copies
-        for (int k = 64 * NS + lane_id(); k < L; k += 64) Tn[b0 + k] = T[b0 + k] + 0.0;
+        for (int k = (HALF ? 32 : 64) + col_lane<HALF>(); k < L; k += HALF ? 32 : 64) Tn[b0 + k] = T[b0 + k] + 0.0;
     }
+}
+
+template <int DM, int KT, int ST>
+__device__ __forceinline__ void pass3_shallow_all(const FusedArgs& a, int n, int2 nr, int2 cnt, int j0) {
+    if (KT == 2 && nr.y < 32) pass3_shallow<DM, KT, ST, true>(a, n, nr, cnt, j0);
+    else pass3_shallow<DM, KT, ST, false>(a, n, nr, cnt, j0);
 }
 
 template <int NS, int DM>

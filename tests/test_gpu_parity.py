@@ -581,3 +581,29 @@ def test_mixed_degree_large_mesh(nl, K, torch_dev):
     for a, b in zip(advect_fct(*args, dt=2700.0, path="fused"),
                     advect_fct(*args, dt=2700.0, path="phased")):
         assert torch.equal(a[0], b[0])
+
+
+@pytest.mark.parametrize("nl,K", [(5, 2), (31, 2), (32, 3), (33, 2), (34, 2), (66, 3)])
+def test_short_columns_share_a_wavefront(nl, K, torch_dev):
+    """Columns of up to 32 interfaces run with two tracers in the halves of a wavefront:
+    depths up to, at and past that line, an odd last tracer, levels past the half that are
+    only copied; bitwise to the oracle, alone and in a batch."""
+    from fesom_jax_amd.batch import FctBatch, Instance
+    from fesom_jax_amd.inputs import make_case
+    from fesom_jax_amd.meshgen import icosahedral_mesh
+    m = icosahedral_mesh(4, nl, seed=101, min_levels=2, land_fraction=0.4)
+    bottom = np.bincount(m.nlevels_nod2D, minlength=nl + 1)
+    assert all(bottom[b] for b in (31, 32, 33) if b <= nl)
+    c = sharp_case(m, make_case(m, seed=102, dt=2700.0), 1.5)
+    dry = ~m.node_layer_mask
+    c["T"] = [np.where(dry, 7.0 + j, c["T"][0] * (1.0 + 0.1 * j)) for j in range(K)]
+    c["T_old"] = [0.98 * t + 0.3 for t in c["T"]]
+    want = [_oracle(m, c, j) for j in range(K)]
+    insts = [Instance.from_case(m, c, torch_dev) for _ in range(2)]
+    insts[0].step_alone()
+    batch = FctBatch(insts[1:])
+    batch.step()
+    for j in range(K):
+        assert np.array_equal(insts[0].T()[j].cpu().numpy(), want[j]), j
+        assert np.array_equal(insts[1].T()[j].cpu().numpy(), want[j]), j
+    batch.close()
