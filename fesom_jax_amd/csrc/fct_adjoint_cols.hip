@@ -26,6 +26,8 @@
 //   kc_tr     (triangle) ka_tr
 //   kc_gather (node)  ka_node_edges and ka_node_final
 //   kc_uv     (triangle) ka_uv, once for all tracers
+//   kc_add    (flat)  small meshes, where a launch takes two tracers (grid.y): the odd
+//                     tracers' w cotangents onto the even ones'
 //
 // Like the forward passes the kernels are bound by the vector memory path (a 64-lane load
 // costs 25 to 36 clocks of a CU, hit or not): kc_limit makes 30 neighbour loads per node,
@@ -75,7 +77,30 @@ struct ColArgs {
     double2* g_tr;                // [E][L]
     double *gw, *gwi;             // every lane; may be null
     const int *ud_off, *ud_ent, *et_off, *et_ent;
+    // a launch over two tracers (gridDim.y = 2): the second one's fields, its w cotangents
+    // (added to the first's at the end), its edge cotangent as kc_uv reads it, and the
+    // distance to its workspace (doubles)
+    const double *T1, *Told1, *g_out1, *g_vf1;
+    double *gT1, *gTold1, *gw1, *gwi1;
+    size_t node_stride, edge_stride, elem_stride;
 };
+
+// the arguments of this workgroup's tracer
+__device__ __forceinline__ ColArgs of_tracer(ColArgs a) {
+    if (blockIdx.y == 0) return a;
+    const size_t NL = (size_t)a.m.N * a.m.L, DL = (size_t)a.m.D * a.m.L;
+    a.T = a.T1; a.Told = a.Told1; a.g_out = a.g_out1;
+    a.gT = a.gT1; a.gTold = a.gTold1; a.gw = a.gw1; a.gwi = a.gwi1;
+    a.LO += NL; a.adfh += DL; a.adfv += NL; a.pm += NL; a.gnode += NL;
+    const size_t d = a.node_stride, d2 = d / 2;
+    a.ghsc += d; a.gA += d; a.gadfv += d; a.gLO += d;
+    a.gpm += d2; a.tv += d2; a.sh += d2; a.gd += d2; a.gnum += d2;
+    a.eg += a.edge_stride / 2;
+    a.g_vf += a.edge_stride;
+    a.edge_up += (size_t)a.m.D * (a.m.L <= 64 ? 1 : 2);
+    a.g_tr += a.elem_stride / 2;
+    return a;
+}
 
 // the wavefront's node: of the node list from `first` where there is one
 __device__ __forceinline__ bool node_task(const ColArgs& a, int first, int count, int& n) {
@@ -867,7 +892,10 @@ __device__ __forceinline__ void uv_body(const ColArgs& a, double2* g_uv, int e) 
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
                 en[i] = ldc(a.et_ent, p + i < p1 ? p + i : p);
-                g[i] = wet && p + i < p1 ? G(a.g_vf)[(size_t)(en[i] >> 1) * L + k] : 0.0;
+                const bool rd = wet && p + i < p1;
+                const size_t x = (size_t)(en[i] >> 1) * L + k;
+                g[i] = rd ? G(a.g_vf)[x] : 0.0;
+                if (a.g_vf1) g[i] = g[i] + (rd ? G(a.g_vf1)[x] : 0.0);
             }
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
@@ -884,42 +912,50 @@ __device__ __forceinline__ void uv_body(const ColArgs& a, double2* g_uv, int e) 
 
 #define KC_OCC(n) __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(n)))
 
-__global__ void KC_OCC(6) kc_ghsc(ColArgs a) {
+__global__ void KC_OCC(6) kc_ghsc(ColArgs a0) {
+    const ColArgs a = of_tracer(a0);
     int w;
     if (single_wave((a.m.N + GH_NODES - 1) / GH_NODES, a.remap, w)) ghsc_body(a, w);
 }
 template <int NS, int DM>
-__global__ void KC_OCC(NS == 1 && DM == 6 ? 4 : 3) kc_limit(ColArgs a, int first, int count) {
+__global__ void KC_OCC(NS == 1 && DM == 6 ? 4 : 3) kc_limit(ColArgs a0, int first, int count) {
+    const ColArgs a = of_tracer(a0);
     int n;
     if (node_task(a, first, count, n)) limit_body<NS, DM>(a, n);
 }
 template <int NS, int DM, bool SPLIT>
-__global__ void KC_OCC(DM == 6 ? 4 : 3) kc_vertex(ColArgs a, int first, int count) {
+__global__ void KC_OCC(DM == 6 ? 4 : 3) kc_vertex(ColArgs a0, int first, int count) {
+    const ColArgs a = of_tracer(a0);
     int n;
     if (node_task(a, first, count, n)) vertex_body<NS, DM, SPLIT>(a, n);
 }
 template <int NS>
-__global__ void KC_OCC(8) kc_split(ColArgs a, int first, int count) {
+__global__ void KC_OCC(8) kc_split(ColArgs a0, int first, int count) {
+    const ColArgs a = of_tracer(a0);
     int n;
     if (node_task(a, first, count, n)) split_body<NS>(a, n);
 }
 template <int NS>
-__global__ void KC_OCC(6) kc_edge(ColArgs a) {
+__global__ void KC_OCC(6) kc_edge(ColArgs a0) {
+    const ColArgs a = of_tracer(a0);
     int e;
     if (single_wave(a.m.D, a.remap, e)) edge_body<NS>(a, e);
 }
 template <int NS, int DM>
-__global__ void KC_OCC(8) kc_gnum(ColArgs a) {
+__global__ void KC_OCC(8) kc_gnum(ColArgs a0) {
+    const ColArgs a = of_tracer(a0);
     int n;
     if (single_wave(a.m.N, a.remap, n)) gnum_body<NS, DM>(a, n);
 }
 template <int NS>
-__global__ void KC_OCC(8) kc_tr(ColArgs a) {
+__global__ void KC_OCC(8) kc_tr(ColArgs a0) {
+    const ColArgs a = of_tracer(a0);
     int w;
     if (single_wave((a.m.E + TR_EL - 1) / TR_EL, a.remap, w)) tr_body<NS>(a, w);
 }
 template <int NS, int DM, int NSL>
-__global__ void KC_OCC(DM == 6 ? 6 : 5) kc_gather(ColArgs a, int first, int count) {
+__global__ void KC_OCC(DM == 6 ? 6 : 5) kc_gather(ColArgs a0, int first, int count) {
+    const ColArgs a = of_tracer(a0);
     int n;
     if (node_task(a, first, count, n)) gather_body<NS, DM, NSL>(a, n);
 }
@@ -929,31 +965,49 @@ __global__ void KC_OCC(8) kc_uv(ColArgs a, double2* g_uv) {
     if (single_wave(a.m.E, a.remap, e)) uv_body<NS>(a, g_uv, e);
 }
 
+// the odd tracers' w cotangents onto the even ones'
+__global__ void __launch_bounds__(256) kc_add(size_t n, double* x, const double* x1, double* y,
+                                              const double* y1) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    if (x) x[i] = x[i] + x1[i];
+    if (y) y[i] = y[i] + y1[i];
+}
+
 constexpr int WPB = 4;
+
+// Meshes of at most this many nodes run two tracers per launch (workspace for both): one
+// tracer's column kernels leave wavefront slots of the chip idle or end in a mostly idle
+// last round, and k_vimpl_reverse has one workgroup per CU or less. Two steps of the pi
+// mesh (3140 nodes) 542 -> 517 us, icosa-6 x 70 with the split (28 700 nodes) 1621 -> 1533;
+// on larger meshes the launches fill the chip and the second workspace (15 node, 3 edge
+// arrays: 1.6 GB at icosa-7 x 47) would buy little.
+constexpr int PAIR_NODES = 32768;
 
 // the node kernels: shallow columns, then (nl > 64) deep ones
 #define KC_NODES(KERN1, KERN2)                                                                \
     do {                                                                                      \
         const int ns = NS == 1 ? a.m.N : a.tab.nshallow, nd = a.m.N - ns;                     \
-        if (ns) KERN1<<<dim3(blocks_for(ns, WPB)), dim3(256), 0, s>>>(a, 0, ns);              \
-        if (nd) KERN2<<<dim3(blocks_for(nd, WPB)), dim3(256), 0, s>>>(a, ns, nd);             \
+        if (ns) KERN1<<<dim3(blocks_for(ns, WPB), y), dim3(256), 0, s>>>(a, 0, ns);              \
+        if (nd) KERN2<<<dim3(blocks_for(nd, WPB), y), dim3(256), 0, s>>>(a, ns, nd);             \
     } while (0)
 
 template <int NS, int DM>
-int reverse_tracer(const ColArgs& a, const double* LOx, hipStream_t s) {
-    kc_ghsc<<<dim3(blocks_for((a.m.N + GH_NODES - 1) / GH_NODES, WPB)), dim3(256), 0, s>>>(a);
+int reverse_tracers(const ColArgs& a, const double* LOx, unsigned y, hipStream_t s) {
+    kc_ghsc<<<dim3(blocks_for((a.m.N + GH_NODES - 1) / GH_NODES, WPB), y), dim3(256), 0, s>>>(a);
     KC_NODES((kc_limit<1, DM>), (kc_limit<NS, DM>));
     if (a.w_i) {
         KC_NODES((kc_vertex<1, DM, true>), (kc_vertex<NS, DM, true>));
-        const int rc = launch_vimpl_reverse(a.m, a.w_i, a.hnn, a.dt, LOx, a.gLO, a.gwi, s);
+        const int rc = launch_vimpl_reverse(a.m, a.w_i, a.hnn, a.dt, LOx, a.gLO, a.gwi,
+                                            y == 2 ? a.gwi1 : nullptr, a.node_stride, s);
         if (rc) return rc;
         KC_NODES((kc_split<1>), (kc_split<NS>));
     } else {
         KC_NODES((kc_vertex<1, DM, false>), (kc_vertex<NS, DM, false>));
     }
-    kc_edge<NS><<<dim3(blocks_for(a.m.D, WPB)), dim3(256), 0, s>>>(a);
-    kc_gnum<NS, DM><<<dim3(blocks_for(a.m.N, WPB)), dim3(256), 0, s>>>(a);
-    kc_tr<NS><<<dim3(blocks_for((a.m.E + TR_EL - 1) / TR_EL, WPB)), dim3(256), 0, s>>>(a);
+    kc_edge<NS><<<dim3(blocks_for(a.m.D, WPB), y), dim3(256), 0, s>>>(a);
+    kc_gnum<NS, DM><<<dim3(blocks_for(a.m.N, WPB), y), dim3(256), 0, s>>>(a);
+    kc_tr<NS><<<dim3(blocks_for((a.m.E + TR_EL - 1) / TR_EL, WPB), y), dim3(256), 0, s>>>(a);
     KC_NODES((kc_gather<1, DM, NS>), (kc_gather<NS, DM, NS>));
     return check_launch("adjoint column kernels");
 }
@@ -966,10 +1020,19 @@ int reverse_uv(const ColArgs& a, double* g_uv, hipStream_t s) {
 
 }  // namespace
 
-// N*L, D*L, E*L doubles of the workspace
-size_t adjoint_cols_node() { return 15; }
-size_t adjoint_cols_edge() { return 3; }
-size_t adjoint_cols_elem() { return 2; }
+// cotangent workspace of one tracer, in doubles (even: double2 arrays lie at its start)
+static size_t even(size_t n) { return (n + 1) / 2 * 2; }
+static size_t node_stride(const DevMesh& m) { return even((size_t)m.N * m.L * 15); }
+static size_t edge_stride(const DevMesh& m) { return even((size_t)m.D * m.L * 3); }
+static size_t elem_stride(const DevMesh& m) { return (size_t)m.E * m.L * 2; }
+
+int adjoint_cols_tracers(const DevMesh& m) { return m.N <= PAIR_NODES ? 2 : 1; }
+// (two tracers: and the second one's w cotangent)
+size_t adjoint_cols_node(const DevMesh& m, int nt) {
+    return nt * node_stride(m) + (nt > 1 ? (size_t)m.N * m.L : 0);
+}
+size_t adjoint_cols_edge(const DevMesh& m, int nt) { return nt * edge_stride(m); }
+size_t adjoint_cols_elem(const DevMesh& m, int nt) { return nt * elem_stride(m); }
 
 int launch_backward_cols(const DevMesh& m, const NodeTab& tab, const int2* ekr, const FusedTape& tp,
                          const AdjointCols& w, const FusedTuning& tune, const fct_step_args* f,
@@ -988,27 +1051,50 @@ int launch_backward_cols(const DevMesh& m, const NodeTab& tab, const int2* ekr, 
     for (double** q : {&a.ghsc, &a.gA, &a.gadfv, &a.gLO}) *q = take(1);
     double* own_wi = take(1);
     a.eg = reinterpret_cast<double2*>(w.edge);
-    a.g_vf = w.edge + 2 * DL;
     a.edge_up = w.edge_up;
     a.g_tr = reinterpret_cast<double2*>(w.elem);
-    a.gw = g_w;
-    a.gwi = f->w_i ? (g_wi ? g_wi : own_wi) : nullptr;
+    a.node_stride = node_stride(m); a.edge_stride = edge_stride(m); a.elem_stride = elem_stride(m);
+    // Small meshes sum the even and the odd tracers' uv and w cotangents apart, whether a
+    // launch takes two tracers or one (a plan with one slot): the bits do not depend on it.
+    const bool pairs = w.tracers == 2 && f->ntracers >= 2;
+    double* vf[2] = {w.edge + 2 * DL, w.edge + 2 * DL + a.edge_stride};
+    double* gw[2] = {g_w, g_w ? w.node + 2 * a.node_stride : nullptr};
+    double* gwi[2] = {nullptr, nullptr};
+    if (f->w_i) { gwi[0] = g_wi ? g_wi : own_wi; gwi[1] = own_wi + a.node_stride; }
     a.ud_off = w.ud_off; a.ud_ent = w.ud_ent; a.et_off = w.et_off; a.et_ent = w.et_ent;
     int rc;
     for (int j0 = 0; j0 < f->ntracers; j0 += tp.kw) {
         const int K = f->ntracers - j0 < tp.kw ? f->ntracers - j0 : tp.kw;
         if ((rc = launch_tape(m, tab, ekr, f, j0, K, tune, tp, s))) return rc;
-        for (int j = 0; j < K; ++j) {
-            a.first = j0 + j == 0;
-            a.T = f->T[j0 + j]; a.Told = f->T_old[j0 + j]; a.g_out = g_out[j0 + j];
-            a.gT = gT[j0 + j]; a.gTold = gTold[j0 + j];
+        for (int j = 0, n = 1; j < K; j += n) {
+            const int t = j0 + j, odd = pairs ? t & 1 : 0;
+            n = pairs && !odd && K - j >= 2 ? 2 : 1;
+            const int t1 = t + n - 1;
+            a.first = pairs ? t < 2 : t == 0;
+            a.g_vf = vf[odd]; a.gw = gw[odd]; a.gwi = gwi[odd];
+            a.gw1 = gw[1]; a.gwi1 = gwi[1];
+            a.T = f->T[t]; a.Told = f->T_old[t]; a.g_out = g_out[t];
+            a.gT = gT[t]; a.gTold = gTold[t];
+            a.T1 = f->T[t1]; a.Told1 = f->T_old[t1]; a.g_out1 = g_out[t1];
+            a.gT1 = gT[t1]; a.gTold1 = gTold[t1];
             a.LO = tp.LO + j * NL; a.adfh = tp.adfh + j * DL; a.adfv = tp.adfv + j * NL;
             a.pm = reinterpret_cast<const double2*>(tp.pf) + j * NL;
             a.gnode = reinterpret_cast<const double2*>(tp.gnode) + j * NL;
             const double* LOx = tp.LOx ? tp.LOx + j * NL : nullptr;
-            if (m.L <= 64) rc = tab.dm == 6 ? reverse_tracer<1, 6>(a, LOx, s) : reverse_tracer<1, 8>(a, LOx, s);
-            else rc = tab.dm == 6 ? reverse_tracer<2, 6>(a, LOx, s) : reverse_tracer<2, 8>(a, LOx, s);
+            if (m.L <= 64)
+                rc = tab.dm == 6 ? reverse_tracers<1, 6>(a, LOx, n, s) : reverse_tracers<1, 8>(a, LOx, n, s);
+            else
+                rc = tab.dm == 6 ? reverse_tracers<2, 6>(a, LOx, n, s) : reverse_tracers<2, 8>(a, LOx, n, s);
             if (rc) return rc;
+        }
+    }
+    a.g_vf = vf[0];
+    if (pairs) {
+        a.g_vf1 = vf[1];
+        double* wi = f->w_i ? g_wi : nullptr;
+        if (g_w || wi) {
+            kc_add<<<dim3((unsigned)((NL + 255) / 256)), dim3(256), 0, s>>>(NL, g_w, gw[1], wi, gwi[1]);
+            if ((rc = check_launch("kc_add"))) return rc;
         }
     }
     if (!g_uv) return FCT_OK;

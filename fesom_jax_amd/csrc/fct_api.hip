@@ -398,18 +398,19 @@ int ensure_adjoint(fct_plan* p) {
     if (p->adj_ready) return FCT_OK;
     int rc;
     const DevMesh& m = p->m;
-    const size_t NL = (size_t)m.N * m.L, DL = (size_t)m.D * m.L, EL = (size_t)m.E * m.L;
     if (adjoint_by_columns(p)) {
         AdjointCols& c = p->ac;
-        if ((rc = dev_alloc(p, &c.node, NL * adjoint_cols_node())) ||
-            (rc = dev_alloc(p, &c.edge_up, (size_t)m.D * (m.L <= 64 ? 1 : 2))) ||
-            (rc = dev_alloc(p, &c.edge, DL * adjoint_cols_edge())) ||
-            (rc = dev_alloc(p, &c.elem, EL * adjoint_cols_elem())) ||
+        const int nt = c.tracers = adjoint_cols_tracers(m);
+        if ((rc = dev_alloc(p, &c.node, adjoint_cols_node(m, nt))) ||
+            (rc = dev_alloc(p, &c.edge_up, (size_t)m.D * (m.L <= 64 ? 1 : 2) * nt)) ||
+            (rc = dev_alloc(p, &c.edge, adjoint_cols_edge(m, nt))) ||
+            (rc = dev_alloc(p, &c.elem, adjoint_cols_elem(m, nt))) ||
             (rc = upload_element_lists(p, &c.ud_off, &c.ud_ent, &c.et_off, &c.et_ent)))
             return rc;
         p->adj_ready = true;
         return FCT_OK;
     }
+    const size_t NL = (size_t)m.N * m.L, DL = (size_t)m.D * m.L, EL = (size_t)m.E * m.L;
     if ((rc = ensure_phased(p))) return rc;
     AdjointWork& w = p->aw;
     w.vflux = p->vflux; w.LO = p->LO; w.trxy = p->trxy; w.gnode = p->gnode; w.adfh = p->adfh;

@@ -119,7 +119,8 @@ int vimpl_call(const DevMesh& m, const double* w_i, const double* hnn, double dt
 // added to gwi; X and gX hold values on wet layers only. The recurrences of the forward
 // solve and of its reverse run one column per lane out of LDS, eight arrays per column;
 // everything else one thread per value (VR_U values per thread at most: a workgroup's LDS
-// holds 2.4 per thread). One thread per column from memory took 883 us per tracer at
+// holds 2.4 per thread). With gwi1 the launch takes two tracers (grid.y): the second one's X
+// at N * L, gX at gX_stride, its w_i cotangent added to gwi1. One thread per column from memory took 883 us per tracer at
 // icosa-6 x 70.
 constexpr int VR_U = 3, VR_ARRAYS = 8;
 static_assert(VI_LDS <= (size_t)VR_U * 256 * VR_ARRAYS * sizeof(double), "values per thread");
@@ -127,8 +128,11 @@ static_assert(VI_LDS <= (size_t)VR_U * 256 * VR_ARRAYS * sizeof(double), "values
 __global__ void __launch_bounds__(256)
 k_vimpl_reverse(DevMesh m, int C, const double* __restrict__ w_i, const double* __restrict__ hnn,
                 double dt, const double* __restrict__ X, double* __restrict__ gX,
-                double* __restrict__ gwi) {
+                double* __restrict__ gwi, double* __restrict__ gwi1, size_t gX_stride) {
     extern __shared__ double sh[];
+    if (blockIdx.y) {      // the second tracer of the launch
+        X += (size_t)m.N * m.L; gX += gX_stride; gwi = gwi1;
+    }
     const int L = m.L, P = (L + 1) | 1, S = C * P;
     const int n0 = blockIdx.x * C;
     const int nc = min(C, m.N - n0), count = nc * L;
@@ -268,10 +272,12 @@ int launch_vimpl_wet(const DevMesh& m, const double* w_i, const double* hnn, dou
 }
 
 int launch_vimpl_reverse(const DevMesh& m, const double* w_i, const double* hnn, double dt,
-                         const double* X, double* gX, double* gwi, hipStream_t s) {
+                         const double* X, double* gX, double* gwi, double* gwi1, size_t gX_stride,
+                         hipStream_t s) {
     const int C = vi_columns(m.L, VR_ARRAYS);
     const size_t lds = ((size_t)VR_ARRAYS * C * vi_pitch(m.L) + VI_SLACK) * sizeof(double);
-    k_vimpl_reverse<<<dim3((m.N + C - 1) / C), dim3(256), lds, s>>>(m, C, w_i, hnn, dt, X, gX, gwi);
+    k_vimpl_reverse<<<dim3((m.N + C - 1) / C, gwi1 ? 2 : 1), dim3(256), lds, s>>>(
+        m, C, w_i, hnn, dt, X, gX, gwi, gwi1, gX_stride);
     return check_launch("k_vimpl_reverse");
 }
 

@@ -185,14 +185,15 @@ int launch_vert_impl(const DevMesh& m, const double* w_i, const double* hnn, dou
 
 // The same through LDS (fct_column.hip), for the nl that fit (vimpl_fits), and its form
 // for K tracer slots [K][N][L] of which only wet layers hold values (out may be X), and
-// the reverse mode of the latter for one tracer (nl <= 128).
+// the reverse mode of the latter for one tracer, or two with gwi1 (nl <= 128).
 bool vimpl_fits(int L);
 int launch_vimpl(const DevMesh& m, const double* w_i, const double* hnn, double dt,
                  const double* X, double* out, hipStream_t s);
 int launch_vimpl_wet(const DevMesh& m, const double* w_i, const double* hnn, double dt,
                      const double* X, double* out, int K, hipStream_t s);
 int launch_vimpl_reverse(const DevMesh& m, const double* w_i, const double* hnn, double dt,
-                         const double* X, double* gX, double* gwi, hipStream_t s);
+                         const double* X, double* gX, double* gwi, double* gwi1, size_t gX_stride,
+                         hipStream_t s);
 int launch_pm(const DevMesh& m, const fct_step_args* a, int j, const double* vflux,
               const double* LO, const double* tr, double* gnode, double* adfh, double* adfv,
               double* tvmax, double* tvmin, double* fplus, double* fminus, hipStream_t s);
@@ -246,17 +247,20 @@ struct FusedTape {
     double *vflux = nullptr, *LO = nullptr, *LOx = nullptr, *gnode = nullptr, *adfh = nullptr;
     double *pf = nullptr, *adfv = nullptr;
 };
-// Workspace of the column adjoint (fct_adjoint_cols.hip): one tracer's cotangents, in
-// adjoint_cols_node() * N*L, ..._edge() * D*L and ..._elem() * E*L doubles, the sign
-// bits of the edges' flux (one word per 64 levels) and the element-side lists.
+// Workspace of the column adjoint (fct_adjoint_cols.hip): the cotangents of one or two
+// tracers (adjoint_cols_tracers), in adjoint_cols_node(), ..._edge() and ..._elem()
+// doubles, the sign bits of the edges' flux (per tracer one word per 64 levels) and the
+// element-side lists.
 struct AdjointCols {
+    int tracers = 1;
     double *node = nullptr, *edge = nullptr, *elem = nullptr;
     uint64_t* edge_up = nullptr;
     const int *ud_off = nullptr, *ud_ent = nullptr, *et_off = nullptr, *et_ent = nullptr;
 };
-size_t adjoint_cols_node();
-size_t adjoint_cols_edge();
-size_t adjoint_cols_elem();
+int adjoint_cols_tracers(const DevMesh& m);
+size_t adjoint_cols_node(const DevMesh& m, int tracers);
+size_t adjoint_cols_edge(const DevMesh& m, int tracers);
+size_t adjoint_cols_elem(const DevMesh& m, int tracers);
 
 // Launch-shape knobs of the fused path (fct_plan_set_tuning / fct_batch_set_tuning);
 // results do not depend on them.

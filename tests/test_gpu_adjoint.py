@@ -261,3 +261,40 @@ def test_flat_adjoint_of_long_columns(torch_dev):
     for opts in ({}, dict(w_i=w_i, Z3d=Z3d, zbar3=zb3)):
         _compare("icosa2 nl130", _gpu(m, c, Ts, Tos, gs, torch_dev, **opts),
                  _oracle(m, c, Ts, Tos, gs, **opts))
+
+
+@pytest.mark.parametrize("level,nl,degree8,K,split", [
+    (2, 13, 0, 2, True), (3, 65, 10, 3, True), (3, 47, 0, 4, False), (3, 31, 0, 5, False)])
+def test_adjoint_two_tracers_per_launch(level, nl, degree8, K, split, torch_dev):
+    """Small meshes reverse two tracers per launch: against a plan with one tracer slot,
+    which reverses them one after the other, bit for bit. Odd N * L (workspace alignment),
+    a last tracer alone, more tracers than slots, pairs cut by an odd number of slots."""
+    import torch
+    from fesom_jax_amd.adjoint import advect_fct_vjp
+    from fesom_jax_amd.inputs import make_case
+    from fesom_jax_amd.meshgen import icosahedral_mesh
+    from fesom_jax_amd.tracer_adv import FctPlan
+    m = icosahedral_mesh(level, nl, seed=111, degree8=degree8)
+    c = sharp_case(m, make_case(m, seed=112, dt=2700.0), 1.5)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(torch_dev)
+    Ts = [t(c["T"][0] * (1.0 + 0.1 * j)) for j in range(K)]
+    Tos = [t(c["T_old"][0] + 0.2 * j) for j in range(K)]
+    gs = [t(g) for g in _cot(m, K, 113)]
+    opts = {}
+    if split:
+        w_i, Z3d, zb3 = _split(m, c, 114)
+        opts = dict(w_i=t(w_i), Z3d=t(Z3d), zbar3=t(zb3))
+    flow = [t(c[k]) for k in ("uv", "w_e", "helem", "hnode", "hnode_new")]
+
+    def run(js, slots):
+        plan = FctPlan(m, torch_dev, max_tracers=slots)
+        return advect_fct_vjp(m, *flow, [Ts[j] for j in js], [Tos[j] for j in js],
+                              [gs[j] for j in js], dt=c["dt"], plan=plan, **opts)
+
+    one = run(range(K), 1)
+    for slots in (2, 3, 4):
+        two = run(range(K), slots)
+        for j in range(K):
+            assert torch.equal(two[0][j], one[0][j]) and torch.equal(two[1][j], one[1][j]), j
+        for i in range(2, len(one)):
+            assert torch.equal(two[i], one[i]), i
