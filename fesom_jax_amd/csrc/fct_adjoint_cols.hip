@@ -35,6 +35,8 @@
 // path's bits (recomputed in the same order), so the branches of the chain rule are too;
 // sums run in table order and agree with the flat form to rounding.
 
+#include <type_traits>
+
 #include "fct_wave.h"
 
 namespace fct {
@@ -102,6 +104,27 @@ __device__ __forceinline__ ColArgs of_tracer(ColArgs a) {
     return a;
 }
 
+// the arguments of this lane's tracer, where a short column's two tracers share a wavefront
+// (lane = 32 * tracer + level)
+__device__ __forceinline__ ColArgs of_half(ColArgs a) {
+    const size_t h = lane_id() >> 5;
+    const auto to = [&](auto& p, auto q) {
+        p = (std::decay_t<decltype(p)>)((uint64_t)p + h * ((uint64_t)q - (uint64_t)p));
+    };
+    to(a.T, a.T1); to(a.Told, a.Told1); to(a.g_out, a.g_out1);
+    to(a.gT, a.gT1); to(a.gTold, a.gTold1); to(a.gw, a.gw1); to(a.gwi, a.gwi1);
+    const size_t NL = h * a.m.N * a.m.L, DL = h * a.m.D * a.m.L;
+    a.LO += NL; a.adfh += DL; a.adfv += NL; a.pm += NL; a.gnode += NL;
+    const size_t d = h * a.node_stride, d2 = d / 2;
+    a.ghsc += d; a.gA += d; a.gadfv += d; a.gLO += d;
+    a.gpm += d2; a.tv += d2; a.sh += d2; a.gd += d2; a.gnum += d2;
+    a.eg += h * a.edge_stride / 2;
+    a.g_vf += h * a.edge_stride;
+    a.edge_up += h * a.m.D * (a.m.L <= 64 ? 1 : 2);
+    a.g_tr += h * a.elem_stride / 2;
+    return a;
+}
+
 // the wavefront's node: of the node list from `first` where there is one
 __device__ __forceinline__ bool node_task(const ColArgs& a, int first, int count, int& n) {
     int w;
@@ -138,7 +161,7 @@ __device__ __forceinline__ void ghsc_body(const ColArgs& a, int w) {
 }
 
 // ---- R2: everything of the limiter that a node owns ------------------------------
-template <int NS, int DM>
+template <int NS, int DM, bool HALF>
 __device__ __forceinline__ void limit_body(const ColArgs& a, int n) {
     const DevMesh& m = a.m;
     const int L = m.L;
@@ -163,7 +186,7 @@ __device__ __forceinline__ void limit_body(const ColArgs& a, int n) {
         tvx[s] = -INFINITY; tvn[s] = INFINITY;
         P[s] = M[s] = cx[s] = cn[s] = 1.0;
         if (64 * s >= kneed) continue;
-        const int k = 64 * s + lane_id();
+        const int k = 64 * s + col_lane<HALF>();
         const bool wet = in_layer(nr, k);
         const size_t i = b0 + k;
         if (k < kneed) {
@@ -241,12 +264,12 @@ __device__ __forceinline__ void limit_body(const ColArgs& a, int n) {
     // limited vertical fluxes (:453-459): interface k's cotangent goes to the factors of
     // levels k and k-1
     double gxm[NS], Pm[NS], Mm[NS], gva[NS], gp[NS], gm[NS], gpp[NS], gmp[NS], nx[NS];
-    col_prev<NS>(gx, gxm, 0.0);
-    col_prev<NS>(P, Pm, 1.0);
-    col_prev<NS>(M, Mm, 1.0);
+    col_prev<NS, HALF>(gx, gxm, 0.0);
+    col_prev<NS, HALF>(P, Pm, 1.0);
+    col_prev<NS, HALF>(M, Mm, 1.0);
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        const int k = 64 * s + lane_id();
+        const int k = 64 * s + col_lane<HALF>();
         const double gvl = in_iface(nr, k) ? gx[s] - gxm[s] : 0.0;
         const bool pv = fv[s] >= 0.0;
         const double g = gvl * fv[s];
@@ -274,15 +297,15 @@ __device__ __forceinline__ void limit_body(const ColArgs& a, int n) {
     for (int s = 0; s < NS; ++s) gm[s] += nx[s] + hm[s];
     // limiter factors (:441-451)
     double tvxm[NS], tvxp[NS], tvnm[NS], tvnp[NS], fvb[NS];
-    col_prev<NS>(tvx, tvxm, col_bcast0<NS>(tvx));
+    col_prev_own<NS, HALF>(tvx, tvxm);
     col_next<NS>(tvx, tvxp, 0.0);
-    col_prev<NS>(tvn, tvnm, col_bcast0<NS>(tvn));
+    col_prev_own<NS, HALF>(tvn, tvnm);
     col_next<NS>(tvn, tvnp, 0.0);
     col_next<NS>(fv, fvb, 0.0);
     double gfp[NS], gfn[NS], mx[NS], mn[NS], W[NS], ar[NS], Zc[NS], zb[NS], A1[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        const int k = 64 * s + lane_id();
+        const int k = 64 * s + col_lane<HALF>();
         const int kc = k < L ? k : L - 1;
         const size_t i = b0 + kc;
         const bool wet = in_layer(nr, k);
@@ -325,11 +348,11 @@ __device__ __forceinline__ void limit_body(const ColArgs& a, int n) {
     }
     // cotangent of adf_v: limited flux, P+/P- of this level and of the one above
     double gfpm[NS], gfnm[NS], gav[NS];
-    col_prev<NS>(gfp, gfpm, 0.0);
-    col_prev<NS>(gfn, gfnm, 0.0);
+    col_prev<NS, HALF>(gfp, gfpm, 0.0);
+    col_prev<NS, HALF>(gfn, gfnm, 0.0);
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        const int k = 64 * s + lane_id();
+        const int k = 64 * s + col_lane<HALF>();
         gav[s] = gva[s] + (gmax_x(gfp[s], fv[s], 0.0) + gmin_x(gfn[s], fv[s], 0.0));
         if (k > 0) gav[s] += -gmax_x(gfpm[s], -fv[s], 0.0) - gmin_x(gfnm[s], -fv[s], 0.0);
     }
@@ -340,7 +363,7 @@ __device__ __forceinline__ void limit_body(const ColArgs& a, int n) {
         double ga[NS], gb[NS], gc[NS], o1[NS], o2[NS];
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-            const int k = 64 * s + lane_id();
+            const int k = 64 * s + col_lane<HALF>();
             const double g = w ? mn[s] : mx[s];
             const double x = w ? tvnm[s] : tvxm[s], y = w ? tvn[s] : tvx[s], z = w ? tvnp[s] : tvxp[s];
             ga[s] = gc[s] = 0.0;
@@ -355,7 +378,7 @@ __device__ __forceinline__ void limit_body(const ColArgs& a, int n) {
             }
         }
         col_next<NS>(ga, o1, 0.0);
-        col_prev<NS>(gc, o2, 0.0);
+        col_prev<NS, HALF>(gc, o2, 0.0);
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             const double v = (gb[s] + o1[s]) + o2[s], c = w ? cn[s] : cx[s];
@@ -364,22 +387,22 @@ __device__ __forceinline__ void limit_body(const ColArgs& a, int n) {
         }
     }
     // QR4C (:241-295): interface j's cotangent goes to A[j], A[j-1], A[j-2], A[j+1], w[j]
-    col_prev<NS>(Ac, A1, col_bcast0<NS>(Ac));
+    col_prev_own<NS, HALF>(Ac, A1);
     double Zm1[NS], dz[NS], qc[NS], qu[NS], qd[NS], dzu[NS], dzd[NS];
-    col_prev<NS>(Zc, Zm1, col_bcast0<NS>(Zc));
+    col_prev_own<NS, HALF>(Zc, Zm1);
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         dz[s] = nz_safe(Zm1[s] - Zc[s]);
         qc[s] = 64 * s <= nr.y ? (A1[s] - Ac[s]) / dz[s] : 0.0;
     }
     col_next<NS>(qc, qu, 0.0);
-    col_prev<NS>(qc, qd, 0.0);
+    col_prev<NS, HALF>(qc, qd, 0.0);
     col_next<NS>(dz, dzu, 1.0);
-    col_prev<NS>(dz, dzd, 1.0);
+    col_prev<NS, HALF>(dz, dzd, 1.0);
     double t0[NS], tm1[NS], tm2[NS], tp1[NS], tw[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        const int k = 64 * s + lane_id();
+        const int k = 64 * s + col_lane<HALF>();
         t0[s] = tm1[s] = tm2[s] = tp1[s] = tw[s] = 0.0;
         if (!in_layer(nr, k)) continue;      // interface nzmax has no high-order flux
         const double g = gav[s] * ar[s];
@@ -407,10 +430,10 @@ __device__ __forceinline__ void limit_body(const ColArgs& a, int n) {
     col_next<NS>(tm2, x1, 0.0);
     col_next<NS>(tm1, x2, 0.0);
     col_next<NS>(x1, x3, 0.0);
-    col_prev<NS>(tp1, x4, 0.0);
+    col_prev<NS, HALF>(tp1, x4, 0.0);
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        const int k = 64 * s + lane_id();
+        const int k = 64 * s + col_lane<HALF>();
         if (k >= L) continue;
         const size_t i = b0 + k;
         if (in_layer(nr, k)) {
@@ -422,7 +445,7 @@ __device__ __forceinline__ void limit_body(const ColArgs& a, int n) {
         if (a.gwi) G(a.gwi)[i] = a.first ? tw[s] : G(a.gwi)[i] + tw[s];
     }
     if (a.first)      // levels past the slots (a shallow column in the one-slot body)
-        for (int k = 64 * NS + lane_id(); k < L; k += 64) {
+        for (int k = (HALF ? 32 : 64 * NS) + col_lane<HALF>(); k < L; k += HALF ? 32 : 64) {
             if (a.gw) G(a.gw)[b0 + k] = 0.0;
             if (a.gwi) G(a.gwi)[b0 + k] = 0.0;
         }
@@ -440,7 +463,7 @@ __device__ __forceinline__ double upwind_v(double g, double W, int k, double& up
 
 // ---- LO (:298-313) and its vertical flux, from the column's gLO -------------------
 // gT receives what the column's T takes from LO, the vertical fluxes and the bounds (gt)
-template <int NS, bool SPLIT>
+template <int NS, bool SPLIT, bool HALF>
 __device__ __forceinline__ void lo_column(const ColArgs& a, int n, int2 nr, const double (&gLO)[NS],
                                           const double (&gt)[NS], const double (&Tc)[NS]) {
     const DevMesh& m = a.m;
@@ -449,7 +472,7 @@ __device__ __forceinline__ void lo_column(const ColArgs& a, int n, int2 nr, cons
     double gdv[NS], gdm[NS], acc[NS], av[NS], We[NS], Wf[NS], ar[NS], gq[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        const int k = 64 * s + lane_id();
+        const int k = 64 * s + col_lane<HALF>();
         gdv[s] = acc[s] = We[s] = Wf[s] = ar[s] = gq[s] = 0.0;
         if (!in_layer(nr, k)) continue;
         const size_t i = b0 + k;
@@ -467,12 +490,12 @@ __device__ __forceinline__ void lo_column(const ColArgs& a, int n, int2 nr, cons
         if (!(hn > 0.0)) acc[s] += G(a.g_out)[i];
         stv(a.gd, i, make_double2(G(a.ghsc)[i], gdv[s]));
     }
-    col_prev<NS>(gdv, gdm, 0.0);
+    col_prev<NS, HALF>(gdv, gdm, 0.0);
     double up[NS], upn[NS], Tm[NS];
-    col_prev<NS>(Tc, Tm, col_bcast0<NS>(Tc));
+    col_prev_own<NS, HALF>(Tc, Tm);
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        const int k = 64 * s + lane_id();
+        const int k = 64 * s + col_lane<HALF>();
         up[s] = 0.0;
         if (!in_layer(nr, k)) continue;
         const double gl0 = gdv[s] - (k > 0 ? gdm[s] : 0.0);
@@ -496,7 +519,7 @@ __device__ __forceinline__ void lo_column(const ColArgs& a, int n, int2 nr, cons
     col_next<NS>(up, upn, 0.0);
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        const int k = 64 * s + lane_id();
+        const int k = 64 * s + col_lane<HALF>();
         if (in_layer(nr, k)) G(a.gT)[b0 + k] = acc[s] + upn[s];
         // the surface interface's flux reads the dry level above it
         if (k + 1 == nr.x) G(a.gT)[b0 + k] = G(a.g_out)[b0 + k] + upn[s];
@@ -504,7 +527,7 @@ __device__ __forceinline__ void lo_column(const ColArgs& a, int n, int2 nr, cons
 }
 
 // ---- R3: vertex cotangents of the bounds; without the split also LO ---------------
-template <int NS, int DM, bool SPLIT>
+template <int NS, int DM, bool SPLIT, bool HALF>
 __device__ __forceinline__ void vertex_body(const ColArgs& a, int n) {
     const DevMesh& m = a.m;
     const int L = m.L;
@@ -522,7 +545,7 @@ __device__ __forceinline__ void vertex_body(const ColArgs& a, int n) {
     for (int s = 0; s < NS; ++s) {
         gLO[s] = gt[s] = Tc[s] = 0.0;
         if (64 * s >= nr.y) continue;
-        const int k = 64 * s + lane_id();
+        const int k = 64 * s + col_lane<HALF>();
         const size_t i = b0 + k;
         if (k < nr.y) Tc[s] = G(a.T)[i];      // the level above the surface too
         if (!in_layer(nr, k)) continue;
@@ -567,7 +590,7 @@ __device__ __forceinline__ void vertex_body(const ColArgs& a, int n) {
             G(a.gT)[i] = gt[s];
         }
     }
-    if (!SPLIT) lo_column<NS, false>(a, n, nr, gLO, gt, Tc);
+    if (!SPLIT) lo_column<NS, false, HALF>(a, n, nr, gLO, gt, Tc);
 }
 
 // ---- R3 under the split, after the column solve's transpose -----------------------
@@ -586,11 +609,11 @@ __device__ __forceinline__ void split_body(const ColArgs& a, int n) {
         gt[s] = wet ? G(a.gT)[b0 + k] : 0.0;
         Tc[s] = k < nr.y ? G(a.T)[b0 + k] : 0.0;
     }
-    lo_column<NS, true>(a, n, nr, gLO, gt, Tc);
+    lo_column<NS, true, false>(a, n, nr, gLO, gt, Tc);
 }
 
 // ---- R4: edges (:196-225, :344-368, :426-435, :460-466, :96-105) -------------------
-template <int NS>
+template <int NS, bool HALF>
 __device__ __forceinline__ void edge_body(const ColArgs& a, int e) {
     const DevMesh& m = a.m;
     const int L = m.L;
@@ -602,7 +625,7 @@ __device__ __forceinline__ void edge_body(const ColArgs& a, int e) {
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         if (64 * s >= kr.y) break;
-        const int k = 64 * s + lane_id();
+        const int k = 64 * s + col_lane<HALF>();
         if (k < kr.x || k >= kr.y) continue;
         const int lo = kr.x > 64 * s ? kr.x : 64 * s, hi = kr.y < 64 * s + 64 ? kr.y : 64 * s + 64;
         const int tl = lo > ur.x ? lo : ur.x, th = hi < ur.y ? hi : ur.y;
@@ -663,7 +686,8 @@ __device__ __forceinline__ void edge_body(const ColArgs& a, int e) {
         gv = gv + (gp + gm + gabs(gp - gm, vf));
         stv(a.eg, t, make_double2(gs2 * v2, gs1 * v2));
         G(a.g_vf)[t] = gv0 + gv;
-        const uint64_t up = __ballot(vf >= 0.0);       // lanes of wet levels
+        uint64_t up = __ballot(vf >= 0.0);             // lanes of wet levels
+        if (HALF) up &= 0xffffffffu;                   // the same in both halves
         if (k == lo) ((gptr<uint64_t>)a.edge_up)[(size_t)e * NS + s] = up;
     }
 }
@@ -917,17 +941,33 @@ __global__ void KC_OCC(6) kc_ghsc(ColArgs a0) {
     int w;
     if (single_wave((a.m.N + GH_NODES - 1) / GH_NODES, a.remap, w)) ghsc_body(a, w);
 }
-template <int NS, int DM>
+template <int NS, int DM, bool HALVES>
 __global__ void KC_OCC(NS == 1 && DM == 6 ? 4 : 3) kc_limit(ColArgs a0, int first, int count) {
     const ColArgs a = of_tracer(a0);
     int n;
-    if (node_task(a, first, count, n)) limit_body<NS, DM>(a, n);
+    if (!node_task(a, first, count, n)) return;
+    if constexpr (HALVES)
+        if (ldc(a0.tab.hdr, n).y < 31) {
+            if (blockIdx.y) return;
+            asm volatile("" ::: "memory");      // no merging of the two bodies' loads
+            limit_body<1, DM, true>(of_half(a0), n);
+            return;
+        }
+    limit_body<NS, DM, false>(a, n);
 }
-template <int NS, int DM, bool SPLIT>
+template <int NS, int DM, bool SPLIT, bool HALVES>
 __global__ void KC_OCC(DM == 6 ? 4 : 3) kc_vertex(ColArgs a0, int first, int count) {
     const ColArgs a = of_tracer(a0);
     int n;
-    if (node_task(a, first, count, n)) vertex_body<NS, DM, SPLIT>(a, n);
+    if (!node_task(a, first, count, n)) return;
+    if constexpr (HALVES)
+        if (ldc(a0.tab.hdr, n).y < 31) {
+            if (blockIdx.y) return;
+            asm volatile("" ::: "memory");      // no merging of the two bodies' loads
+            vertex_body<1, DM, SPLIT, true>(of_half(a0), n);
+            return;
+        }
+    vertex_body<NS, DM, SPLIT, false>(a, n);
 }
 template <int NS>
 __global__ void KC_OCC(8) kc_split(ColArgs a0, int first, int count) {
@@ -935,11 +975,19 @@ __global__ void KC_OCC(8) kc_split(ColArgs a0, int first, int count) {
     int n;
     if (node_task(a, first, count, n)) split_body<NS>(a, n);
 }
-template <int NS>
+template <int NS, bool HALVES>
 __global__ void KC_OCC(6) kc_edge(ColArgs a0) {
     const ColArgs a = of_tracer(a0);
     int e;
-    if (single_wave(a.m.D, a.remap, e)) edge_body<NS>(a, e);
+    if (!single_wave(a.m.D, a.remap, e)) return;
+    if constexpr (HALVES)
+        if (ldc(a0.ekr, e).y < 32) {
+            if (blockIdx.y) return;
+            asm volatile("" ::: "memory");
+            edge_body<NS, true>(of_half(a0), e);
+            return;
+        }
+    edge_body<NS, false>(a, e);
 }
 template <int NS, int DM>
 __global__ void KC_OCC(8) kc_gnum(ColArgs a0) {
@@ -977,12 +1025,21 @@ __global__ void __launch_bounds__(256) kc_add(size_t n, double* x, const double*
 constexpr int WPB = 4;
 
 // Meshes of at most this many nodes run two tracers per launch (workspace for both): one
-// tracer's column kernels leave wavefront slots of the chip idle or end in a mostly idle
-// last round, and k_vimpl_reverse has one workgroup per CU or less. Two steps of the pi
-// mesh (3140 nodes) 542 -> 517 us, icosa-6 x 70 with the split (28 700 nodes) 1621 -> 1533;
-// on larger meshes the launches fill the chip and the second workspace (15 node, 3 edge
-// arrays: 1.6 GB at icosa-7 x 47) would buy little.
-constexpr int PAIR_NODES = 32768;
+// tracer's column kernels leave wavefront slots of a small mesh's chip idle or end in a
+// mostly idle last round, and k_vimpl_reverse has one workgroup per CU or less (two steps
+// of the pi mesh 542 -> 508 us, icosa-6 x 70 with the split 1621 -> 1530). On larger meshes
+// the launches fill the chip, but short columns then share wavefronts (HALF_NODES), while
+// the second tracer's edge cotangents and workspace (15 node, 3 edge, 2 triangle arrays: at
+// most 4 GB here) cost about as much as they bring at nl = 70.
+constexpr int PAIR_NODES = 131072;
+// From this many nodes on, the launches of two tracers put both tracers of a short node
+// or edge column (31 levels and the bottom interface at most) into the halves of one
+// wavefront in kc_limit, kc_vertex and kc_edge; the tables stay wave-uniform. icosa-7 x 47
+// 3519 -> 3411 us (kc_limit 642 -> 602, kc_edge 601 -> 572, kc_vertex 514 -> 440), three
+// tracers with 1 % of the nodes at eight neighbours 6061 -> 5753, x 70 4337 -> 4316; icosa-6
+// x 47 922 -> 900. Smaller meshes need the wavefronts, and kernels without the halves, which
+// take 16 registers less: icosa-5 x 60 324 us, 331 with them.
+constexpr int HALF_NODES = 16384;
 
 // the node kernels: shallow columns, then (nl > 64) deep ones
 #define KC_NODES(KERN1, KERN2)                                                                \
@@ -992,20 +1049,20 @@ constexpr int PAIR_NODES = 32768;
         if (nd) KERN2<<<dim3(blocks_for(nd, WPB), y), dim3(256), 0, s>>>(a, ns, nd);             \
     } while (0)
 
-template <int NS, int DM>
+template <int NS, int DM, bool HALVES>
 int reverse_tracers(const ColArgs& a, const double* LOx, unsigned y, hipStream_t s) {
     kc_ghsc<<<dim3(blocks_for((a.m.N + GH_NODES - 1) / GH_NODES, WPB), y), dim3(256), 0, s>>>(a);
-    KC_NODES((kc_limit<1, DM>), (kc_limit<NS, DM>));
+    KC_NODES((kc_limit<1, DM, HALVES>), (kc_limit<NS, DM, false>));
     if (a.w_i) {
-        KC_NODES((kc_vertex<1, DM, true>), (kc_vertex<NS, DM, true>));
+        KC_NODES((kc_vertex<1, DM, true, HALVES>), (kc_vertex<NS, DM, true, false>));
         const int rc = launch_vimpl_reverse(a.m, a.w_i, a.hnn, a.dt, LOx, a.gLO, a.gwi,
                                             y == 2 ? a.gwi1 : nullptr, a.node_stride, s);
         if (rc) return rc;
         KC_NODES((kc_split<1>), (kc_split<NS>));
     } else {
-        KC_NODES((kc_vertex<1, DM, false>), (kc_vertex<NS, DM, false>));
+        KC_NODES((kc_vertex<1, DM, false, HALVES>), (kc_vertex<NS, DM, false, false>));
     }
-    kc_edge<NS><<<dim3(blocks_for(a.m.D, WPB), y), dim3(256), 0, s>>>(a);
+    kc_edge<NS, HALVES><<<dim3(blocks_for(a.m.D, WPB), y), dim3(256), 0, s>>>(a);
     kc_gnum<NS, DM><<<dim3(blocks_for(a.m.N, WPB), y), dim3(256), 0, s>>>(a);
     kc_tr<NS><<<dim3(blocks_for((a.m.E + TR_EL - 1) / TR_EL, WPB), y), dim3(256), 0, s>>>(a);
     KC_NODES((kc_gather<1, DM, NS>), (kc_gather<NS, DM, NS>));
@@ -1071,6 +1128,7 @@ int launch_backward_cols(const DevMesh& m, const NodeTab& tab, const int2* ekr, 
             n = pairs && !odd && K - j >= 2 ? 2 : 1;
             const int t1 = t + n - 1;
             a.first = pairs ? t < 2 : t == 0;
+            const bool halves = n == 2 && m.N >= HALF_NODES;
             a.g_vf = vf[odd]; a.gw = gw[odd]; a.gwi = gwi[odd];
             a.gw1 = gw[1]; a.gwi1 = gwi[1];
             a.T = f->T[t]; a.Told = f->T_old[t]; a.g_out = g_out[t];
@@ -1081,10 +1139,13 @@ int launch_backward_cols(const DevMesh& m, const NodeTab& tab, const int2* ekr, 
             a.pm = reinterpret_cast<const double2*>(tp.pf) + j * NL;
             a.gnode = reinterpret_cast<const double2*>(tp.gnode) + j * NL;
             const double* LOx = tp.LOx ? tp.LOx + j * NL : nullptr;
-            if (m.L <= 64)
-                rc = tab.dm == 6 ? reverse_tracers<1, 6>(a, LOx, n, s) : reverse_tracers<1, 8>(a, LOx, n, s);
-            else
-                rc = tab.dm == 6 ? reverse_tracers<2, 6>(a, LOx, n, s) : reverse_tracers<2, 8>(a, LOx, n, s);
+            const auto reverse = [&](auto ns) {
+                constexpr int NS = decltype(ns)::value;
+                if (tab.dm == 6)
+                    return halves ? reverse_tracers<NS, 6, true>(a, LOx, n, s) : reverse_tracers<NS, 6, false>(a, LOx, n, s);
+                return halves ? reverse_tracers<NS, 8, true>(a, LOx, n, s) : reverse_tracers<NS, 8, false>(a, LOx, n, s);
+            };
+            rc = m.L <= 64 ? reverse(std::integral_constant<int, 1>{}) : reverse(std::integral_constant<int, 2>{});
             if (rc) return rc;
         }
     }

@@ -339,7 +339,7 @@ __device__ __forceinline__ void pass1_shallow(const FusedArgs& a, int n, int4 hd
                 nb[ST * 64] = Tk;
             }
         }
-        const double Tm = HALF ? half_prev(Tk) : wave_prev(Tk, Tk);
+        const double Tm = HALF ? half_prev(Tk, Tk) : wave_prev(Tk, Tk);
         const double Tp = wave_next(Tk, 0.0);
         if (!wet) continue;
         double acc = 0.0;
@@ -762,15 +762,14 @@ __device__ __forceinline__ void adfv_compute(const FusedArgs& a, int2 nr,
                                              double (&out)[NS]) {
     const int L = a.m.L;
     double Tm[NS], A1[NS];
-    col_prev<NS, HALF>(Tc, Tm, col_bcast0<NS>(Tc));
-    col_prev<NS, HALF>(Ac, A1, col_bcast0<NS>(Ac));
+    col_prev_own<NS, HALF>(Tc, Tm);
+    col_prev_own<NS, HALF>(Ac, A1);
     // The reference's stencil depths (_z_stencil, tracer_adv.py:228-238) clamp Z[k-1] and
     // Z[k-2] at the top and Z[k+1] at the bottom. qc is needed at levels nr.x+1 .. nr.y-1
     // only (qd at nr.x+2 reads nr.x+1, qu at nr.y-2 reads nr.y-1): there 1 <= k <= L-2,
     // no clamp applies, and Z[k-1] is the plain lane shift of Z.
-    const double z0 = col_bcast0<NS>(Zc);
     double Zm1[NS], qc[NS], qu[NS], qd[NS];
-    col_prev<NS, HALF>(Zc, Zm1, z0);
+    col_prev_own<NS, HALF>(Zc, Zm1);
 #pragma unroll
     for (int s = 0; s < NS; ++s)
         qc[s] = 64 * s <= nr.y ? (A1[s] - Ac[s]) / nz_safe(Zm1[s] - Zc[s]) : 0.0;
@@ -1012,9 +1011,9 @@ __device__ __forceinline__ void pass2_shallow(const FusedArgs& a, int n, int2 nr
             }
         }
         double tvxm[NS], tvxp[NS], tvnm[NS], tvnp[NS];
-        col_prev<NS, HALF>(tvx, tvxm, col_bcast0<NS>(tvx));
+        col_prev_own<NS, HALF>(tvx, tvxm);
         col_next<NS>(tvx, tvxp, 0.0);
-        col_prev<NS, HALF>(tvn, tvnm, col_bcast0<NS>(tvn));
+        col_prev_own<NS, HALF>(tvn, tvnm);
         col_next<NS>(tvn, tvnp, 0.0);
         double fvc[NS], fvb[NS];
         adfv_compute<NS, HALF>(a, nr, Tc, Ac, Ws, ars, Zcs, zbs, fvc);
@@ -1255,8 +1254,8 @@ __device__ __forceinline__ void pass3_shallow(const FusedArgs& a, int n, int2 nr
             }
         }
         double Pm[NS], Mm[NS];
-        col_prev<NS, HALF>(Pc, Pm, col_bcast0<NS>(Pc));
-        col_prev<NS, HALF>(Mc, Mm, col_bcast0<NS>(Mc));
+        col_prev_own<NS, HALF>(Pc, Pm);
+        col_prev_own<NS, HALF>(Mc, Mm);
         double vl[NS];
 #pragma unroll
         for (int s = 0; s < NS; ++s) {

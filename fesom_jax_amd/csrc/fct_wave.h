@@ -42,32 +42,36 @@ __device__ __forceinline__ double lane_value(double v, int l) {
 template <bool HALF>
 __device__ __forceinline__ int col_lane() { return HALF ? lane_id() & 31 : lane_id(); }
 
-// wave_prev of the two half-wavefront columns, each one's level 0 keeping its own value:
-// row_bcast:15 puts lanes 15 and 47 into rows 1 and 3, row_shr:1 then moves within the rows
-// and leaves lanes 16 and 48 at that, lanes 0 and 32 at their own. (wave_next serves both
-// halves: it hands lane 31 the other column's level 0, and no caller uses that lane's.)
-__device__ __forceinline__ double half_prev(double v) {
-    int2 x = __builtin_bit_cast(int2, v), o;
-    o.x = __builtin_amdgcn_update_dpp(x.x, x.x, 0x142, 0xa, 0xf, false);
-    o.y = __builtin_amdgcn_update_dpp(x.y, x.y, 0x142, 0xa, 0xf, false);
+// wave_prev of the two half-wavefront columns, `first` at each one's level 0: row_bcast:15
+// puts lanes 15 and 47 into rows 1 and 3, row_shr:1 then moves within the rows and leaves
+// lanes 16 and 48 at that, lanes 0 and 32 at `first`. (wave_next serves both halves: it
+// hands lane 31 the other column's level 0, and no caller uses that lane's.)
+__device__ __forceinline__ double half_prev(double v, double first) {
+    int2 x = __builtin_bit_cast(int2, v), o = __builtin_bit_cast(int2, first);
+    o.x = __builtin_amdgcn_update_dpp(o.x, x.x, 0x142, 0xa, 0xf, false);
+    o.y = __builtin_amdgcn_update_dpp(o.y, x.y, 0x142, 0xa, 0xf, false);
     x.x = __builtin_amdgcn_update_dpp(o.x, x.x, 0x111, 0xf, 0xf, false);
     x.y = __builtin_amdgcn_update_dpp(o.y, x.y, 0x111, 0xf, 0xf, false);
     asm volatile("" : "+v"(x.x), "+v"(x.y));
     return __builtin_bit_cast(double, x);
 }
 
-// value at level k-1 of a column held as NS slots; `at0` is used at k = 0 (half-wavefront
-// columns: their own level 0)
+// value at level k-1 of a column held as NS slots; `at0` is used at k = 0
 template <int NS, bool HALF = false>
 __device__ __forceinline__ void col_prev(const double (&v)[NS], double (&o)[NS], double at0) {
     if constexpr (HALF) {
         static_assert(NS == 1);
-        o[0] = half_prev(v[0]);
+        o[0] = half_prev(v[0], at0);
         return;
     }
 #pragma unroll
     for (int s = 0; s < NS; ++s)
         o[s] = wave_prev(v[s], (s > 0) ? lane_value(v[s > 0 ? s - 1 : 0], 63) : at0);
+}
+// ... the column's own level 0 at k = 0
+template <int NS, bool HALF = false>
+__device__ __forceinline__ void col_prev_own(const double (&v)[NS], double (&o)[NS]) {
+    col_prev<NS, HALF>(v, o, HALF ? v[0] : lane_value(v[0], 0));
 }
 
 // value at level k+1; `atend` is used past the last slot lane

@@ -264,11 +264,14 @@ def test_flat_adjoint_of_long_columns(torch_dev):
 
 
 @pytest.mark.parametrize("level,nl,degree8,K,split", [
-    (2, 13, 0, 2, True), (3, 65, 10, 3, True), (3, 47, 0, 4, False), (3, 31, 0, 5, False)])
+    (2, 13, 0, 2, True), (3, 65, 10, 3, True), (3, 47, 0, 4, False), (3, 31, 0, 5, False),
+    (6, 31, 0, 2, False), (6, 34, 20, 3, True), (6, 66, 0, 2, False)])
 def test_adjoint_two_tracers_per_launch(level, nl, degree8, K, split, torch_dev):
     """Small meshes reverse two tracers per launch: against a plan with one tracer slot,
     which reverses them one after the other, bit for bit. Odd N * L (workspace alignment),
-    a last tracer alone, more tracers than slots, pairs cut by an odd number of slots."""
+    a last tracer alone, more tracers than slots, pairs cut by an odd number of slots; and
+    from level 6 on short columns' two tracers in the halves of a wavefront, with depths to
+    either side of the line."""
     import torch
     from fesom_jax_amd.adjoint import advect_fct_vjp
     from fesom_jax_amd.inputs import make_case
