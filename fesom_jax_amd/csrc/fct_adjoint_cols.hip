@@ -11,8 +11,8 @@
 // slots), so that their vertices are registers at fixed indices; through LDS rows indexed by
 // slot codes kc_vertex took 376 us per tracer of icosa-7 x 47 instead of 259. An edge hands
 // on two numbers and the sign of its flux (a bit per level) instead of eight: kc_edge 395
-// -> 301 us. icosa-7 x 47, two tracers: 7.56 -> 3.57 ms (tape 0.88); with the split at
-// icosa-6 x 70: 5.34 -> 1.63 ms.
+// -> 301 us. icosa-7 x 47, two tracers: 7.60 -> 3.39 ms (tape 0.79; two tracers per launch and
+// short columns in halves, below, included); with the split at icosa-6 x 70: 5.38 -> 1.54 ms.
 //
 //   kc_ghsc   (node)  cotangent of the horizontal divergence, read by edges and neighbours
 //   kc_limit  (node)  limited fluxes, limiter factors, P+/P-, cluster bounds, QR4C, and the

@@ -357,7 +357,8 @@ int fct_tracer_ab(const double* values, const double* valuesold, double* ttf_ab,
  * reversed through the Thomas recurrence (ops.py:121-168) and g_w_i is returned; the
  * moving-level stencil (Z3d, zbar3) is supported. Z3d, zbar3, helem, hnode and
  * hnode_new are constants (no cotangent). The first call allocates the adjoint
- * workspace (and the first with w_i one to max_tracers more [nod2D][nl] arrays) and reads
+ * workspace (15 node, 3 edge and 2 triangle arrays, twice that on meshes of up to
+ * 131072 nodes; nl > 128: the flat kernels' 30, 11 and 4; and the first with w_i one to max_tracers more [nod2D][nl] arrays) and reads
  * mesh tables back once; it also uses the forward workspace as its tape. Later calls
  * allocate nothing. */
 typedef struct fct_adjoint_args {
