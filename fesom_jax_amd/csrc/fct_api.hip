@@ -325,9 +325,12 @@ bool node_ring(const fct_mesh_desc* d, int dm, int de, int ne, const int4* es, c
             continue;
         }
         const int4 t = es[slot[i]];
-        // the edge's first triangle is the one before it in the ring, or the one behind
+        // the edge's first triangle is the one before it in the ring, or the one behind; a
+        // coastal edge has either of the two alone, which may be its second
         const int prev = i > 0 ? join[i - 1] : (closed >= 0 ? join[closed - 1] : -1);
-        const bool first_prev = prev >= 0 && els[prev] == d->edge_tri[2 * (t.x >> 1)];
+        const int32_t* et = d->edge_tri + 2 * (size_t)(t.x >> 1);
+        const bool first_prev = (prev >= 0 && els[prev] == et[0]) ||
+                                (join[i] >= 0 && els[join[i]] == et[1]);
         r[i] = make_int4(t.y, join[i] >= 0 ? els[join[i]] : (ne ? els[0] : 0), t.x,
                          (join[i] >= 0 ? range(join[i]) : 0) | (slot[i] << 16) |
                              (first_prev ? FCT_RING_PREV : 0));

@@ -1,0 +1,62 @@
+"""Meshes that the entry points accept besides those that the generator makes: an edge's
+triangles on either side (a coastal edge whose only triangle is its second one). compute_w
+and the upwind step against the oracle, bit for bit (every per-node sum runs in the oracle's
+(edge, side) order)."""
+
+import numpy as np
+import pytest
+
+from oracle import fct_numpy as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _rebuilt(m, **changed):
+    """The mesh with the given arrays in place of its own."""
+    from fesom_jax_amd.mesh import MESH_ARRAY_FIELDS, MESH_META_FIELDS, mesh_from_arrays
+    arrays = {k: np.array(changed.get(k, getattr(m, k))) for k in MESH_ARRAY_FIELDS}
+    meta = {k: getattr(m, k) for k in MESH_META_FIELDS}
+    meta["edge2D"] = len(arrays["edges"])
+    return mesh_from_arrays(arrays, meta, check_orientation=False)
+
+
+def _sides_swapped(m, which):
+    """The edges ``which`` with their two triangles exchanged. An edge's flux is the first
+    triangle's term minus the second one's, so the vectors change places and sign."""
+    et, cr = m.edge_tri.copy(), m.edge_cross_dxdy.copy()
+    et[which] = et[which][:, ::-1]
+    cr[which] = -cr[which][:, [2, 3, 0, 1]]
+    return _rebuilt(m, edge_tri=et, edge_cross_dxdy=cr)
+
+
+def _mesh(form, nl, degree8):
+    from fesom_jax_amd.meshgen import icosahedral_mesh
+    m = icosahedral_mesh(3, nl, seed=51, degree8=degree8, min_levels=3, polar_cap_deg=60.0)
+    coast = np.nonzero((m.edge_tri < 0).any(axis=1))[0]
+    if form == "coast_second":
+        return _sides_swapped(m, coast)
+    return _sides_swapped(m, np.nonzero(np.random.default_rng(52).random(m.edge2D) < 0.5)[0])
+
+
+FORMS = [("coast_second", 48, 0), ("coast_second", 70, 10), ("sides_mixed", 48, 0),
+         ("sides_mixed", 70, 10)]
+
+
+@pytest.mark.parametrize("form,nl,degree8", FORMS)
+def test_compute_w_and_upwind(form, nl, degree8, torch_dev):
+    import torch
+    from fesom_jax_amd.ale import compute_w
+    from fesom_jax_amd.inputs import make_case
+    from fesom_jax_amd.tracer_adv import advect_one, get_plan
+    m = _mesh(form, nl, degree8)
+    c = make_case(m, seed=54, dt=2700.0)
+    assert get_plan(m, torch_dev).fused_available
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(torch_dev)
+    print(f"[forms] {form} N={m.nod2D} D={m.edge2D} nl={nl}", flush=True)
+    w = compute_w(m, t(c["uv"]), t(c["helem"])).cpu().numpy()
+    assert np.array_equal(w, O.compute_w(m, c["uv"], c["helem"]))
+    T, To = c["T"][0], 0.98 * c["T"][0] + 0.3
+    flow = [c[k] for k in ("uv", "w_e", "helem", "hnode", "hnode_new")]
+    got, _ = advect_one(m, *map(t, flow), t(T), t(To), dt=c["dt"])
+    want, _ = O.advect_one(m, *flow, T, To, dt=c["dt"])
+    assert np.array_equal(got.cpu().numpy(), want)
