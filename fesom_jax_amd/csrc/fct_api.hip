@@ -270,7 +270,8 @@ bool fused_mesh_ok(const fct_mesh_desc* d, const std::vector<int>& eoff,
 
 // Ring of node n (NodeTab::ring): from its table edges `es` (de of them; .x code, .y
 // neighbour, .w >> 16 the vertex slots of element slot q), its ne elements `els` and their
-// layer ranges (es[q].w, low 16 bits). False if the fans do not fit dm slots.
+// layer ranges (es[q].w, low 16 bits). False if the fans do not fit dm slots, or if an edge's
+// triangles are not the two beside its slot.
 bool node_ring(const fct_mesh_desc* d, int dm, int de, int ne, const int4* es, const int* els, int4* r) {
     int nb[8][2], el[8][2], cnt[8] = {};      // per slot: the slots its triangles join it to
     for (int q = 0; q < ne; ++q) {
@@ -325,12 +326,14 @@ bool node_ring(const fct_mesh_desc* d, int dm, int de, int ne, const int4* es, c
             continue;
         }
         const int4 t = es[slot[i]];
-        // the edge's first triangle is the one before it in the ring, or the one behind; a
-        // coastal edge has either of the two alone, which may be its second
+        // the edge's first triangle is the one before it in the ring, or the one behind (a
+        // coastal edge has either of the two alone, which may be its second); where two
+        // edges join the same nodes, the slots' triangles are not their edges' own
         const int prev = i > 0 ? join[i - 1] : (closed >= 0 ? join[closed - 1] : -1);
+        const int before = prev >= 0 ? els[prev] : -1, behind = join[i] >= 0 ? els[join[i]] : -1;
         const int32_t* et = d->edge_tri + 2 * (size_t)(t.x >> 1);
-        const bool first_prev = (prev >= 0 && els[prev] == et[0]) ||
-                                (join[i] >= 0 && els[join[i]] == et[1]);
+        const bool first_prev = before == et[0] && behind == et[1];
+        if (!first_prev && !(before == et[1] && behind == et[0])) return false;
         r[i] = make_int4(t.y, join[i] >= 0 ? els[join[i]] : (ne ? els[0] : 0), t.x,
                          (join[i] >= 0 ? range(join[i]) : 0) | (slot[i] << 16) |
                              (first_prev ? FCT_RING_PREV : 0));

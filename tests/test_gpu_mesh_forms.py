@@ -1,7 +1,7 @@
 """Meshes that the entry points accept besides those that the generator makes: an edge's
-triangles on either side (a coastal edge whose only triangle is its second one). compute_w
-and the upwind step against the oracle, bit for bit (every per-node sum runs in the oracle's
-(edge, side) order)."""
+triangles on either side (a coastal edge whose only triangle is its second one), two edges
+between the same nodes (a crack). compute_w and the upwind step against the oracle, bit for
+bit (every per-node sum runs in the oracle's (edge, side) order)."""
 
 import numpy as np
 import pytest
@@ -29,17 +29,49 @@ def _sides_swapped(m, which):
     return _rebuilt(m, edge_tri=et, edge_cross_dxdy=cr)
 
 
+def _coastal(m):
+    c = np.zeros(m.nod2D, bool)
+    c[m.edges[(m.edge_tri < 0).any(axis=1)].reshape(-1)] = True
+    return c
+
+
+def _cracked(m, count, seed):
+    """``count`` interior edges between coastal nodes (whose fans are open), no two at one
+    node, as two edges between the same nodes: the first keeps the first triangle, a new one
+    at the end of the list has the second."""
+    rng = np.random.default_rng(seed)
+    deg = np.bincount(m.edges.reshape(-1), minlength=m.nod2D)
+    coast = _coastal(m)
+    seen, pick = set(), []
+    for e in rng.permutation(np.nonzero((m.edge_tri >= 0).all(axis=1) & coast[m.edges].all(axis=1))[0]):
+        a, b = m.edges[e]
+        if len(pick) < count and a not in seen and b not in seen and max(deg[a], deg[b]) < 8:
+            pick.append(e)
+            seen.update((a, b))
+    assert pick
+    pick = np.array(pick)
+    et, cr, ud = m.edge_tri.copy(), m.edge_cross_dxdy.copy(), m.edge_up_dn_tri.copy()
+    more_et, more_cr = et[pick].copy(), cr[pick].copy()
+    more_et[:, 0], more_cr[:, :2] = -1, 0.0
+    et[pick, 1], cr[pick, 2:], ud[pick] = -1, 0.0, -1
+    return _rebuilt(m, edges=np.r_[m.edges, m.edges[pick]], edge_tri=np.r_[et, more_et],
+                    edge_cross_dxdy=np.r_[cr, more_cr], edge_up_dn_tri=np.r_[ud, ud[pick]],
+                    edge_dxdy=np.r_[m.edge_dxdy, m.edge_dxdy[pick]])
+
+
 def _mesh(form, nl, degree8):
     from fesom_jax_amd.meshgen import icosahedral_mesh
     m = icosahedral_mesh(3, nl, seed=51, degree8=degree8, min_levels=3, polar_cap_deg=60.0)
     coast = np.nonzero((m.edge_tri < 0).any(axis=1))[0]
     if form == "coast_second":
         return _sides_swapped(m, coast)
-    return _sides_swapped(m, np.nonzero(np.random.default_rng(52).random(m.edge2D) < 0.5)[0])
+    if form == "sides_mixed":
+        return _sides_swapped(m, np.nonzero(np.random.default_rng(52).random(m.edge2D) < 0.5)[0])
+    return _cracked(m, 40, 53)
 
 
 FORMS = [("coast_second", 48, 0), ("coast_second", 70, 10), ("sides_mixed", 48, 0),
-         ("sides_mixed", 70, 10)]
+         ("sides_mixed", 70, 10), ("cracked", 48, 0), ("cracked", 70, 10)]
 
 
 @pytest.mark.parametrize("form,nl,degree8", FORMS)
