@@ -1068,32 +1068,52 @@ int check_vdiff(const fct_plan* p, const fct_vdiff_args* a) {
     return FCT_OK;
 }
 
+// tracers j0 and j0 + 1 (or the last one alone) of a checked call
+VdiffCall vdiff_chunk(const fct_vdiff_args* a, int j0) {
+    VdiffCall c;
+    c.K = std::min(2, a->ntracers - j0);
+    c.dt = a->dt;
+    c.Kv = a->Kv;
+    c.hnn = a->hnode_new;
+    c.Z3d = a->Z3d;
+    for (int j = 0; j < c.K; ++j) {
+        c.T[j] = a->T[j0 + j];
+        c.Tn[j] = a->T_new[j0 + j];
+        c.bc[j] = a->bc_surf ? a->bc_surf[j0 + j] : nullptr;
+        c.sw[j] = a->sw_3d ? a->sw_3d[j0 + j] : nullptr;
+    }
+    if (a->floor_tracer >= j0 && a->floor_tracer < j0 + c.K) {
+        c.floor_j = a->floor_tracer - j0;
+        c.floor_v = a->floor_value;
+    }
+    return c;
+}
+
+// whether some solve of the call is one for the kernel with scratch
+bool vdiff_wants_scratch(const fct_plan* p, const fct_vdiff_args* a) {
+    for (int j0 = 0; j0 < a->ntracers; j0 += 2)
+        if (!vdiff_by_lds(p->m, vdiff_chunk(a, j0))) return true;
+    return false;
+}
+
 // the solves of a checked call, tracers two at a time, on `grid` workgroups whose
-// scratch slots start at `scratch`
+// scratch slots start at `scratch` (NULL: all through LDS)
 int run_vdiff(const fct_plan* p, const fct_vdiff_args* a, int grid, double* scratch,
               hipStream_t s) {
-    const int K = a->ntracers;
-    for (int j0 = 0; j0 < K; j0 += 2) {
-        VdiffCall c;
-        c.K = std::min(2, K - j0);
-        c.dt = a->dt;
-        c.Kv = a->Kv;
-        c.hnn = a->hnode_new;
-        c.Z3d = a->Z3d;
-        for (int j = 0; j < c.K; ++j) {
-            c.T[j] = a->T[j0 + j];
-            c.Tn[j] = a->T_new[j0 + j];
-            c.bc[j] = a->bc_surf ? a->bc_surf[j0 + j] : nullptr;
-            c.sw[j] = a->sw_3d ? a->sw_3d[j0 + j] : nullptr;
-        }
-        if (a->floor_tracer >= j0 && a->floor_tracer < j0 + c.K) {
-            c.floor_j = a->floor_tracer - j0;
-            c.floor_v = a->floor_value;
-        }
-        const int rc = launch_vdiff(p->m, c, grid, scratch, s);
+    for (int j0 = 0; j0 < a->ntracers; j0 += 2) {
+        const int rc = launch_vdiff(p->m, vdiff_chunk(a, j0), grid, scratch, s);
         if (rc) return rc;
     }
     return FCT_OK;
+}
+
+// A capture takes no allocation: a call that would make one then does without where the
+// other form can (both give the same bits).
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;      // (the null stream while another one is captured)
 }
 
 }  // namespace
@@ -1103,12 +1123,15 @@ extern "C" {
 int fct_impl_vert_diff(fct_plan* p, const fct_vdiff_args* a, void* stream) {
     int rc = check_vdiff(p, a);
     if (rc) return rc;
-    if (!p->vd_scratch && !vdiff_fits(p->m.L)) {
+    const bool fits = vdiff_fits(p->m.L);
+    if (!p->vd_scratch && vdiff_wants_scratch(p, a) && !(fits && capturing((hipStream_t)stream))) {
         int cus = 0;
         HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device));
         int grid = 0;
         if ((rc = vdiff_max_grid(cus, &grid))) return rc;
-        if ((rc = dev_alloc(p, &p->vd_scratch, vdiff_scratch_doubles(p->m.L, grid)))) return rc;
+        rc = dev_alloc(p, &p->vd_scratch, vdiff_scratch_doubles(p->m.L, grid));
+        if (rc && !fits) return rc;
+        if (rc) (void)hipGetLastError();
         p->vd_grid = grid;
     }
     return run_vdiff(p, a, p->vd_grid, p->vd_scratch, (hipStream_t)stream);
@@ -1117,7 +1140,7 @@ int fct_impl_vert_diff(fct_plan* p, const fct_vdiff_args* a, void* stream) {
 int fct_impl_vert_diff_static(fct_plan* p, const fct_vdiff_args* a, void* stream) {
     int rc = check_vdiff(p, a);
     if (rc) return rc;
-    if (vdiff_fits(p->m.L)) return run_vdiff(p, a, 0, nullptr, (hipStream_t)stream);
+    if (!vdiff_wants_scratch(p, a)) return run_vdiff(p, a, 0, nullptr, (hipStream_t)stream);
     // workgroups: as many as the fixed scratch has slots for, at most the resident count
     const size_t slot = vdiff_scratch_doubles(p->m.L, 1);
     const size_t slots = (size_t)FCT_VDIFF_STATIC_BYTES / sizeof(double) / slot;

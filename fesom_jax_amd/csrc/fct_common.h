@@ -392,12 +392,14 @@ struct VdiffCall {
     int floor_j = -1;               // index within the call, -1 = none
     double floor_v = 0.0;
 };
-// Whether columns of L levels fit LDS; launch_vdiff then needs no scratch (and ignores
-// max_grid and scratch).
+// Whether columns of L levels fit LDS, and whether such a call is better solved there
+// (k_vdiff_lds, no scratch) or by k_vdiff out of the scratch.
 bool vdiff_fits(int L);
+bool vdiff_by_lds(const DevMesh& m, const VdiffCall& c);
 // Workgroups the GPU holds at once over every kernel variant (cus compute units).
 int vdiff_max_grid(int cus, int* out);
 size_t vdiff_scratch_doubles(int L, int grid);
+// scratch may be NULL where the columns fit LDS
 int launch_vdiff(const DevMesh& m, const VdiffCall& c, int max_grid, double* scratch,
                  hipStream_t s);
 // Device address of the fixed scratch of fct_impl_vert_diff_static on `device` (the

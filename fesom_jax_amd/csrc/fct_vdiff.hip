@@ -3,8 +3,8 @@
 // the optional lower bound on wet layers that the step applies to salinity right after
 // it (step.py:456).
 //
-// Columns that fit LDS (nl up to about 980) take k_vdiff_lds below; k_vdiff is for longer
-// ones. Its mapping: a workgroup is one 64-lane wavefront; lane = node column. The Thomas
+// Two forms with the same results: k_vdiff_lds below, columns in LDS, and k_vdiff, which is
+// better for short and for very long columns (vdiff_by_lds). k_vdiff's mapping: a workgroup is one 64-lane wavefront; lane = node column. The Thomas
 // recurrence (ops.py:121-168) runs down each lane's column in the reference's operation
 // order, over the rows [0, Lw) where Lw is the deepest bottom in the wavefront (rows
 // further down are dry in every lane and solve to +0 in the reference too). The inputs
@@ -559,6 +559,33 @@ int vd_resident_k(bool z3d, bool sw, int cus, int* out) {
 
 bool vdiff_fits(int L) { return vi_columns(L, 5) >= 1; }
 
+// k_vdiff_lds has a wavefront per column, so short columns leave lanes and whole rounds of
+// workgroups empty; long ones leave few columns per workgroup, and so few recurrences in
+// flight. k_vdiff always has 64 per wavefront, but waits out one level's chain on a mesh
+// that does not fill the chip, and reads 64-byte pieces, one more per row unless rows start on
+// one (`pieces` counts that as seven levels). Both timed (us, k_vdiff then k_vdiff_lds, bc):
+//   short, two tracers: 114,689 x 16  48,  65;  x 24  73,  76;  x 30  106,  83
+//                       458,753 x 24 261, 317;  x 30 379, 338;  x 48  583, 471
+//   short, one tracer:  114,689 x 24  52,  66;  x 34  83,  77;  458,753 x 32 238, 318
+//   long, two tracers:   28,673 x 200 217, 206; x 256 270, 349; 114,689 x 128 367, 380;
+//                       458,753 x 110 1469, 1123; x 160 1720, 2039
+//   long, one tracer:    28,673 x 128  92,  86; x 160 116, 127; 114,689 x 320 660, 1479;
+//                         7,167 x 600 379, 343; x 640 411, 591;  1,790 x 1000 634, 346
+// Z3d and shortwave cost k_vdiff_lds less (`extra`). Between the lines below and the sizes
+// where the two are equal lie at most a few per cent.
+bool vdiff_by_lds(const DevMesh& m, const VdiffCall& c) {
+    if (!vdiff_fits(m.L)) return false;
+    const bool sw = c.sw[0] || (c.K > 1 && c.sw[1]);
+    const int extra = (c.Z3d != nullptr) + sw, L = m.L, C = vi_columns(L, 3 + c.K);
+    const int pieces = L + (L % VD_KC ? VD_KC - 1 : 0);
+    const int size = m.N < 65536 ? 0 : (m.N < 262144 ? 1 : 2);
+    if (pieces < (c.K == 1 ? 32 + 7 * size - 4 * extra : 24 + 9 * size / 2 - 2 * extra)) return false;
+    // rounds of the chip's 1024 resident workgroups
+    const double rounds = m.N / (1024.0 * C);
+    if (rounds <= 3.0 * c.K + 0.5 + 0.75 * extra) return true;
+    return C + (L % VD_KC != 0) >= (c.K == 1 ? 11 - extra : 8 - extra / 2);
+}
+
 int vdiff_max_grid(int cus, int* out) {
     int best = 0;
     for (int K = 1; K <= 2; ++K)
@@ -602,7 +629,7 @@ int launch_vdiff(const DevMesh& m, const VdiffCall& c, int max_grid, double* scr
         sw = sw || c.sw[j] != nullptr;
     }
     if (a.nblk == 0) return FCT_OK;
-    if (vdiff_fits(m.L))
+    if (!scratch || vdiff_by_lds(m, c))
         return c.K == 1 ? vd_lds_dispatch<1>(m, a, c.Z3d != nullptr, sw, s)
                         : vd_lds_dispatch<2>(m, a, c.Z3d != nullptr, sw, s);
     const int grid = std::min(a.nblk, max_grid);

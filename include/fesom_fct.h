@@ -246,10 +246,13 @@ int fct_compute_w(fct_plan* plan, const double* uv, const double* helem, double*
  * (fesom_jax/tracer_diff.py:68-128; impl_vert_diff, :131-141, is the two-tracer call
  * with sw_3d on the first tracer only). One tridiagonal solve per node column, the
  * same matrix for every tracer of the call. Optionally clamps one tracer from below on
- * wet layers, the salinity floor of fesom_jax/step.py:456. The first call allocates a
- * scratch bounded by the GPU's resident workgroups (3 * nl * 64 doubles each), later
- * calls allocate nothing. T_new[j] may be T[j] (in place); no other aliasing between
- * the tracers' fields is allowed (FCT_E_INVALID). */
+ * wet layers, the salinity floor of fesom_jax/step.py:456. Columns are solved out of LDS
+ * without scratch, or, where that is slower (below about 30 levels and above about 115, by
+ * mesh size and tracers) or nl > 1010, out of a scratch bounded by the GPU's resident
+ * workgroups (3 * nl * 64 doubles each) that the first such call allocates; one that is
+ * captured before that goes without it where nl <= 1010. Both forms give the same bits.
+ * T_new[j] may be T[j] (in place); no other aliasing between the tracers' fields is allowed
+ * (FCT_E_INVALID). */
 #define FCT_VDIFF_MAX_TRACERS 8
 typedef struct fct_vdiff_args {
     int32_t ntracers;                 /* 1 .. FCT_VDIFF_MAX_TRACERS */
@@ -270,15 +273,15 @@ int fct_impl_vert_diff(fct_plan* plan, const fct_vdiff_args* args, void* stream)
 /* ---- implicit vertical diffusion that allocates nothing ----------------------------
  * No counterpart in the reference. For callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid it): the
- * same arguments, checks and results as fct_impl_vert_diff, bit for bit, but the solver
- * scratch is a fixed device array of FCT_VDIFF_STATIC_BYTES per GPU (reserved when the
- * library is loaded, held until the process ends) instead of plan workspace, and the
- * call makes no allocation. The workgroup count is capped to the array's slots
- * (3 * nl * 64 doubles each), so at large nl the call may run below
+ * same arguments, checks and results as fct_impl_vert_diff, bit for bit, but where that
+ * takes a scratch this one takes a fixed device array of FCT_VDIFF_STATIC_BYTES per GPU
+ * (reserved when the library is loaded, held until the process ends) instead of plan
+ * workspace, and the call makes no allocation. The workgroup count is then capped to the
+ * array's slots (3 * nl * 64 doubles each), so at large nl the call may run below
  * fct_impl_vert_diff's speed; an nl whose single slot exceeds the array is refused
- * (FCT_E_INVALID). Nothing in the array needs to start at zero. Every call on a GPU
- * shares that GPU's array and leaves its contents behind: calls that overlap on one GPU
- * (other streams, other threads) race. */
+ * (FCT_E_INVALID). Nothing in the array needs to start at zero. Such calls on a GPU share
+ * that GPU's array and leave their contents behind: any that overlap on one GPU (other
+ * streams, other threads) race. */
 #define FCT_VDIFF_STATIC_BYTES (64 << 20)
 int fct_impl_vert_diff_static(fct_plan* plan, const fct_vdiff_args* args, void* stream);
 

@@ -181,3 +181,33 @@ def test_column_sizes(level, nl, K, moving, torch_dev):
     for j in range(K):
         _eq(got[j], VD.impl_vert_diff_one(m, Ts[j], Kv, h, dt=2700.0, bc_surf=bc,
                                           sw_3d=sw if j == 0 else None, **Z), (nl, j))
+
+
+@pytest.mark.parametrize("level,nl,K,moving,scratch", [
+    (6, 16, 2, False, True), (6, 24, 2, False, False), (6, 23, 1, False, True),
+    (6, 23, 1, True, False), (6, 200, 2, False, False), (6, 256, 2, True, True),
+    (5, 640, 1, False, True), (4, 640, 1, False, False), (6, 23, 3, False, True)])
+def test_kernel_by_size(level, nl, K, moving, scratch, torch_dev):
+    """Short columns, and long ones on a mesh that fills the chip, take the kernel with
+    scratch, which then allocates it; the others the LDS solve (of three tracers at nl = 23
+    the pair, while the last one alone takes the other kernel). Both are the oracle's bits."""
+    from fesom_jax_amd.meshgen import icosahedral_mesh
+    from fesom_jax_amd.tracer_adv import get_plan
+    from fesom_jax_amd.tracer_diff import diffuse_tracers
+    m = icosahedral_mesh(level, nl, seed=121, min_levels=2)
+    t = _t(torch_dev)
+    rng = np.random.default_rng(122)
+    h = np.where(m.node_layer_mask, 5.0 + 40.0 * rng.random(m.area.shape), 0.0)
+    Ts = [10.0 + rng.standard_normal(m.area.shape) for _ in range(K)]
+    Kv = _kv(m, 123)
+    bc, sw = _forcing(m, 124)
+    Z3d = m.zbar_3d_n * (1.0 + 0.01 * rng.random(m.zbar_3d_n.shape)) if moving else None
+    before = get_plan(m, torch_dev).own_bytes()
+    out = diffuse_tracers(m, [t(x) for x in Ts], t(Kv), t(h), dt=2700.0, bc_surf=[t(bc)] * K,
+                          sw_3d=[t(sw)] + [None] * (K - 1) if moving else None,
+                          Z3d=None if Z3d is None else t(Z3d))
+    assert (get_plan(m, torch_dev).own_bytes() > before) == scratch
+    for j in range(K):
+        want = VD.impl_vert_diff_one(m, Ts[j], Kv, h, dt=2700.0, bc_surf=bc,
+                                     sw_3d=sw if moving and j == 0 else None, Z3d=Z3d)
+        _eq(out[j], want, j)

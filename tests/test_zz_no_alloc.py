@@ -77,3 +77,53 @@ def test_static_scratch_argument_errors(torch_dev):
     rc = plan.lib.fct_impl_vert_diff_static(plan.ptr, ctypes.byref(args), None)
     assert rc == _lib.FCT_E_INVALID
     assert b"ntracers" in plan.lib.fct_last_error()
+
+
+def test_static_scratch_of_the_scratch_kernel(torch_dev):
+    """Sizes that the kernel with scratch solves (the ones above are solved out of LDS):
+    long columns on more workgroups than the array has slots for, then short ones of
+    another mesh on what the first call left in it."""
+    import torch
+    from fesom_jax_amd import _lib
+    for level, nl, K, seed in ((7, 256, 2, 70), (6, 16, 1, 80)):
+        m, plan, T, Kv, hnn, bc, sw = _case(level, nl, K, seed, torch_dev)
+        resident = 4 * torch.cuda.get_device_properties(torch_dev).multi_processor_count
+        slots = (64 << 20) // (3 * nl * 64 * 8)
+        print(f"[no-alloc] icosa-{level} N={m.nod2D} nl={nl} K={K} slots={slots}", flush=True)
+        assert nl < 256 or slots < min(resident, m.nod2D // 64)
+        before = plan.own_bytes()
+        got = _call("fct_impl_vert_diff_static", plan, torch_dev, T, Kv, hnn, 2700.0, bc=bc, sw=sw)
+        assert plan.own_bytes() == before
+        want = _call("fct_impl_vert_diff", plan, torch_dev, T, Kv, hnn, 2700.0, bc=bc, sw=sw)
+        assert plan.own_bytes() > before        # its own scratch: the kernel that needs one
+        for j in range(K):
+            assert np.array_equal(got[j], want[j]), (nl, j)
+            assert not np.array_equal(got[j], T[j].cpu().numpy())
+
+
+def test_first_call_under_capture(torch_dev):
+    """A first call that would allocate its scratch runs without it when captured."""
+    import torch
+    from fesom_jax_amd import _lib
+    m, plan, T, Kv, hnn, bc, sw = _case(6, 16, 1, 90, torch_dev)
+    out = torch.empty_like(T[0])
+    Tp, Op = (c_void_p * 1)(T[0].data_ptr()), (c_void_p * 1)(out.data_ptr())
+    P = lambda a: ctypes.cast(a, ctypes.POINTER(c_void_p))
+    args = _lib.FctVdiffArgs(ntracers=1, floor_tracer=-1, dt=2700.0, floor_value=0.0,
+                             Kv=Kv.data_ptr(), hnode_new=hnn.data_ptr(), Z3d=None, T=P(Tp),
+                             bc_surf=None, sw_3d=None, T_new=P(Op))
+    before = plan.own_bytes()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        s = torch.cuda.current_stream(torch_dev).cuda_stream
+        _lib.check(plan.lib.fct_impl_vert_diff(plan.ptr, ctypes.byref(args), c_void_p(s)), "captured")
+    assert plan.own_bytes() == before
+    want = _call("fct_impl_vert_diff", plan, torch_dev, T, Kv, hnn, 2700.0)
+    assert plan.own_bytes() > before
+    for scale in (1.0, 1.5, 0.5):
+        T[0].mul_(scale)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = _call("fct_impl_vert_diff", plan, torch_dev, T, Kv, hnn, 2700.0)
+        assert np.array_equal(out.cpu().numpy(), want[0]), scale
