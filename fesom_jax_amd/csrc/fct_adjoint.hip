@@ -1,7 +1,7 @@
 // Reverse mode of one FP64 FCT step for the meshes that the column kernels
-// (fct_adjoint_cols.hip) do not take: nl > 128, or no fused node tables. With or without
-// the implicit split w_i and the moving-level stencil Z3d/zbar3, which are treated as
-// constants.
+// (fct_adjoint_cols.hip) do not take: nl > 128, no rings of triangles, or short columns on
+// a mesh that fills the chip (adjoint_by_columns). With or without the implicit split w_i
+// and the moving-level stencil Z3d/zbar3, which are treated as constants.
 //
 // The forward tape is the phased path's dense intermediates of the same step (vflux,
 // LO, tr_xy, gnode, adf_h, adf_v, the node bounds tvmax/tvmin, P+/P-, the limiter

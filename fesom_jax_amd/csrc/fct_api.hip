@@ -76,9 +76,9 @@ struct fct_plan {
     // fpf holds the limiter factors as (plus, minus) pairs; fadfv the vertical
     // antidiffusive flux pass 2 computes and pass 3 reads
     double *fLO = nullptr, *fgnode = nullptr, *fadfh = nullptr, *fpf = nullptr, *fadfv = nullptr;
-    // adjoint workspace (allocated on the first fct_backward): the column kernels' where
-    // the mesh has node tables and nl <= 128, else the flat kernels'
-    bool adj_ready = false;
+    // adjoint workspaces of the flat and of the column kernels, each allocated on the first
+    // fct_backward that takes them (adjoint_by_columns)
+    bool flat_ready = false, cols_ready = false;
     AdjointWork aw{};
     AdjointCols ac{};
     double* adj_LOx = nullptr;
@@ -397,25 +397,43 @@ int upload_element_lists(fct_plan* p, const int** ud_off, const int** ud_list, c
     return FCT_OK;
 }
 
-bool adjoint_by_columns(const fct_plan* p) { return p->tab.ring != nullptr && p->m.L <= 128; }
+// Whether the backward of K tracers takes the column kernels. They cost a wavefront per
+// column whatever its levels, so on a mesh that fills the chip short columns are faster one
+// thread per level (us, flat kernels then column kernels):
+//   one tracer:   28,673 x 12   323,  373;  x 16  373,  378;  114,689 x 16 1396, 1506;
+//                114,689 x 20  1759, 1578;  458,753 x 16 5379, 5830;  x 20 6766, 6025
+//   two tracers:  28,673 x 8    473,  512;  x 12  614,  551;  114,689 x 12 2088, 2177;
+//                114,689 x 16  2667, 2266;  458,753 x 12 8004, 10035; x 16 10284, 10322
+//   under the split, one tracer: 114,689 x 8 949, 1472;  x 12 1527, 1582; x 16 2158, 1657
+bool adjoint_by_columns(const fct_plan* p, int K, bool split) {
+    const DevMesh& m = p->m;
+    if (!p->tab.ring || m.L > 128) return false;
+    if (m.N < 16384) return true;
+    return m.L > (split ? 8 : (m.N < 65536 ? 8 : 12) + (K == 1 ? 4 : 0));
+}
 
-// Adjoint workspace: of the column kernels, or of the flat ones with their phased tape.
-int ensure_adjoint(fct_plan* p) {
-    if (p->adj_ready) return FCT_OK;
+// Workspace of the backward's column kernels.
+int ensure_columns(fct_plan* p) {
+    if (p->cols_ready) return FCT_OK;
     int rc;
     const DevMesh& m = p->m;
-    if (adjoint_by_columns(p)) {
-        AdjointCols& c = p->ac;
-        const int nt = c.tracers = adjoint_cols_tracers(m);
-        if ((rc = dev_alloc(p, &c.node, adjoint_cols_node(m, nt))) ||
-            (rc = dev_alloc(p, &c.edge_up, (size_t)m.D * (m.L <= 64 ? 1 : 2) * nt)) ||
-            (rc = dev_alloc(p, &c.edge, adjoint_cols_edge(m, nt))) ||
-            (rc = dev_alloc(p, &c.elem, adjoint_cols_elem(m, nt))) ||
-            (rc = upload_element_lists(p, &c.ud_off, &c.ud_ent, &c.et_off, &c.et_ent)))
-            return rc;
-        p->adj_ready = true;
-        return FCT_OK;
-    }
+    AdjointCols& c = p->ac;
+    const int nt = c.tracers = adjoint_cols_tracers(m);
+    if ((rc = dev_alloc(p, &c.node, adjoint_cols_node(m, nt))) ||
+        (rc = dev_alloc(p, &c.edge_up, (size_t)m.D * (m.L <= 64 ? 1 : 2) * nt)) ||
+        (rc = dev_alloc(p, &c.edge, adjoint_cols_edge(m, nt))) ||
+        (rc = dev_alloc(p, &c.elem, adjoint_cols_elem(m, nt))) ||
+        (rc = upload_element_lists(p, &c.ud_off, &c.ud_ent, &c.et_off, &c.et_ent)))
+        return rc;
+    p->cols_ready = true;
+    return FCT_OK;
+}
+
+// Workspace of the backward's flat kernels, with their phased tape.
+int ensure_flat(fct_plan* p) {
+    if (p->flat_ready) return FCT_OK;
+    int rc;
+    const DevMesh& m = p->m;
     const size_t NL = (size_t)m.N * m.L, DL = (size_t)m.D * m.L, EL = (size_t)m.E * m.L;
     if ((rc = ensure_phased(p))) return rc;
     AdjointWork& w = p->aw;
@@ -433,7 +451,7 @@ int ensure_adjoint(fct_plan* p) {
         (rc = dev_alloc(p, &w.g_tr, 2 * EL)) ||
         (rc = upload_element_lists(p, &w.ud_off, &w.ud_ent, &w.et_off, &w.et_ent)))
         return rc;
-    p->adj_ready = true;
+    p->flat_ready = true;
     return FCT_OK;
 }
 
@@ -1552,10 +1570,10 @@ int fct_backward(fct_plan* p, const fct_step_args* a, const fct_adjoint_args* g,
     for (int j = 0; j < a->ntracers; ++j)
         if (!a->T[j] || !a->T_old[j] || !g->g_T_new[j] || !g->g_T[j] || !g->g_T_old[j])
             return set_error(FCT_E_INVALID, "tracer %d has a NULL field", j);
-    int rc = ensure_adjoint(p);
-    if (rc) return rc;
+    int rc;
     const size_t NL = (size_t)p->m.N * p->m.L;
-    if (adjoint_by_columns(p)) {
+    if (adjoint_by_columns(p, a->ntracers, a->w_i != nullptr)) {
+        if ((rc = ensure_columns(p))) return rc;
         if (a->w_i && !p->adj_LOx && (rc = dev_alloc(p, &p->adj_LOx, NL * p->kw))) return rc;
         FusedTape t;
         t.kw = p->kw; t.vflux = p->vflux; t.LO = p->fLO; t.LOx = p->adj_LOx; t.gnode = p->fgnode;
@@ -1563,6 +1581,7 @@ int fct_backward(fct_plan* p, const fct_step_args* a, const fct_adjoint_args* g,
         return launch_backward_cols(p->m, p->tab, p->ekr, t, p->ac, p->tune, a, g->g_T_new, g->g_T,
                                     g->g_T_old, g->g_uv, g->g_w_e, g->g_w_i, (hipStream_t)stream);
     }
+    if ((rc = ensure_flat(p))) return rc;
     if (a->w_i && !p->aw.LOx &&
         ((rc = dev_alloc(p, &p->aw.LOx, NL)) || (rc = dev_alloc(p, &p->aw.gwi, NL))))
         return rc;

@@ -94,6 +94,9 @@ def estimate_work_bytes(mesh, K, adjoint):
         # phased tape, cotangent scratch, element -> edge lists
         total += 8 * (12 * NL + 2 * EL + DL) + 8 * (20 * NL + 10 * DL + 2 * EL)
         total += 16 * D + 8 * E + 64
+        if L <= 16:
+            # short columns: requests of one and of more tracers may take either form
+            total += 8 * (31 * NL + 6 * DL + 4 * EL) + 32 * D + 8 * E + 64
     return int(total)
 
 

@@ -234,8 +234,10 @@ int fct_ice_fct_solve(fct_plan* plan, const fct_ice_args* args, void* stream);
  * w = compute_w(mesh, uv, helem) (fesom_jax/ale.py:309-365), the w_e the step takes:
  * per-level edge divergence into the nodes, cumulative sum from the bottom, divided by
  * the interface area; zero outside each node's interfaces [nzmin, nzmax]. uv is
- * [elem2D][nl][2], helem [elem2D][nl], w [nod2D][nl] (device). nl <= 128. Uses
- * no workspace and allocates nothing. */
+ * [elem2D][nl][2], helem [elem2D][nl], w [nod2D][nl] (device). nl <= 128. Each triangle
+ * around a node is loaded once where the node's triangles form a ring (one fan, closed, or
+ * open ones) of at most 8 neighbours and no two edges join the same nodes; a mesh with
+ * other nodes takes the edge lists. Uses no workspace and allocates nothing. */
 int fct_compute_w(fct_plan* plan, const double* uv, const double* helem, double* w,
                   void* stream);
 
@@ -360,10 +362,12 @@ int fct_tracer_ab(const double* values, const double* valuesold, double* ttf_ab,
  * reversed through the Thomas recurrence (ops.py:121-168) and g_w_i is returned; the
  * moving-level stencil (Z3d, zbar3) is supported. Z3d, zbar3, helem, hnode and
  * hnode_new are constants (no cotangent). The first call allocates the adjoint
- * workspace (15 node, 3 edge and 2 triangle arrays, twice that on meshes of up to
- * 131072 nodes; nl > 128: the flat kernels' 30, 11 and 4; and the first with w_i one to max_tracers more [nod2D][nl] arrays) and reads
- * mesh tables back once; it also uses the forward workspace as its tape. Later calls
- * allocate nothing. */
+ * workspace: 15 node, 3 edge and 2 triangle arrays, twice that on meshes of up to 131072
+ * nodes, and the first with w_i one [nod2D][nl] array per tracer slot of the plan; it also
+ * uses the forward workspace as its tape. Other kernels, with 30 node, 11 edge and 4
+ * triangle arrays (and two node arrays for w_i), allocated by the first call that takes
+ * them, serve nl > 128, meshes without rings (fct_compute_w) and, from 16384 nodes on,
+ * columns of up to 8 to 16 levels. Later calls allocate nothing. */
 typedef struct fct_adjoint_args {
     const double* const* g_T_new;  /* ntracers x [nod2D][nl], device */
     double* const* g_T;            /* out: ntracers x [nod2D][nl] */

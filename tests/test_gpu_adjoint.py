@@ -301,3 +301,32 @@ def test_adjoint_two_tracers_per_launch(level, nl, degree8, K, split, torch_dev)
             assert torch.equal(two[0][j], one[0][j]) and torch.equal(two[1][j], one[1][j]), j
         for i in range(2, len(one)):
             assert torch.equal(two[i], one[i]), i
+
+
+@pytest.mark.parametrize("level,nl,K,split,flat", [
+    (6, 8, 2, False, True), (6, 9, 2, False, False), (6, 12, 1, False, True),
+    (6, 13, 1, False, False), (6, 8, 1, True, True), (6, 9, 1, True, False),
+    (5, 6, 1, False, False)])
+def test_short_columns(level, nl, K, split, flat, torch_dev):
+    """On a mesh that fills the chip short columns take the flat kernels, either side of the
+    line and on a small mesh: the oracle's cotangents, and the workspace of that form."""
+    from fesom_jax_amd.inputs import make_case
+    from fesom_jax_amd.meshgen import icosahedral_mesh
+    from fesom_jax_amd.tracer_adv import get_plan
+    m = icosahedral_mesh(level, nl, seed=131, min_levels=3)
+    c = sharp_case(m, make_case(m, seed=132, dt=2700.0), 1.5)
+    Ts = [c["T"][0] * (1.0 + 0.1 * j) for j in range(K)]
+    Tos = [c["T_old"][0] + 0.2 * j for j in range(K)]
+    opts = {}
+    if split:
+        w_i, Z3d, zb3 = _split(m, c, 133)
+        opts = dict(w_i=w_i, Z3d=Z3d, zbar3=zb3)
+    gs = _cot(m, K, 134)
+    plan = get_plan(m, torch_dev)
+    before = plan.own_bytes()
+    got = _gpu(m, c, Ts, Tos, gs, torch_dev, **opts)
+    NL, DL, EL = m.nod2D * nl, m.edge2D * nl, m.elem2D * nl
+    # the flat kernels hold 11 edge arrays, the column kernels 6 (with 30 node and 4
+    # triangle arrays each)
+    assert (plan.own_bytes() - before > 8 * (34 * NL + 8 * DL + 4 * EL)) == flat
+    _compare(f"icosa{level} nl{nl}", got, _oracle(m, c, Ts, Tos, gs, **opts))
