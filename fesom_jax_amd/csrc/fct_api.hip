@@ -921,6 +921,15 @@ int fct_plan_destroy(fct_plan* p) {
 
 namespace {
 
+// A capture takes no allocation: a call that would make one then does without where the
+// other form can (both give the same bits).
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;      // (the null stream while another one is captured)
+}
+
 int check_args(const fct_plan* p, const fct_step_args* a) {
     if (!p || !a) return set_error(FCT_E_INVALID, "NULL plan or args");
     int cur = -1;
@@ -963,6 +972,23 @@ static int forward_phased(fct_plan* p, const fct_step_args* a, hipStream_t s) {
     return FCT_OK;
 }
 
+// With the split, one thread per level (the phased kernels) is faster than a wavefront per
+// column where the columns are short and the mesh fills the chip (us, phased, fused):
+//   one tracer:   28,673 x 8    90, 123;  x 16 123, 134;  x 20 172, 140;
+//                458,753 x 8   920, 1609; x 16 1775, 1817
+//   two tracers: 114,689 x 8   444, 472;  x 10 556, 514;  458,753 x 4 993, 1768
+// Where its workspace cannot be had (a captured first call, no memory) the fused path
+// gives the same bits.
+static bool split_by_phases(fct_plan* p, const fct_step_args* a, hipStream_t s) {
+    const DevMesh& m = p->m;
+    if (!a->w_i || (a->ntracers == 1 ? m.N < 16384 || m.L > 16 : m.N < 65536 || m.L > 8)) return false;
+    if (p->LO) return true;
+    if (capturing(s)) return false;
+    const bool ok = ensure_phased(p) == FCT_OK;
+    if (!ok) (void)hipGetLastError();
+    return ok;
+}
+
 int fct_forward_ex(fct_plan* p, const fct_step_args* a, int32_t path, void* stream) {
     int rc = check_args(p, a);
     if (rc) return rc;
@@ -972,7 +998,7 @@ int fct_forward_ex(fct_plan* p, const fct_step_args* a, int32_t path, void* stre
     if (path == FCT_PATH_FUSED && (!fused_ok || a->w_i))
         return set_error(FCT_E_UNSUPPORTED,
                          "fused path needs w_i == NULL, nl <= 128 and node degree <= 8");
-    if (path == FCT_PATH_PHASED || (path == FCT_PATH_AUTO && !fused_ok))
+    if (path == FCT_PATH_PHASED || (path == FCT_PATH_AUTO && (!fused_ok || split_by_phases(p, a, s))))
         return forward_phased(p, a, s);
     if (path != FCT_PATH_AUTO && path != FCT_PATH_FUSED)
         return set_error(FCT_E_INVALID, "unknown path %d", path);
@@ -1123,15 +1149,6 @@ int run_vdiff(const fct_plan* p, const fct_vdiff_args* a, int grid, double* scra
         if (rc) return rc;
     }
     return FCT_OK;
-}
-
-// A capture takes no allocation: a call that would make one then does without where the
-// other form can (both give the same bits).
-bool capturing(hipStream_t s) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
-    (void)hipGetLastError();
-    return true;      // (the null stream while another one is captured)
 }
 
 }  // namespace

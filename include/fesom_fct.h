@@ -104,7 +104,8 @@ enum {
 };
 
 enum {
-    FCT_PATH_AUTO = 0,    /* fused unless nl > 128 or node degree > 8               */
+    FCT_PATH_AUTO = 0,    /* fused unless nl > 128 or node degree > 8, or w_i is
+                             given on a large mesh of few levels                    */
     FCT_PATH_PHASED = 1,  /* one kernel per reference stage                         */
     FCT_PATH_FUSED = 2    /* edge pass + three node-column passes                   */
 };
@@ -162,7 +163,7 @@ const char* fct_last_error(void);
  * Replaces the per-call mesh handling of fesom_jax/tracer_adv.py:532-578 (the Mesh
  * pytree, fesom_jax/mesh.py:62-129). Allocates device memory: the topology and the
  * fused path's workspace here; the phased path's workspace on the first call that takes
- * that path (exch hook, or meshes the fused path does not support). */
+ * that path (exch hook, meshes the fused path does not support, w_i on short columns). */
 int fct_plan_create(const fct_mesh_desc* mesh, fct_plan** out);
 
 int fct_plan_get_info(const fct_plan* plan, fct_plan_info* info);
@@ -185,8 +186,11 @@ int fct_plan_set_tuning(fct_plan* plan, int32_t knob, int32_t value);
  *                           dt=dt, exch=None, Z3d, zbar3, w_i)[0]
  * (fesom_jax/tracer_adv.py:532-578). T_old_new is T itself and is not written.
  * Stream-ordered. On the fused path it allocates nothing; the first call that takes
- * the phased path (nl > 128 or node degree > 8) allocates 10 * nod2D * nl +
- * 2 * elem2D * nl + edge2D * nl doubles of workspace, later calls nothing. */
+ * the phased path (nl > 128 or node degree > 8; with w_i also one tracer on at least 16384
+ * nodes and at most 16 levels, or more on at least 65536 and at most 8) allocates
+ * 10 * nod2D * nl + 2 * elem2D * nl + edge2D * nl doubles of workspace, later calls
+ * nothing. In the w_i cases a first call under capture takes the fused path instead (the
+ * same bits). */
 int fct_forward(fct_plan* plan, const fct_step_args* args, void* stream);
 
 /* fct_forward with an explicit kernel path (FCT_PATH_*); both paths give the same

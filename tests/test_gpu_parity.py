@@ -607,3 +607,32 @@ def test_short_columns_share_a_wavefront(nl, K, torch_dev):
         assert np.array_equal(insts[0].T()[j].cpu().numpy(), want[j]), j
         assert np.array_equal(insts[1].T()[j].cpu().numpy(), want[j]), j
     batch.close()
+
+
+@pytest.mark.parametrize("level,nl,K,phased", [
+    (6, 16, 1, True), (6, 17, 1, False), (5, 16, 1, False), (6, 8, 2, False), (7, 8, 2, True),
+    (7, 9, 3, False)])
+def test_split_of_short_columns(level, nl, K, phased, torch_dev):
+    """Short columns with the implicit split on a large mesh take the phased kernels, which
+    then allocate their workspace: both sides of each line, bit for bit to the oracle."""
+    import torch
+    from fesom_jax_amd import tracer_adv
+    from fesom_jax_amd.inputs import make_case
+    from fesom_jax_amd.meshgen import icosahedral_mesh
+    m = icosahedral_mesh(level, nl, seed=141, min_levels=3)
+    c = sharp_case(m, make_case(m, seed=142, dt=2700.0), 1.5)
+    rng = np.random.default_rng(143)
+    im = m.node_iface_mask
+    w_i = np.where(im, 0.3 * np.abs(c["w_e"]).max() * rng.standard_normal(im.shape), 0.0)
+    Ts = [c["T"][0] * (1.0 + 0.1 * j) for j in range(K)]
+    Tos = [c["T_old"][0] + 0.2 * j for j in range(K)]
+    flow = [c[k] for k in ("uv", "w_e", "helem", "hnode", "hnode_new")]
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(torch_dev)
+    plan = tracer_adv.get_plan(m, torch_dev)
+    before = plan.own_bytes()
+    got = tracer_adv._run(m, *map(t, flow), [t(x) for x in Ts], [t(x) for x in Tos], c["dt"], None,
+                          None, None, t(w_i))
+    assert (plan.own_bytes() > before) == phased
+    for j in range(K):
+        want = O.advect_one_fct(m, *flow, Ts[j], Tos[j], dt=c["dt"], w_i=w_i)[0]
+        assert np.array_equal(got[j].cpu().numpy(), want), j
