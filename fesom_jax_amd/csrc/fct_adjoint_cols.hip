@@ -1024,13 +1024,14 @@ __global__ void __launch_bounds__(256) kc_add(size_t n, double* x, const double*
 
 constexpr int WPB = 4;
 
-// Meshes of at most this many nodes run two tracers per launch (workspace for both): one
-// tracer's column kernels leave wavefront slots of a small mesh's chip idle or end in a
-// mostly idle last round, and k_vimpl_reverse has one workgroup per CU or less (two steps
-// of the pi mesh 542 -> 508 us, icosa-6 x 70 with the split 1621 -> 1530). On larger meshes
-// the launches fill the chip, but short columns then share wavefronts (HALF_NODES), while
-// the second tracer's edge cotangents and workspace (15 node, 3 edge, 2 triangle arrays: at
-// most 4 GB here) cost about as much as they bring at nl = 70.
+// Meshes of at most this many nodes run two tracers per launch (workspace for both, if the
+// plan has two tracer slots): one tracer's column kernels leave wavefront slots of a small
+// mesh's chip idle or end in a mostly idle last round, and k_vimpl_reverse has one workgroup
+// per CU or less (two steps of the pi mesh 542 -> 508 us, icosa-6 x 70 with the split 1621 ->
+// 1530). Where one tracer's launches fill the chip the pair gains by short columns in halves
+// (HALF_NODES): icosa-7 x 47 3519 -> 3411, x 70 4337 -> 4316. Above the line, which keeps
+// the second set (15 node, 3 edge, 2 triangle arrays) below about 4 GB, every tracer is
+// reversed alone and no column shares a wavefront.
 constexpr int PAIR_NODES = 131072;
 // From this many nodes on, the launches of two tracers put both tracers of a short node
 // or edge column (31 levels and the bottom interface at most) into the halves of one
@@ -1084,12 +1085,15 @@ static size_t edge_stride(const DevMesh& m) { return even((size_t)m.D * m.L * 3)
 static size_t elem_stride(const DevMesh& m) { return (size_t)m.E * m.L * 2; }
 
 int adjoint_cols_tracers(const DevMesh& m) { return m.N <= PAIR_NODES ? 2 : 1; }
-// (two tracers: and the second one's w cotangent)
-size_t adjoint_cols_node(const DevMesh& m, int nt) {
-    return nt * node_stride(m) + (nt > 1 ? (size_t)m.N * m.L : 0);
+// (two tracers: and the second one's w cotangent; in one set, its w_i cotangent too)
+size_t adjoint_cols_node(const DevMesh& m, int nt, int sets) {
+    return sets * node_stride(m) + ((nt > 1) + (nt > sets)) * (size_t)m.N * m.L;
 }
-size_t adjoint_cols_edge(const DevMesh& m, int nt) { return nt * edge_stride(m); }
-size_t adjoint_cols_elem(const DevMesh& m, int nt) { return nt * elem_stride(m); }
+// (two tracers in one set: and the second one's vflux cotangent)
+size_t adjoint_cols_edge(const DevMesh& m, int nt, int sets) {
+    return sets * edge_stride(m) + (nt > sets) * (size_t)m.D * m.L;
+}
+size_t adjoint_cols_elem(const DevMesh& m, int sets) { return sets * elem_stride(m); }
 
 int launch_backward_cols(const DevMesh& m, const NodeTab& tab, const int2* ekr, const FusedTape& tp,
                          const AdjointCols& w, const FusedTuning& tune, const fct_step_args* f,
@@ -1114,10 +1118,15 @@ int launch_backward_cols(const DevMesh& m, const NodeTab& tab, const int2* ekr, 
     // Small meshes sum the even and the odd tracers' uv and w cotangents apart, whether a
     // launch takes two tracers or one (a plan with one slot): the bits do not depend on it.
     const bool pairs = w.tracers == 2 && f->ntracers >= 2;
-    double* vf[2] = {w.edge + 2 * DL, w.edge + 2 * DL + a.edge_stride};
-    double* gw[2] = {g_w, g_w ? w.node + 2 * a.node_stride : nullptr};
+    const bool own_set = w.sets == 2;      // the odd tracers' lie in the second set
+    double* more = w.node + w.sets * a.node_stride;
+    double* vf[2] = {w.edge + 2 * DL, w.edge + a.edge_stride + (own_set ? 2 * DL : 0)};
+    double* gw[2] = {g_w, g_w ? more : nullptr};
     double* gwi[2] = {nullptr, nullptr};
-    if (f->w_i) { gwi[0] = g_wi ? g_wi : own_wi; gwi[1] = own_wi + a.node_stride; }
+    if (f->w_i) {
+        gwi[0] = g_wi ? g_wi : own_wi;
+        gwi[1] = own_set ? own_wi + a.node_stride : more + NL;
+    }
     a.ud_off = w.ud_off; a.ud_ent = w.ud_ent; a.et_off = w.et_off; a.et_ent = w.et_ent;
     int rc;
     for (int j0 = 0; j0 < f->ntracers; j0 += tp.kw) {

@@ -418,11 +418,11 @@ int ensure_columns(fct_plan* p) {
     int rc;
     const DevMesh& m = p->m;
     AdjointCols& c = p->ac;
-    const int nt = c.tracers = adjoint_cols_tracers(m);
-    if ((rc = dev_alloc(p, &c.node, adjoint_cols_node(m, nt))) ||
-        (rc = dev_alloc(p, &c.edge_up, (size_t)m.D * (m.L <= 64 ? 1 : 2) * nt)) ||
-        (rc = dev_alloc(p, &c.edge, adjoint_cols_edge(m, nt))) ||
-        (rc = dev_alloc(p, &c.elem, adjoint_cols_elem(m, nt))) ||
+    const int nt = c.tracers = adjoint_cols_tracers(m), sets = c.sets = std::min(nt, p->kw);
+    if ((rc = dev_alloc(p, &c.node, adjoint_cols_node(m, nt, sets))) ||
+        (rc = dev_alloc(p, &c.edge_up, (size_t)m.D * (m.L <= 64 ? 1 : 2) * sets)) ||
+        (rc = dev_alloc(p, &c.edge, adjoint_cols_edge(m, nt, sets))) ||
+        (rc = dev_alloc(p, &c.elem, adjoint_cols_elem(m, sets))) ||
         (rc = upload_element_lists(p, &c.ud_off, &c.ud_ent, &c.et_off, &c.et_ent)))
         return rc;
     p->cols_ready = true;

@@ -247,20 +247,21 @@ struct FusedTape {
     double *vflux = nullptr, *LO = nullptr, *LOx = nullptr, *gnode = nullptr, *adfh = nullptr;
     double *pf = nullptr, *adfv = nullptr;
 };
-// Workspace of the column adjoint (fct_adjoint_cols.hip): the cotangents of one or two
-// tracers (adjoint_cols_tracers), in adjoint_cols_node(), ..._edge() and ..._elem()
-// doubles, the sign bits of the edges' flux (per tracer one word per 64 levels) and the
-// element-side lists.
+// Workspace of the column adjoint (fct_adjoint_cols.hip): the cotangents of one tracer per
+// set, `sets` of them (no more than the plan has tracer slots), in adjoint_cols_node(),
+// ..._edge() and ..._elem() doubles, the sign bits of the edges' flux (per set one word per
+// 64 levels) and the element-side lists. tracers (adjoint_cols_tracers): 2 where the even
+// and the odd tracers' uv and w cotangents are summed apart, whatever the sets.
 struct AdjointCols {
-    int tracers = 1;
+    int tracers = 1, sets = 1;
     double *node = nullptr, *edge = nullptr, *elem = nullptr;
     uint64_t* edge_up = nullptr;
     const int *ud_off = nullptr, *ud_ent = nullptr, *et_off = nullptr, *et_ent = nullptr;
 };
 int adjoint_cols_tracers(const DevMesh& m);
-size_t adjoint_cols_node(const DevMesh& m, int tracers);
-size_t adjoint_cols_edge(const DevMesh& m, int tracers);
-size_t adjoint_cols_elem(const DevMesh& m, int tracers);
+size_t adjoint_cols_node(const DevMesh& m, int tracers, int sets);
+size_t adjoint_cols_edge(const DevMesh& m, int tracers, int sets);
+size_t adjoint_cols_elem(const DevMesh& m, int sets);
 
 // Launch-shape knobs of the fused path (fct_plan_set_tuning / fct_batch_set_tuning);
 // results do not depend on them.

@@ -96,7 +96,7 @@ def estimate_work_bytes(mesh, K, adjoint):
         total += 16 * D + 8 * E + 64
         if L <= 16:
             # short columns: requests of one and of more tracers may take either form
-            total += 8 * (31 * NL + 6 * DL + 4 * EL) + 32 * D + 8 * E + 64
+            total += 8 * (17 * NL + 4 * DL + 2 * EL) + 24 * D + 8 * E + 64
     return int(total)
 
 

@@ -366,8 +366,8 @@ int fct_tracer_ab(const double* values, const double* valuesold, double* ttf_ab,
  * reversed through the Thomas recurrence (ops.py:121-168) and g_w_i is returned; the
  * moving-level stencil (Z3d, zbar3) is supported. Z3d, zbar3, helem, hnode and
  * hnode_new are constants (no cotangent). The first call allocates the adjoint
- * workspace: 15 node, 3 edge and 2 triangle arrays, twice that on meshes of up to 131072
- * nodes, and the first with w_i one [nod2D][nl] array per tracer slot of the plan; it also
+ * workspace: 15 node, 3 edge and 2 triangle arrays, on meshes of up to 131072 nodes twice
+ * that (a plan of one tracer slot: 17, 4 and 2), and the first with w_i one [nod2D][nl] array per tracer slot of the plan; it also
  * uses the forward workspace as its tape. Other kernels, with 30 node, 11 edge and 4
  * triangle arrays (and two node arrays for w_i), allocated by the first call that takes
  * them, serve nl > 128, meshes without rings (fct_compute_w) and, from 16384 nodes on,

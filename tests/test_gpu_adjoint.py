@@ -330,3 +330,37 @@ def test_short_columns(level, nl, K, split, flat, torch_dev):
     # triangle arrays each)
     assert (plan.own_bytes() - before > 8 * (34 * NL + 8 * DL + 4 * EL)) == flat
     _compare(f"icosa{level} nl{nl}", got, _oracle(m, c, Ts, Tos, gs, **opts))
+
+
+def test_workspace_of_one_slot(torch_dev):
+    """A plan with one tracer slot reverses no two tracers in one launch, and holds one set of
+    cotangents (and the three arrays in which odd tracers are summed apart); its results are
+    those of a plan with two sets, bit for bit, with and without the split."""
+    import torch
+    from fesom_jax_amd.adjoint import advect_fct_vjp
+    from fesom_jax_amd.inputs import make_case
+    from fesom_jax_amd.meshgen import icosahedral_mesh
+    from fesom_jax_amd.tracer_adv import FctPlan
+    m = icosahedral_mesh(4, 35, seed=151, degree8=10)
+    c = sharp_case(m, make_case(m, seed=152, dt=2700.0), 1.5)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(torch_dev)
+    Ts = [t(c["T"][0] * (1.0 + 0.1 * j)) for j in range(3)]
+    Tos = [t(c["T_old"][0] + 0.2 * j) for j in range(3)]
+    gs = [t(g) for g in _cot(m, 3, 153)]
+    w_i, Z3d, zb3 = _split(m, c, 154)
+    flow = [t(c[k]) for k in ("uv", "w_e", "helem", "hnode", "hnode_new")]
+    NL, DL, EL = m.nod2D * 35, m.edge2D * 35, m.elem2D * 35
+    lists = 24 * m.edge2D + 8 * m.elem2D + 64
+    outs = []
+    for slots in (1, 2):
+        plan = FctPlan(m, torch_dev, max_tracers=slots)
+        before = plan.own_bytes()
+        out = list(advect_fct_vjp(m, *flow, Ts, Tos, gs, dt=c["dt"], plan=plan))
+        grown = plan.own_bytes() - before
+        most = 8 * ((17 * NL + 4 * DL + 2 * EL) if slots == 1 else (31 * NL + 6 * DL + 4 * EL))
+        assert grown <= most + slots * (lists + 8 * m.edge2D), (slots, grown, most)
+        out += advect_fct_vjp(m, *flow, Ts, Tos, gs, dt=c["dt"], plan=plan, w_i=t(w_i), Z3d=t(Z3d),
+                              zbar3=t(zb3))
+        outs.append([x for o in out for x in (o if isinstance(o, list) else [o])])
+    for i, (x, y) in enumerate(zip(*outs)):
+        assert torch.equal(x, y), i
