@@ -9,14 +9,18 @@
 // C loop (for nz = nzmax-1 .. nzmin: w[nz] += w[nz+1]), run by one lane per column on
 // the columns staged in LDS.
 //
-// Two forms of the divergence, term by term the same arithmetic in the same order.
+// Three forms of the divergence, term by term the same arithmetic in the same order.
+// k_compute_w_tab (meshes whose nodes have rings) loads each of a node's triangles once:
+// icosa-8 x 70 478 us, 278 for the compulsory bytes at the rate of a copy; with (u, v,
+// helem) taken from LDS rows by slot and four columns summed per workgroup 890.
+// k_compute_w_vf (other meshes with node tables) takes the terms from the FCT's edge volume
+// flux, computed once per edge by kf_vflux: 869 us on that mesh (436 and 471), 1253 by
+// k_compute_w.
+//   term(e, k) = (v1 dx1 - u1 dy1) h1 - (v2 dx2 - u2 dy2) h2 = -vflux(e, k)
+// exactly: x - y = -(y - x) and (-x) h = -(x h) in IEEE arithmetic, and a masked triangle
+// gives +0 in both; a sum that starts at +0.0 absorbs the sign of a zero.
 // k_compute_w evaluates each (edge, side) from the edge's two triangles, so that a node
-// loads every triangle around it twice. k_compute_w_tab (meshes whose nodes have rings)
-// loads each of the node's triangles once. icosa-8 x 70: 869 us with the edge terms computed
-// once per edge into memory and gathered from there (edge flux 436, gather 471, both slots
-// of every column loaded), 478 here against 278 for the compulsory bytes at the rate of a
-// copy; with (u, v, helem) taken from LDS rows by slot and four columns summed per
-// workgroup 890.
+// loads every triangle around it twice.
 
 #include <hip/hip_runtime.h>
 
@@ -30,7 +34,7 @@ using gp = __attribute__((address_space(1))) T*;
 template <class T>
 __device__ __forceinline__ gp<T> glb(T* p) { return (gp<T>)p; }
 
-// stage 2 and 3 of both kernels for node n (valid: n < nod2D), whose divergence is div.
+// stage 2 and 3 of k_compute_w and k_compute_w_vf for node n (valid: n < nod2D), whose divergence is div.
 // Blocks are FCT_W_WPB wavefronts, one node each; every thread reaches the barriers.
 constexpr int FCT_W_WPB = 4;
 template <int NS>
@@ -184,6 +188,45 @@ __global__ void __launch_bounds__(256) k_compute_w_tab(DevMesh m, NodeTab tab, i
     }
 }
 
+// divergence from the edge volume flux (see the top of the file); the node's edge slots
+// come from the fused node table, in the same 2e+side order as the CSR list
+template <int NS, int DM>
+__global__ void __launch_bounds__(256) k_compute_w_vf(DevMesh m, NodeTab tab,
+                                                      const int2* ekr, const double* vflux,
+                                                      double* w_) {
+    const int lane = threadIdx.x & 63;
+    // the node index is wave-uniform: scalar registers, so the table loads are scalar
+    const int n0 = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+    const bool valid = n0 < m.N;
+    const int n = valid ? n0 : m.N - 1;
+    const int L = m.L;
+    const int cnt = ldc(tab.hdr, n).z & 0xff;
+    int code[DM];
+    int2 kr[DM];
+#pragma unroll
+    for (int q = 0; q < DM; ++q) {
+        code[q] = ldc(tab.edge, (size_t)n * DM + q).x;
+        kr[q] = ldc(ekr, code[q] >> 1);
+    }
+    double div[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        const int k = lane + 64 * s;
+        const int kc = k < L ? k : L - 1;
+        double vf[DM];
+#pragma unroll
+        for (int q = 0; q < DM; ++q) vf[q] = G(vflux)[(size_t)(code[q] >> 1) * L + kc];
+        double d = 0.0;
+#pragma unroll
+        for (int q = 0; q < DM; ++q) {
+            const bool use = q < cnt && k >= kr[q].x && k < kr[q].y;
+            d = d + (use ? ((code[q] & 1) ? vf[q] : -vf[q]) : 0.0);
+        }
+        div[s] = d;
+    }
+    finish_w<NS>(m, n, valid, lane, div, w_);
+}
+
 template <int NS>
 __global__ void __launch_bounds__(256) k_compute_w(DevMesh m, const double* uv_,
                                                    const double* helem_, double* w_) {
@@ -246,6 +289,18 @@ int launch_compute_w(const DevMesh& m, const double* uv, const double* helem, do
     else
         return set_error(FCT_E_UNSUPPORTED, "compute_w supports nl <= 128 (got %d)", m.L);
     return check_launch("k_compute_w");
+}
+
+int launch_compute_w_vf(const DevMesh& m, const NodeTab& tab, const int2* ekr,
+                        const double* vflux, double* w, hipStream_t s) {
+    if (m.N == 0) return FCT_OK;
+    const int wpb = FCT_W_WPB;
+    const dim3 grid((m.N + wpb - 1) / wpb), block(64 * wpb);
+    if (tab.dm == 6 && m.L <= 64) k_compute_w_vf<1, 6><<<grid, block, 0, s>>>(m, tab, ekr, vflux, w);
+    else if (tab.dm == 6) k_compute_w_vf<2, 6><<<grid, block, 0, s>>>(m, tab, ekr, vflux, w);
+    else if (m.L <= 64) k_compute_w_vf<1, 8><<<grid, block, 0, s>>>(m, tab, ekr, vflux, w);
+    else k_compute_w_vf<2, 8><<<grid, block, 0, s>>>(m, tab, ekr, vflux, w);
+    return check_launch("k_compute_w_vf");
 }
 
 int launch_compute_w_tab(const DevMesh& m, const NodeTab& tab, int remap, const double* uv,

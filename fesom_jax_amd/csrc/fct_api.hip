@@ -270,9 +270,10 @@ bool fused_mesh_ok(const fct_mesh_desc* d, const std::vector<int>& eoff,
 
 // Ring of node n (NodeTab::ring): from its table edges `es` (de of them; .x code, .y
 // neighbour, .w >> 16 the vertex slots of element slot q), its ne elements `els` and their
-// layer ranges (es[q].w, low 16 bits). False if the fans do not fit dm slots, or if an edge's
-// triangles are not the two beside its slot.
-bool node_ring(const fct_mesh_desc* d, int dm, int de, int ne, const int4* es, const int* els, int4* r) {
+// layer ranges (es[q].w, low 16 bits). False if the fans do not fit dm slots; `flux` turns
+// false if an edge's triangles are not the two beside its slot.
+bool node_ring(const fct_mesh_desc* d, int dm, int de, int ne, const int4* es, const int* els, int4* r,
+               bool& flux) {
     int nb[8][2], el[8][2], cnt[8] = {};      // per slot: the slots its triangles join it to
     for (int q = 0; q < ne; ++q) {
         const unsigned w = (unsigned)es[q].w;
@@ -333,7 +334,7 @@ bool node_ring(const fct_mesh_desc* d, int dm, int de, int ne, const int4* es, c
         const int before = prev >= 0 ? els[prev] : -1, behind = join[i] >= 0 ? els[join[i]] : -1;
         const int32_t* et = d->edge_tri + 2 * (size_t)(t.x >> 1);
         const bool first_prev = before == et[0] && behind == et[1];
-        if (!first_prev && !(before == et[1] && behind == et[0])) return false;
+        flux = flux && (first_prev || (before == et[1] && behind == et[0]));
         r[i] = make_int4(t.y, join[i] >= 0 ? els[join[i]] : (ne ? els[0] : 0), t.x,
                          (join[i] >= 0 ? range(join[i]) : 0) | (slot[i] << 16) |
                              (first_prev ? FCT_RING_PREV : 0));
@@ -608,7 +609,7 @@ int fct_plan_create(const fct_mesh_desc* d, fct_plan** out) {
     std::vector<int4> h_thdr;
     std::vector<int4> h_tedge, h_telem;
     std::vector<int4> h_ring;
-    bool ring_ok = true;
+    bool ring_ok = true, ring_flux = true;
     bool vertex_missing = false;   // an element vertex that is not an edge neighbour
     if (dm) {
         // levels at which the adf_h pass reads a node's averaged gradient gnode: the wet
@@ -692,7 +693,7 @@ int fct_plan_create(const fct_mesh_desc* d, fct_plan** out) {
                 h_telem[(size_t)n * dm + q] = h_telem[(size_t)n * dm];
             ring_ok = ring_ok && !vertex_missing &&
                       node_ring(d, dm, de, ne, &h_tedge[(size_t)n * dm], &h_ncsr[h_noff[n]],
-                                &h_ring[(size_t)n * dm]);
+                                &h_ring[(size_t)n * dm], ring_flux);
         }
         if (vertex_missing) dm = 0;   // the fused kernels read element vertices by slot
     }
@@ -845,6 +846,7 @@ int fct_plan_create(const fct_mesh_desc* d, fct_plan** out) {
         free_plan(p);
         return rc;
     }
+    p->tab.ring_flux = p->tab.ring && ring_flux;
     // everything allocated so far is the mesh's tables; what follows is the plan's own
     p->tables = new (std::nothrow) TableSet();
     if (!p->tables) {
@@ -1078,8 +1080,13 @@ int fct_compute_w(fct_plan* p, const double* uv, const double* helem, double* w,
         return set_error(FCT_E_INVALID, "current device %d is not the plan's device %d", cur,
                          p->device);
     const hipStream_t s = (hipStream_t)stream;
-    if (p->tune.w_vflux && p->tab.ring && p->m.L <= 128)
+    if (p->tune.w_vflux && p->tab.ring_flux && p->m.L <= 128)
         return launch_compute_w_tab(p->m, p->tab, p->tune.remap(), uv, helem, w, s);
+    if (p->tune.w_vflux && p->tab.dm && p->m.L <= 128) {
+        // edge terms once per edge into the plan's vflux workspace, then summed per node
+        int rc = launch_vflux_fused(p->m, p->tab, p->ekr, uv, helem, p->tune, p->vflux, s);
+        return rc ? rc : launch_compute_w_vf(p->m, p->tab, p->ekr, p->vflux, w, s);
+    }
     return launch_compute_w(p->m, uv, helem, w, s);
 }
 

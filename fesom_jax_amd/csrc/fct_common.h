@@ -102,6 +102,9 @@ struct NodeTab {
     // its last triangle there (FCT_RING_DUP, edge code -1, range 0). NULL if a node's
     // triangles form no such ring.
     const int4* ring = nullptr;
+    // whether every edge's triangles are the two beside its slot (not where two edges join
+    // the same nodes), so that the edges' fluxes can be formed from the ring
+    bool ring_flux = false;
     // Node list of the passes: the nodes whose wet layers end above level 64 (`nshallow` of
     // them; for nl <= 64 all), in visit order, then the others; the passes take each set
     // in a launch of its own, the first with one 64-level slot per wavefront and fewer
@@ -374,8 +377,15 @@ int launch_ice_fct(const DevMesh& m, const IceCall& c, double* work, const doubl
                    void* slots, hipStream_t s);
 
 // Vertical velocity from continuity (fct_ale.hip).
+// over the rings (tab.ring_flux), or, for other meshes with node tables, the FCT's edge volume
+// flux alone (kf_vflux) into vflux [D][L] and the divergence from that; else per node from
+// the edge lists
 int launch_compute_w_tab(const DevMesh& m, const NodeTab& tab, int remap, const double* uv,
                          const double* helem, double* w, hipStream_t s);
+int launch_vflux_fused(const DevMesh& m, const NodeTab& tab, const int2* ekr, const double* uv,
+                       const double* helem, const FusedTuning& t, double* vflux, hipStream_t s);
+int launch_compute_w_vf(const DevMesh& m, const NodeTab& tab, const int2* ekr,
+                        const double* vflux, double* w, hipStream_t s);
 int launch_compute_w(const DevMesh& m, const double* uv, const double* helem, double* w,
                      hipStream_t s);
 

@@ -1937,13 +1937,26 @@ int launch_tape(const DevMesh& m, const NodeTab& tab, const int2* ekr, const fct
                      : launch_tape_t<2, 8>(fa, a, j0, K, tune, tp, s);
 }
 
+int launch_vflux_fused(const DevMesh& m, const NodeTab& tab, const int2* ekr, const double* uv,
+                       const double* helem, const FusedTuning& tune, double* vflux,
+                       hipStream_t s) {
+    if (!tuning_ok(tune)) return set_error(FCT_E_INVALID, "bad launch-shape knobs");
+    if (!m.D) return FCT_OK;
+    FusedArgs fa{};
+    fa.m = m; fa.tab = tab; fa.ekr = ekr; fa.uv = uv; fa.helem = helem; fa.vflux = vflux;
+    fa.remap = tune.remap(); fa.K = 1;
+    if (m.L <= 64) launch_single<1, 8>(fa, tune, s, 0);      // (the edge pass reads no node table)
+    else launch_single<2, 8>(fa, tune, s, 0);
+    return check_launch("kf_vflux");
+}
+
 template <int NS, int DM>
 static int launch_upwind_t(FusedArgs& fa, const fct_step_args* a, const FusedTuning& t,
                            hipStream_t s) {
     const DevMesh& m = fa.m;
     fa.K = 1;
     // (meshes with a node whose triangles make no ring: fluxes once per edge into memory)
-    if (m.D && !fa.tab.ring) launch_single<NS, DM>(fa, t, s, 0);
+    if (m.D && !fa.tab.ring_flux) launch_single<NS, DM>(fa, t, s, 0);
     int rc = check_launch("kf_vflux");
     if (rc) return rc;
     for (int j0 = 0; j0 < a->ntracers; j0 += FCT_KCHUNK) {
@@ -1953,7 +1966,7 @@ static int launch_upwind_t(FusedArgs& fa, const fct_step_args* a, const FusedTun
             const int jj = j0 + (j < K ? j : 0);
             fa.T[j] = a->T[jj]; fa.Told[j] = a->T_old[jj]; fa.Tnew[j] = a->T_new[jj];
         }
-        if (fa.tab.ring)
+        if (fa.tab.ring_flux)
             hipLaunchKernelGGL((kf_upwind_ring<NS, DM>), dim3(blocks_for(m.N, t.wpb)), dim3(64 * t.wpb), 0, s, fa);
         else
             hipLaunchKernelGGL((kf_upwind<NS, DM>), dim3(blocks_for(node_waves(m.N, K), t.wpb)), dim3(64 * t.wpb), 0, s, fa);

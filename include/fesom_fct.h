@@ -240,8 +240,10 @@ int fct_ice_fct_solve(fct_plan* plan, const fct_ice_args* args, void* stream);
  * the interface area; zero outside each node's interfaces [nzmin, nzmax]. uv is
  * [elem2D][nl][2], helem [elem2D][nl], w [nod2D][nl] (device). nl <= 128. Each triangle
  * around a node is loaded once where the node's triangles form a ring (one fan, closed, or
- * open ones) of at most 8 neighbours and no two edges join the same nodes; a mesh with
- * other nodes takes the edge lists. Uses no workspace and allocates nothing. */
+ * open ones) of at most 8 neighbours and no two edges join the same nodes; such a call
+ * uses no workspace. On a mesh with a node beyond that it uses the plan's edge-flux
+ * workspace, as fct_forward does (calls on one plan race if they overlap), or, with more than
+ * 8 neighbours, the edge lists. No allocation. */
 int fct_compute_w(fct_plan* plan, const double* uv, const double* helem, double* w,
                   void* stream);
 
