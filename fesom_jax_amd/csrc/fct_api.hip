@@ -903,7 +903,8 @@ int fct_plan_get_info(const fct_plan* p, fct_plan_info* info) {
     info->table_bytes = p->tables ? p->tables->bytes : 0;
     info->table_id = (uint64_t)(uintptr_t)p->tables;
     info->patch_order = p->tab.vorder != nullptr;
-    info->reserved = 0;
+    info->adfh_segments =
+        p->tune.adfh_kc ? adfh_segments(p->tab.ep.np, p->m.L, p->tune.adfh_kc) : 0;
     info->device = p->device;
     info->paths = FCT_PATH_BIT_PHASED | (p->tab.dm > 0 ? FCT_PATH_BIT_FUSED : 0);
     return FCT_OK;

@@ -127,6 +127,12 @@ class FctPlan:
         vertical-flux passes visit it in the edge patches' breadth-first order."""
         return bool(self._info().patch_order)
 
+    @property
+    def adfh_segments(self) -> int:
+        """Workgroups per edge patch in a step's adf_h pass under the plan's tuning; 0 where
+        the pass runs one wavefront per edge instead."""
+        return int(self._info().adfh_segments)
+
     def close(self):
         self._finalizer()
 

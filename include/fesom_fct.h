@@ -146,7 +146,8 @@ typedef struct fct_plan_info {
     int32_t patch_order;       /* 1: the caller's numbering is not local, so the node
                                   passes and the vertical-flux pass visit nodes and edges
                                   in the edge patches' breadth-first order; 0: id order */
-    int32_t reserved;
+    int32_t adfh_segments;     /* workgroups per edge patch in a step's adf_h pass under the
+                                  plan's tuning; 0: one wavefront per edge instead */
 } fct_plan_info;
 
 #define FCT_PATH_BIT_PHASED 1

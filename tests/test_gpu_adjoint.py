@@ -364,3 +364,42 @@ def test_workspace_of_one_slot(torch_dev):
         outs.append([x for o in out for x in (o if isinstance(o, list) else [o])])
     for i, (x, y) in enumerate(zip(*outs)):
         assert torch.equal(x, y), i
+
+
+@pytest.mark.parametrize("K,split", [(2, False), (3, True)])
+def test_backward_of_large_meshes(K, split, torch_dev):
+    """Above 131072 nodes every tracer is reversed alone and the uv, w and w_i cotangents of
+    all go into one array each: g_T and g_T_old are those of single-tracer calls bit for
+    bit, the others their sums. (A sum of K + 3 K terms of the fields' size, in another
+    order: well within 1e-12 of the largest.)"""
+    import torch
+    from fesom_jax_amd.adjoint import advect_fct_vjp
+    from fesom_jax_amd.inputs import make_case
+    from fesom_jax_amd.meshgen import icosahedral_mesh
+    from fesom_jax_amd.tracer_adv import get_plan
+    m = icosahedral_mesh(7, 18, seed=171, land_fraction=0.1)
+    assert m.nod2D > 131072
+    c = sharp_case(m, make_case(m, seed=172, dt=2700.0), 1.5)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(torch_dev)
+    Ts = [t(c["T"][0] * (1.0 + 0.1 * j)) for j in range(K)]
+    Tos = [t(c["T_old"][0] + 0.2 * j) for j in range(K)]
+    gs = [t(g) for g in _cot(m, K, 173)]
+    opts = {}
+    if split:
+        w_i, Z3d, zb3 = _split(m, c, 174)
+        opts = dict(w_i=t(w_i), Z3d=t(Z3d), zbar3=t(zb3))
+    flow = [t(c[k]) for k in ("uv", "w_e", "helem", "hnode", "hnode_new")]
+    run = lambda js: advect_fct_vjp(m, *flow, [Ts[j] for j in js], [Tos[j] for j in js],
+                                    [gs[j] for j in js], dt=c["dt"], **opts)
+    print(f"[adjoint] N={m.nod2D} K={K} split={split}", flush=True)
+    before = get_plan(m, torch_dev).own_bytes()
+    both = run(range(K))
+    NL, DL, EL = m.nod2D * 18, m.edge2D * 18, m.elem2D * 18
+    # the column kernels' one set (15, 3 and 2 arrays, and the split's), not the flat ones'
+    assert get_plan(m, torch_dev).own_bytes() - before < 8 * (20 * NL + 5 * DL + 3 * EL)
+    alone = [run([j]) for j in range(K)]
+    for j in range(K):
+        assert torch.equal(both[0][j], alone[j][0][0]) and torch.equal(both[1][j], alone[j][1][0]), j
+    for i in range(2, len(both)):
+        want = sum(a[i] for a in alone)
+        assert (both[i] - want).abs().max() <= 1e-12 * want.abs().max(), i

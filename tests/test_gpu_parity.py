@@ -636,3 +636,58 @@ def test_split_of_short_columns(level, nl, K, phased, torch_dev):
     for j in range(K):
         want = O.advect_one_fct(m, *flow, Ts[j], Tos[j], dt=c["dt"], w_i=w_i)[0]
         assert np.array_equal(got[j].cpu().numpy(), want), j
+
+
+@pytest.mark.parametrize("scattered", [False, True])
+def test_adfh_patch_forms(scattered, torch_dev):
+    """The edge-patch form of the adf_h pass, on a mesh with enough patches that it runs:
+    both chunk sizes, one, two and four threads per edge, one to three tracers, in local
+    and in scattered numbering with nodes of degree 8, alone and in a batch; bit for bit to
+    the wavefront-per-edge form, and that to the oracle."""
+    from fesom_jax_amd import _lib
+    from fesom_jax_amd.batch import FctBatch, Instance
+    from fesom_jax_amd.inputs import make_case
+    from fesom_jax_amd.meshgen import icosahedral_mesh, shuffled
+    from fesom_jax_amd.tracer_adv import FctPlan, get_plan
+    m = icosahedral_mesh(5, 70, seed=161, degree8=40 if scattered else 0)
+    if scattered:
+        m = shuffled(m, 162)
+    c = make_case(m, seed=163, dt=2700.0)
+    sharp = sharp_case(m, c, 2.0)
+    sharp["T"] = [sharp["T"][0], c["T"][0], c["T"][1]]
+    sharp["T_old"] = [sharp["T_old"][0], c["T"][0], c["T"][1]]
+    plan = get_plan(m, torch_dev)
+    assert plan.patch_order == scattered
+
+    def tune(chunk, threads):
+        for k, v in (("ADFH_CHUNK", chunk), ("ADFH_THREADS", threads)):
+            _lib.check(plan.lib.fct_plan_set_tuning(plan.ptr, getattr(_lib, "FCT_TUNE_" + k), v),
+                       "tuning")
+
+    def cut(K):
+        return dict(sharp, T=sharp["T"][:K], T_old=sharp["T_old"][:K])
+
+    tune(0, 1)
+    assert plan.adfh_segments == 0
+    ref = _gpu_step(m, cut(3), torch_dev, path="fused")
+    for j in range(3):
+        assert np.array_equal(ref[j], _oracle(m, sharp, j)), j
+    for chunk in (4, 8):
+        for threads in (1, 2, 4):
+            tune(chunk, threads)
+            assert plan.adfh_segments > 0
+            for K in (1, 2, 3):
+                got = _gpu_step(m, cut(K), torch_dev, path="fused")
+                for j in range(K):
+                    assert np.array_equal(got[j], ref[j]), (chunk, threads, K, j)
+            insts = [Instance.from_case(m, cut(K), torch_dev, plan=FctPlan(m, torch_dev, max_tracers=3,
+                                                                          share=plan)) for K in (1, 3)]
+            batch = FctBatch(insts)
+            batch.set_tuning(_lib.FCT_TUNE_ADFH_CHUNK, chunk)
+            batch.set_tuning(_lib.FCT_TUNE_ADFH_THREADS, threads)
+            batch.step()
+            for inst in insts:
+                for j, x in enumerate(inst.T()):
+                    assert np.array_equal(x.cpu().numpy(), ref[j]), ("batch", chunk, threads, j)
+            batch.close()
+    tune(8, 1)
