@@ -1607,10 +1607,8 @@ FCT_NODE_KERNELS(pass2, 5)
 FCT_NODE_KERNELS(pass3, 6)
 #undef FCT_NODE_KERNELS
 
-// Passes 2 and 3 over `count` nodes of the node list from `first`, all of whose wet
-// layers fit NSB slots: shallow columns (NSB = 1) run with fewer registers per
-// wavefront and so more wavefronts per SIMD than the two-slot body needs.
-// (occupancy on 8-slot tables, 1 % of the nodes at 8: one slot 225 us at three wavefronts,
+// The upwind step over the rings, one wavefront per node for all tracers, a 64-level slot at
+// a time (occupancy on 8-slot tables, 1 % of the nodes at 8: one slot 225 us at three wavefronts,
 // 235 at four, with spills; two slots 324 and 270)
 template <int NS, int DM>
 __global__ void FCT_OCC(DM == 8 && NS == 1 ? 3 : 4) kf_upwind_ring(FusedArgs a) {
@@ -1632,6 +1630,9 @@ __global__ void FCT_OCC(DM == 8 && NS == 1 ? 3 : 4) kf_upwind_ring(FusedArgs a) 
     }
 }
 
+// Passes 2 and 3 over `count` nodes of the node list from `first`, all of whose wet
+// layers fit NSB slots: shallow columns (NSB = 1) run with fewer registers per
+// wavefront and so more wavefronts per SIMD than the two-slot body needs.
 #define FCT_LIST_KERNELS(PASS, OCC1, OCC2)                                                  template <int NSB, int DM>                                                              __global__ void FCT_OCC(DM == 6 ? (NSB == 1 ? OCC1 : OCC2) : 4)                              kl_##PASS(FusedArgs a, int first, int count) {                                          int w;                                                                                  if (!single_wave((int64_t)count * a.K, a.remap, w)) return;                              const int t = w / a.K;                                                                  const int n = ldc(a.tab.nlist, (size_t)first + t);                                      const int4 hd = ldc(a.tab.hdr, n);                                                      PASS##_body<NSB, DM>(a, n, w - t * a.K, make_int2(hd.x, hd.y),                                               make_int2(hd.z & 0xff, hd.w));                                 }
 
 FCT_LIST_KERNELS(pass2, 7, 4)

@@ -145,9 +145,11 @@ __device__ __forceinline__ double2 ldv(const double2* p, size_t i) {
 __device__ __forceinline__ double4 ldv(const double4* p, size_t i) {
     return __builtin_bit_cast(double4, ((gptr<const fct_dv4>)p)[i]);
 }
-// Loads at wave-uniform addresses of data that no kernel writes (mesh tables), through
-// the constant address space so that the compiler issues scalar loads: they go through
-// the scalar cache and leave the vector memory pipeline to the column gathers.
+// Loads at wave-uniform addresses of data that the same launch does not write (mesh tables;
+// the adjoint's edge signs, from an earlier launch on the stream: the scalar cache is
+// invalidated where a kernel starts), through the constant address space so that the compiler
+// issues scalar loads: they go through the scalar cache and leave the vector memory pipeline
+// to the column gathers.
 template <class T>
 using cptr = __attribute__((address_space(4))) const T*;
 __device__ __forceinline__ int ldc(const int* p, size_t i) { return ((cptr<int>)p)[i]; }

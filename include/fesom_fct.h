@@ -118,17 +118,22 @@ enum {
     FCT_TUNE_ADFH_EDGES = 4,        /* edges per wavefront in the adf_h pass: 1 or 2 (2)   */
     FCT_TUNE_XCD_CHUNK = 5,         /* workgroups per range of one XCD under FCT_TUNE_XCD:
                                        0 = one range per XCD, else 1..2^20 (default 8)    */
-    FCT_TUNE_W_EDGE_FLUX = 6,       /* fct_compute_w: 1 = over the node tables, each
-                                       triangle around a node loaded once, 0 = over the edge
-                                       lists; same bits either way (default 1)            */
-    FCT_TUNE_PAIR_TRACERS = 7,      /* nl > 64, two tracers, node degree <= 6: 1 = the
-                                       shallow columns' node passes take both tracers
-                                       in one wavefront, 0 = one wavefront per tracer
+    FCT_TUNE_W_EDGE_FLUX = 6,       /* fct_compute_w on meshes with node tables: 1 = over the
+                                       nodes' rings, each triangle loaded once, or, where
+                                       there are none, from the step's edge flux pass, 0 =
+                                       over the edge lists; same bits (default 1)         */
+    FCT_TUNE_PAIR_TRACERS = 7,      /* two tracers or more: 1 = the node passes take two
+                                       tracers in one wavefront on columns that end at or
+                                       above level 64 (nodes with more than 6 neighbours,
+                                       and, in a batch or below 16384 nodes, all nodes of
+                                       a mesh that has such: one), 0 = one each
                                        (default 1)                                         */
     FCT_TUNE_ADFH_CHUNK = 8,        /* adf_h pass: 4 or 8 = edge-patch kernel (edge
                                        patches with their node columns staged in LDS,
-                                       that many levels at a time), 0 = one wavefront
-                                       per edge column; same bits (default 8)             */
+                                       that many levels at a time) where the launch, in a
+                                       batch the group, has 256 chunks of them or more,
+                                       0 = one wavefront per edge column; same bits
+                                       (default 8)                                        */
     FCT_TUNE_ADFH_THREADS = 9       /* edge-patch adf_h kernel: threads per edge, 1, 2 or
                                        4, splitting each chunk's levels (default 1)       */
 };
