@@ -68,6 +68,8 @@ struct fct_plan {
     double *vflux = nullptr, *LO = nullptr, *trxy = nullptr, *gnode = nullptr;
     double *adfh = nullptr, *adfv = nullptr, *tvmax = nullptr, *tvmin = nullptr;
     double *fplus = nullptr, *fminus = nullptr, *pf = nullptr, *mf = nullptr;
+    // no memory for the phased path, or the backward's flat kernels, where others serve
+    bool no_phased = false, no_flat = false;
     // fused path: per-edge wet level range and per-tracer workspace (kw tracers)
     const int2* ekr = nullptr;
     int kw = 0;
@@ -76,8 +78,8 @@ struct fct_plan {
     // fpf holds the limiter factors as (plus, minus) pairs; fadfv the vertical
     // antidiffusive flux pass 2 computes and pass 3 reads
     double *fLO = nullptr, *fgnode = nullptr, *fadfh = nullptr, *fpf = nullptr, *fadfv = nullptr;
-    // adjoint workspaces of the flat and of the column kernels, each allocated on the first
-    // fct_backward that takes them (adjoint_by_columns)
+    // adjoint workspaces of the flat and of the column kernels (nl <= 128, meshes with
+    // rings), each allocated on the first fct_backward that takes them (adjoint_by_columns)
     bool flat_ready = false, cols_ready = false;
     AdjointWork aw{};
     AdjointCols ac{};
@@ -86,6 +88,7 @@ struct fct_plan {
     // implicit vertical diffusion scratch (allocated on the first call)
     double* vd_scratch = nullptr;
     int vd_grid = 0;
+    bool no_vd_scratch = false;   // no memory for it where LDS serves
     // sea-ice FCT workspace and element table (allocated on the first call)
     double* ice_work = nullptr;
     double* ice_tab = nullptr;
@@ -342,6 +345,23 @@ bool node_ring(const fct_mesh_desc* d, int dm, int de, int ne, const int4* es, c
     return true;
 }
 
+// The workspace of a form that another one can stand in for. Without the memory: gives back
+// what came, and does not ask again on every call.
+bool ensure_or_give_up(fct_plan* p, int (*ensure)(fct_plan*), bool& given_up) {
+    if (given_up) return false;
+    const size_t held = p->allocs.size();
+    const int64_t bytes = p->bytes;
+    double* const LO = p->LO;             // (the phased workspace counts as held by it)
+    if (ensure(p) == FCT_OK) return true;
+    (void)hipGetLastError();
+    for (size_t i = held; i < p->allocs.size(); ++i) (void)hipFree(p->allocs[i]);
+    p->allocs.resize(held);
+    p->bytes = bytes;
+    p->LO = LO;
+    given_up = true;
+    return false;
+}
+
 // Workspace of the phased path, allocated on the first call that takes it (the fused
 // path, which batches and most callers use, never needs it).
 int ensure_phased(fct_plan* p) {
@@ -398,7 +418,7 @@ int upload_element_lists(fct_plan* p, const int** ud_off, const int** ud_list, c
     return FCT_OK;
 }
 
-// Whether the backward of K tracers takes the column kernels. They cost a wavefront per
+// Whether the backward of K tracers is better by the column kernels. They cost a wavefront per
 // column whatever its levels, so on a mesh that fills the chip short columns are faster one
 // thread per level (us, flat kernels then column kernels):
 //   one tracer:   28,673 x 12   323,  373;  x 16  373,  378;  114,689 x 16 1396, 1506;
@@ -408,7 +428,6 @@ int upload_element_lists(fct_plan* p, const int** ud_off, const int** ud_list, c
 //   under the split, one tracer: 114,689 x 8 949, 1472;  x 12 1527, 1582; x 16 2158, 1657
 bool adjoint_by_columns(const fct_plan* p, int K, bool split) {
     const DevMesh& m = p->m;
-    if (!p->tab.ring || m.L > 128) return false;
     if (m.N < 16384) return true;
     return m.L > (split ? 8 : (m.N < 65536 ? 8 : 12) + (K == 1 ? 4 : 0));
 }
@@ -985,11 +1004,7 @@ static int forward_phased(fct_plan* p, const fct_step_args* a, hipStream_t s) {
 static bool split_by_phases(fct_plan* p, const fct_step_args* a, hipStream_t s) {
     const DevMesh& m = p->m;
     if (!a->w_i || (a->ntracers == 1 ? m.N < 16384 || m.L > 16 : m.N < 65536 || m.L > 8)) return false;
-    if (p->LO) return true;
-    if (capturing(s)) return false;
-    const bool ok = ensure_phased(p) == FCT_OK;
-    if (!ok) (void)hipGetLastError();
-    return ok;
+    return p->LO || (!capturing(s) && ensure_or_give_up(p, ensure_phased, p->no_phased));
 }
 
 int fct_forward_ex(fct_plan* p, const fct_step_args* a, int32_t path, void* stream) {
@@ -1167,14 +1182,18 @@ int fct_impl_vert_diff(fct_plan* p, const fct_vdiff_args* a, void* stream) {
     int rc = check_vdiff(p, a);
     if (rc) return rc;
     const bool fits = vdiff_fits(p->m.L);
-    if (!p->vd_scratch && vdiff_wants_scratch(p, a) && !(fits && capturing((hipStream_t)stream))) {
+    if (!p->vd_scratch && vdiff_wants_scratch(p, a) &&
+        !(fits && (p->no_vd_scratch || capturing((hipStream_t)stream)))) {
         int cus = 0;
         HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device));
         int grid = 0;
         if ((rc = vdiff_max_grid(cus, &grid))) return rc;
         rc = dev_alloc(p, &p->vd_scratch, vdiff_scratch_doubles(p->m.L, grid));
         if (rc && !fits) return rc;
-        if (rc) (void)hipGetLastError();
+        if (rc) {
+            (void)hipGetLastError();
+            p->no_vd_scratch = true;
+        }
         p->vd_grid = grid;
     }
     return run_vdiff(p, a, p->vd_grid, p->vd_scratch, (hipStream_t)stream);
@@ -1597,7 +1616,12 @@ int fct_backward(fct_plan* p, const fct_step_args* a, const fct_adjoint_args* g,
             return set_error(FCT_E_INVALID, "tracer %d has a NULL field", j);
     int rc;
     const size_t NL = (size_t)p->m.N * p->m.L;
-    if (adjoint_by_columns(p, a->ntracers, a->w_i != nullptr)) {
+    const bool columns = p->tab.ring && p->m.L <= 128;
+    const auto have_flat = [&] {
+        return p->flat_ready || (!capturing((hipStream_t)stream) &&
+                                 ensure_or_give_up(p, ensure_flat, p->no_flat));
+    };
+    if (columns && (adjoint_by_columns(p, a->ntracers, a->w_i != nullptr) || !have_flat())) {
         if ((rc = ensure_columns(p))) return rc;
         if (a->w_i && !p->adj_LOx && (rc = dev_alloc(p, &p->adj_LOx, NL * p->kw))) return rc;
         FusedTape t;
