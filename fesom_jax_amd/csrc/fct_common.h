@@ -87,6 +87,8 @@ constexpr int FCT_RING_PREV = 1 << 20, FCT_RING_DUP = 1 << 21;
 // Per-node stencil table of the fused path (dm slots per node).
 struct NodeTab {
     int dm = 0;               // slots per node (6 or 8); 0 = mesh not supported
+    bool ring_flux = false;   // `ring` holds every edge's own triangles beside its slot (not
+                              //  where two edges join the same nodes): fluxes from it
     const int4* hdr;          // [N] (nzmin, nzmax, incident edges | glo << 8 | ghi << 16,
                               //  incident elements); [glo, ghi) = levels at which the
                               //  adf_h pass reads the node's gnode (empty = none)
@@ -102,9 +104,6 @@ struct NodeTab {
     // its last triangle there (FCT_RING_DUP, edge code -1, range 0). NULL if a node's
     // triangles form no such ring.
     const int4* ring = nullptr;
-    // whether every edge's triangles are the two beside its slot (not where two edges join
-    // the same nodes), so that the edges' fluxes can be formed from the ring
-    bool ring_flux = false;
     // Node list of the passes: the nodes whose wet layers end above level 64 (`nshallow` of
     // them; for nl <= 64 all), in visit order, then the others; the passes take each set
     // in a launch of its own, the first with one 64-level slot per wavefront and fewer
